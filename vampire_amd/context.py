@@ -109,9 +109,7 @@ class Context:
 
     def get_spins(self) -> np.ndarray:
         out = np.empty((3, self.n), dtype=np.float64)
-        x, y, z = np.empty(self.n), np.empty(self.n), np.empty(self.n)
-        L.check(self.lib.vmx_get_spins(self.h, L.dptr(x), L.dptr(y), L.dptr(z)))
-        out[0], out[1], out[2] = x, y, z
+        L.check(self.lib.vmx_get_spins(self.h, L.dptr(out[0]), L.dptr(out[1]), L.dptr(out[2])))
         return out
 
     def set_conditions(self, temperature: float, H: Sequence[float] = (0.0, 0.0, 0.0), thermal: bool = True,
@@ -268,9 +266,9 @@ class Context:
 
     def dipole_field(self):
         """(B, mu0 Hd): per-atom [3][n] fields of the last refresh, caller's order."""
-        out = [np.empty(self.n) for _ in range(6)]
-        L.check(self.lib.vmx_get_dipole_field(self.h, *[L.dptr(a) for a in out]))
-        return np.stack(out[:3]), np.stack(out[3:])
+        b, hd = np.empty((3, self.n)), np.empty((3, self.n))
+        L.check(self.lib.vmx_get_dipole_field(self.h, *[L.dptr(a) for a in (*b, *hd)]))
+        return b, hd
 
     def set_atom_field(self, h: Optional[np.ndarray]) -> None:
         """A per-atom field [3][n] (tesla) added to H_ext in the dipole field's place; None removes it."""

@@ -10,6 +10,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <unordered_map>
 #include <vector>
 
@@ -106,6 +107,96 @@ struct PinnedRing {
     }
 };
 
+// Transfers between device memory and the caller's ordinary (pageable) arrays, in chunks of at most
+// 1 MiB through pinned slots: a worker has one chunk on the link while it copies the other between its
+// slot and the caller's array.  Bound by the host side: one worker moves 25 GB/s into memory that is
+// mapped and 4.7 GB/s into fresh pages (each is faulted in), four 13 GB/s into fresh pages and 25 into
+// mapped ones; the link takes 56.  A pageable hipMemcpy of the same arrays runs at 4.2 GB/s (fresh) and
+// costs 0.4 ms at 1 MiB against 0.07.  So: a second worker for every 8 MiB, four at most (eight gain
+// another third at 64 MiB and cost more at 8).  The first worker's two slots are allocated with the
+// context, the others by the first transfer that uses them; all are freed with it.
+struct HostPipe {
+    struct Seg { void* host; void* dev; size_t bytes; };
+    static constexpr size_t kChunk = (size_t)1 << 20;
+    static constexpr int kWorkers = 4;
+    void* slot[2 * kWorkers] = {};
+    hipEvent_t done[2 * kWorkers] = {};
+    size_t bytes = 0;              // of a slot
+    ~HostPipe() {
+        for (int k = 0; k < 2 * kWorkers; ++k) {
+            if (slot[k]) (void)hipHostFree(slot[k]);
+            if (done[k]) (void)hipEventDestroy(done[k]);
+        }
+    }
+    int ready(int workers) {
+        for (int k = 0; k < 2 * workers; ++k) {
+            if (!slot[k]) VMX_HIP(hipHostMalloc(&slot[k], bytes, hipHostMallocDefault));
+            if (!done[k]) VMX_HIP(hipEventCreateWithFlags(&done[k], hipEventDisableTiming));
+        }
+        return VMX_OK;
+    }
+    int init(size_t largest) {     // largest: the largest transfer expected
+        bytes = std::min(kChunk, std::max<size_t>(largest, 4096));
+        return ready(1);
+    }
+    // Moves every segment, after the work queued on st.  To the host: returns when the data has
+    // arrived.  To the device: returns when the caller's arrays may be reused.
+    int move(const Seg* seg, int nseg, bool to_host, hipStream_t st) {
+        std::vector<Seg> chunks;
+        size_t total = 0;
+        for (int k = 0; k < nseg; ++k)
+            for (size_t o = 0; o < seg[k].bytes; o += bytes) {
+                chunks.push_back(Seg{(char*)seg[k].host + o, (char*)seg[k].dev + o, std::min(bytes, seg[k].bytes - o)});
+                total += chunks.back().bytes;
+            }
+        const int workers = (int)std::min<size_t>(kWorkers, 1 + total / ((size_t)8 << 20));
+        VMX_TRY(ready(workers));
+        int dev = 0;
+        VMX_HIP(hipGetDevice(&dev));
+        hipError_t err[kWorkers] = {};
+        auto work = [&](int w) {
+            if (w > 0 && (err[w] = hipSetDevice(dev)) != hipSuccess) return;
+            bool used[2] = {false, false};
+            auto wait = [&](int b) {
+                const hipError_t e = used[b] ? hipEventSynchronize(done[2 * w + b]) : hipSuccess;
+                if (err[w] == hipSuccess) err[w] = e;
+                return e == hipSuccess;
+            };
+            const Seg* last = nullptr;          // to the host: the chunk in flight in the other slot
+            int b = 0;
+            for (size_t k = (size_t)w; k < chunks.size() && err[w] == hipSuccess; k += (size_t)workers, b ^= 1) {
+                const Seg& c = chunks[k];
+                if (!to_host) {
+                    if (!wait(b)) break;
+                    std::memcpy(slot[2 * w + b], c.host, c.bytes);
+                }
+                err[w] = to_host ? hipMemcpyAsync(slot[2 * w + b], c.dev, c.bytes, hipMemcpyDeviceToHost, st)
+                                 : hipMemcpyAsync(c.dev, slot[2 * w + b], c.bytes, hipMemcpyHostToDevice, st);
+                if (err[w] == hipSuccess) err[w] = hipEventRecord(done[2 * w + b], st);
+                if (err[w] != hipSuccess) break;
+                used[b] = true;
+                if (to_host && last && wait(b ^ 1)) std::memcpy(last->host, slot[2 * w + (b ^ 1)], last->bytes);
+                last = &c;
+            }
+            if (to_host && last && err[w] == hipSuccess && wait(b ^ 1))
+                std::memcpy(last->host, slot[2 * w + (b ^ 1)], last->bytes);
+            if (!to_host) { (void)wait(0); (void)wait(1); }   // the slots are free again
+        };
+        std::vector<std::thread> more;
+        int started = 1;
+        try {
+            for (; started < workers; ++started) more.emplace_back(work, started);
+        } catch (...) {                          // no more threads: this one takes their chunks
+        }
+        work(0);
+        for (std::thread& t : more) t.join();
+        for (int w = started; w < workers; ++w) work(w);
+        for (int w = 0; w < workers; ++w)
+            if (err[w] != hipSuccess) return fail(VMX_ERR_HIP, "host transfer failed: %s", hipGetErrorString(err[w]));
+        return VMX_OK;
+    }
+};
+
 // Small host->device updates (a few condition records) written by one workgroup whose kernel
 // arguments carry the bytes: they travel in the dispatch packet and the write is ordered on the
 // stream like the copy it replaces, without a DMA transfer between kernel launches.
@@ -144,19 +235,22 @@ int scratch_on_current_device(double** out) {
     return VMX_OK;
 }
 
-struct MagStat {
+// A registered statistic.  res holds what a caller reads, in one piece: the latest values [W nbins],
+// the running sums [W nbins] and the update counter (int64), so that reading it is one transfer and
+// resetting it one fill.
+template <int W>
+struct Statistic {
     int nbins;
-    DevBuf mask, cur, mean;
+    DevBuf mask, res, empty_dev;
     std::vector<int> empty;  // mask ids (< nbins-1) without atoms
-    DevBuf empty_dev;
-    DevBuf counter;          // int64 on device
+    size_t values() const { return (size_t)W * nbins; }
+    size_t bytes() const { return (2 * values() + 1) * sizeof(double); }
+    double* cur() const { return res.as<double>(); }
+    double* mean() const { return cur() + values(); }
+    long long* counter() const { return reinterpret_cast<long long*>(mean() + values()); }
 };
-
-struct EnergyStat {
-    int nbins;
-    DevBuf mask, cur, mean, empty_dev, counter;
-    std::vector<int> empty;
-};
+using MagStat = Statistic<4>;
+using EnergyStat = Statistic<5>;
 
 __global__ void k_advance_step(unsigned long long* base, unsigned int n) { *base += n; }
 __global__ void k_set_step(unsigned long long* base, unsigned long long v) { *base = v; }
@@ -414,6 +508,19 @@ __global__ void k_dip_unroll(int n, int nc, const int* __restrict__ acell, const
     hd[2 * (size_t)n + i] = Hd[2 * (size_t)nc + c];
 }
 
+// The cell field of every atom in the caller's order (cell -1: zero), [3][n] doubles
+__global__ void k_dip_to_caller(SysDev<double> s, int nc, const int* __restrict__ acell, const double* __restrict__ F,
+                                double* __restrict__ out) {
+    const int lb = logical_block(s.xcd_remap);
+    if (lb >= s.nblocks) return;
+    const int4 b = s.blk[lb];
+    const int i = b.x + (int)threadIdx.x;
+    if (i >= b.z) return;
+    const size_t o = (size_t)(b.w + caller_local(s, b.y, i - b.w)), n = (size_t)s.n;
+    const int c = acell[i];
+    for (int k = 0; k < 3; ++k) out[k * n + o] = c < 0 ? 0.0 : F[(size_t)k * nc + c];
+}
+
 }  // namespace
 
 // ============================================================================================
@@ -533,7 +640,6 @@ struct vmx_ctx {
         DevBuf start, atoms;      // per cell: its magnetic atoms (internal index), ascending caller index
         DevBuf local_cell, count, volume, tensor, mag, B, Hd, acell, mus;
         DevBuf hd_atom;           // [3][n] doubles, internal order: mu0 Hd for the energies
-        std::vector<int> acell_h; // internal order, -1: no field
     } dip;
     int hdip_on = 0;
     DevBuf hdip;
@@ -584,7 +690,12 @@ struct vmx_ctx {
     static constexpr int kMcOrderedMinSweeps = 4;   // calls with fewer sweeps stay in storage order
     static constexpr int kMcBlock = 256;   // slots per constrained Monte Carlo workgroup
     std::vector<int> mc_blk_start;         // launch l's workgroups: mc_blk[mc_blk_start[l] ...]
-    DevBuf mc_atom, mc_pat, mc_blk, mc_sigma, mc_rej, mc_tot_moves, mc_tot_rej;
+    DevBuf mc_atom, mc_pat, mc_blk, mc_rej;
+    // [nrep] each, in one piece (vmx_mc_get_state reads it in one transfer): cone widths, moves, rejects
+    DevBuf mc_state;
+    double* mc_sigma() const { return mc_state.as<double>(); }
+    double* mc_tot_moves() const { return mc_sigma() + nrep; }
+    double* mc_tot_rej() const { return mc_sigma() + 2 * (size_t)nrep; }
     // Metropolis in colour order (stencil rows only): each replica's atoms colour by colour,
     // storage order within a colour.  mco_perm[p]: storage index of colour-order atom p; the
     // stencils, material ids and caller indices (Philox counters) of the colour order; the sweep's
@@ -603,6 +714,28 @@ struct vmx_ctx {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int timed_steps = 0;
     PinnedRing ring;
+    HostPipe pipe;
+    // The caller's three component arrays to and from device arrays: permuted and converted by the
+    // device through `staging`, in order on the stream.
+    template <typename R>
+    int download(Spin3<R> src, double* x, double* y, double* z) {
+        double* st = staging.as<double>();
+        VMX_HIP(Ops<R>::to_caller(launch(), sys<R>(), src, st));
+        const size_t b = (size_t)n * sizeof(double);
+        const HostPipe::Seg seg[3] = {{x, st, b}, {y, st + n, b}, {z, st + 2 * (size_t)n, b}};
+        return pipe.move(seg, 3, true, stream);
+    }
+    template <typename R>
+    int upload3(const double* x, const double* y, const double* z, Spin3<R> dst) {
+        double* st = staging.as<double>();
+        const size_t b = (size_t)n * sizeof(double);
+        const HostPipe::Seg seg[3] = {{const_cast<double*>(x), st, b},
+                                      {const_cast<double*>(y), st + n, b},
+                                      {const_cast<double*>(z), st + 2 * (size_t)n, b}};
+        VMX_TRY(pipe.move(seg, 3, false, stream));
+        VMX_HIP(Ops<R>::from_caller(launch(), sys<R>(), st, dst));
+        return VMX_OK;
+    }
 
     ~vmx_ctx() {
         for (auto* m : mags) delete m;
@@ -1065,8 +1198,7 @@ int vmx_ctx::stats_update(double* fixed) {
         const int grid = stats_grid(st->nbins);
         VMX_HIP(Ops<R>::mag_partial(grid, stream, n, S, st->mask.as<int>(), moments(), st->nbins, part));
         hipLaunchKernelGGL(k_mag_finish, dim3(1), dim3(256), 0, stream, grid, part, st->nbins,
-                           st->cur.as<double>(), st->mean.as<double>(), st->empty_dev.as<int>(),
-                           (int)st->empty.size(), st->counter.as<long long>());
+                           st->cur(), st->mean(), st->empty_dev.as<int>(), (int)st->empty.size(), st->counter());
         VMX_HIP(hipGetLastError());
     }
     if (!energies.empty()) {
@@ -1076,8 +1208,7 @@ int vmx_ctx::stats_update(double* fixed) {
             VMX_HIP(Ops<R>::energy_partial(grid, stream, et, am(), s, S, st->mask.as<int>(), moments(),
                                            nrep > 1 ? atom_rep.as<int>() : nullptr, st->nbins, part));
             hipLaunchKernelGGL(k_energy_finish, dim3(1), dim3(256), 0, stream, grid, part, st->nbins,
-                               st->cur.as<double>(), st->mean.as<double>(), st->empty_dev.as<int>(),
-                               (int)st->empty.size(), st->counter.as<long long>());
+                               st->cur(), st->mean(), st->empty_dev.as<int>(), (int)st->empty.size(), st->counter());
             VMX_HIP(hipGetLastError());
         }
     }
@@ -1394,17 +1525,17 @@ int vmx_ctx::mc_sweeps(int nsweeps) {
             if (ordered) {
                 VMX_HIP(Ops<R>::mc_colour_ordered(stream, et, am(), so, C, mco_lidx.as<int>(), mco_blk.as<int4>(),
                                                   mco_blk_start[k], mco_blk_start[k + 1] - mco_blk_start[k],
-                                                  mc_sigma.as<double>(), sweep, mc_rej.as<double>()));
+                                                  mc_sigma(), sweep, mc_rej.as<double>()));
                 continue;
             }
             VMX_HIP(Ops<R>::mc_colour(stream, et, am(), s, S, mc_atom.as<int>(), mc_pat.as<uint16_t>(),
                                       mc_blk.as<int2>(), mc_blk_start[k], mc_blk_start[k + 1] - mc_blk_start[k],
-                                      mc_sigma.as<double>(), sweep,
+                                      mc_sigma(), sweep,
                                       mc_rej.as<double>()));
         }
         hipLaunchKernelGGL(k_mc_adapt, dim3((nrep + 3) / 4), dim3(256), 0, stream, nrep, rep_off.as<int>(),
-                           mc_sigma.as<double>(), mc_rej.as<double>(), mc_tot_moves.as<double>(),
-                           mc_tot_rej.as<double>());
+                           mc_sigma(), mc_rej.as<double>(), mc_tot_moves(),
+                           mc_tot_rej());
         VMX_HIP(hipGetLastError());
         ++sweep;
         // a sweep advances sim::time like a Heun step (sim.cpp:608-615, 191-200)
@@ -1495,7 +1626,7 @@ int vmx_ctx::cmc_sweeps(int nsweeps) {
                 VMX_HIP(Ops<R>::cmc_pairs(stream, et, am(), so, C, pmm, plist, plidx,
                                           cmc_tab.as<int4>() + cmc_tab_start[k], ntab,
                                           cmc_perm.as<int4>() + (size_t)(2 * k + round) * nrep,
-                                          cmc_frame.as<CmcFrame<R>>(), cmc_M.as<double>(), mc_sigma.as<double>(),
+                                          cmc_frame.as<CmcFrame<R>>(), cmc_M.as<double>(), mc_sigma(),
                                           cmc_move, round, sweep, cmc_counts.as<double>(), dm));
                 if (k < last || round == 0)
                     VMX_HIP(Ops<R>::moment_add(stream, cmc_range.as<int>() + (size_t)k * (nrep + 1), nrep, dm,
@@ -1536,28 +1667,15 @@ int vmx_ctx::fit_forward(const double* h, const double* spins0, double* mz_out) 
     VMX_TRY(fit.P.alloc(N3 * sizeof(R)));
     VMX_TRY(fit.h.alloc(N3 * sizeof(R)));
     VMX_TRY(fit.mz.alloc((size_t)4 * std::max(fit.nrec, 1) * sizeof(double)));
-    double* st = staging.as<double>();
-    VMX_HIP(hipStreamSynchronize(stream));
     fit.has_h = h != nullptr;
-    if (h) {
-        std::vector<double> hi(N3);
-        to_internal(h, hi.data(), 3);
-        VMX_HIP(hipMemcpy(st, hi.data(), N3 * sizeof(double), hipMemcpyHostToDevice));
-        VMX_HIP(Ops<R>::from_double(stream, (int)N3, st, fit.h.as<R>()));
-        VMX_HIP(hipStreamSynchronize(stream));
-    }
-    {
-        std::vector<double> si(N3);
-        to_internal(spins0, si.data(), 3);
-        VMX_HIP(hipMemcpy(st, si.data(), N3 * sizeof(double), hipMemcpyHostToDevice));
-    }
     R* ck = fit.ckpt.as<R>();
-    VMX_HIP(Ops<R>::from_double(stream, (int)N3, st, ck));
+    auto state = [&](R* base) { return Spin3<R>{base, base + n, base + 2 * (size_t)n}; };
+    if (h) VMX_TRY(upload3(h, h + n, h + 2 * (size_t)n, arr3<R>(fit.h)));
+    VMX_TRY(upload3(spins0, spins0 + n, spins0 + 2 * (size_t)n, state(ck)));
     VMX_HIP(hipMemsetAsync(fit.mz.p, 0, (size_t)4 * std::max(fit.nrec, 1) * sizeof(double), stream));
     const SysDev<R> s = sys<R>();
     const FitPrm<R> p = fit_prm<R>();
     const Spin3<R> hh = fit.has_h ? arr3<R>(fit.h) : Spin3<R>{nullptr, nullptr, nullptr};
-    auto state = [&](R* base) { return Spin3<R>{base, base + n, base + 2 * (size_t)n}; };
     R* seg = fit.seg.as<R>();
     R* cur = seg;
     R* nxt = seg + N3;
@@ -1682,14 +1800,7 @@ int vmx_ctx::fit_backward(const double* dmz, double* grad, double* dh_out) {
     grad[0] = acc[0];
     grad[1] = acc[1];
     grad[2] = acc[2] * da_dal + acc[3] * db_dal;
-    if (dh_out) {
-        double* st = staging.as<double>();
-        VMX_HIP(Ops<R>::to_double(stream, (int)N3, fit.dh.as<R>(), st));
-        VMX_HIP(hipStreamSynchronize(stream));
-        std::vector<double> tmp(N3);
-        VMX_HIP(hipMemcpy(tmp.data(), st, N3 * sizeof(double), hipMemcpyDeviceToHost));
-        to_caller(tmp.data(), dh_out, 3);
-    }
+    if (dh_out) VMX_TRY(download(arr3<R>(fit.dh), dh_out, dh_out + n, dh_out + 2 * (size_t)n));
     return VMX_OK;
 }
 
@@ -2134,22 +2245,21 @@ int vmx_create(const vmx_system* sys, const vmx_options* opt, vmx_ctx** out) {
         VMX_TRY(c->euler_buf.alloc(3 * (size_t)n * rs));
     if (c->kernel == VMX_KERNEL_FUSED && c->store_field) VMX_TRY(c->field_buf.alloc(3 * (size_t)n * rs));
     const size_t cond_bytes = (size_t)nrep * c->nmat * sizeof(Cond<double>) + 64;
-    VMX_TRY(c->ring.init(std::max<size_t>(cond_bytes, 8 * (size_t)nrep + 64)));
+    // tables that fit a launch's arguments never use the ring
+    if (cond_bytes > sizeof(ArgWords)) VMX_TRY(c->ring.init(std::max<size_t>(cond_bytes, 8 * (size_t)nrep + 64)));
+    VMX_TRY(c->pipe.init((size_t)n * sizeof(double)));
     VMX_TRY(c->upload_conditions_any());
     // Monte Carlo state: adaptive sigma starts at 60 (src/montecarlo/data.cpp:46)
-    VMX_TRY(c->mc_sigma.alloc(nrep * sizeof(double)));
+    VMX_TRY(c->mc_state.alloc(3 * (size_t)nrep * sizeof(double)));
     VMX_TRY(c->mc_rej.alloc((size_t)nrep * kRejectSlots * kRejectStride * sizeof(double)));
-    VMX_TRY(c->mc_tot_moves.alloc(nrep * sizeof(double)));
-    VMX_TRY(c->mc_tot_rej.alloc(nrep * sizeof(double)));
     VMX_TRY(c->cmc_counts.alloc((size_t)nrep * kRejectSlots * kRejectStride * sizeof(double)));
     c->cmc_frame_h.assign(21 * (size_t)nrep, 0.0);
     c->cmc_frame_set.assign(nrep, 0);
     {
-        std::vector<double> s60(nrep, 60.0);
-        VMX_HIP(hipMemcpy(c->mc_sigma.p, s60.data(), nrep * sizeof(double), hipMemcpyHostToDevice));
+        std::vector<double> s60(3 * (size_t)nrep, 0.0);
+        std::fill(s60.begin(), s60.begin() + nrep, 60.0);
+        VMX_HIP(hipMemcpy(c->mc_state.p, s60.data(), s60.size() * sizeof(double), hipMemcpyHostToDevice));
         VMX_HIP(hipMemset(c->mc_rej.p, 0, (size_t)nrep * kRejectSlots * kRejectStride * sizeof(double)));
-        VMX_HIP(hipMemset(c->mc_tot_moves.p, 0, nrep * sizeof(double)));
-        VMX_HIP(hipMemset(c->mc_tot_rej.p, 0, nrep * sizeof(double)));
         VMX_HIP(hipMemset(c->cmc_counts.p, 0, (size_t)nrep * kRejectSlots * kRejectStride * sizeof(double)));
     }
     VMX_HIP(hipDeviceSynchronize());
@@ -2181,20 +2291,8 @@ int vmx_destroy(vmx_ctx* ctx) {
 int vmx_set_spins(vmx_ctx* c, const double* sx, const double* sy, const double* sz) {
     if (!c || !sx || !sy || !sz) return fail(VMX_ERR_ARG, "null argument");
     VMX_TRY(c->use_device());
-    const size_t nb = (size_t)c->n * sizeof(double);
-    double* st = c->staging.as<double>();
-    VMX_HIP(hipStreamSynchronize(c->stream));
-    std::vector<double> host(3 * (size_t)c->n), perm(3 * (size_t)c->n);
-    std::memcpy(host.data(), sx, nb);
-    std::memcpy(host.data() + c->n, sy, nb);
-    std::memcpy(host.data() + 2 * (size_t)c->n, sz, nb);
-    c->to_internal(host.data(), perm.data(), 3);
-    VMX_HIP(hipMemcpy(st, perm.data(), 3 * nb, hipMemcpyHostToDevice));
-    if (c->precision == VMX_FP64) {
-        VMX_HIP(hipMemcpyAsync(c->spin[c->s_idx].p, st, 3 * nb, hipMemcpyDeviceToDevice, c->stream));
-    } else {
-        VMX_HIP(Ops<float>::from_double(c->stream, 3 * c->n, st, c->spin[c->s_idx].as<float>()));
-    }
+    VMX_TRY(c->precision == VMX_FP64 ? c->upload3(sx, sy, sz, c->spins<double>(c->s_idx))
+                                     : c->upload3(sx, sy, sz, c->spins<float>(c->s_idx)));
     VMX_HIP(hipStreamSynchronize(c->stream));
     return VMX_OK;
 }
@@ -2202,21 +2300,8 @@ int vmx_set_spins(vmx_ctx* c, const double* sx, const double* sy, const double* 
 int vmx_get_spins(vmx_ctx* c, double* sx, double* sy, double* sz) {
     if (!c || !sx || !sy || !sz) return fail(VMX_ERR_ARG, "null argument");
     VMX_TRY(c->use_device());
-    const size_t nb = (size_t)c->n * sizeof(double);
-    double* st = c->staging.as<double>();
-    if (c->precision == VMX_FP64) {
-        VMX_HIP(hipMemcpyAsync(st, c->spin[c->s_idx].p, 3 * nb, hipMemcpyDeviceToDevice, c->stream));
-    } else {
-        VMX_HIP(Ops<float>::to_double(c->stream, 3 * c->n, c->spin[c->s_idx].as<float>(), st));
-    }
-    VMX_HIP(hipStreamSynchronize(c->stream));
-    std::vector<double> perm(3 * (size_t)c->n), host(3 * (size_t)c->n);
-    VMX_HIP(hipMemcpy(perm.data(), st, 3 * nb, hipMemcpyDeviceToHost));
-    c->to_caller(perm.data(), host.data(), 3);
-    std::memcpy(sx, host.data(), nb);
-    std::memcpy(sy, host.data() + c->n, nb);
-    std::memcpy(sz, host.data() + 2 * (size_t)c->n, nb);
-    return VMX_OK;
+    return c->precision == VMX_FP64 ? c->download(c->spins<double>(c->s_idx), sx, sy, sz)
+                                    : c->download(c->spins<float>(c->s_idx), sx, sy, sz);
 }
 
 int vmx_set_time_step(vmx_ctx* c, double dt, double half_dt) {
@@ -2419,9 +2504,7 @@ int vmx_checkpoint_load(vmx_ctx* c, const void* buf, uint64_t bytes) {
     get(tmp.data(), 24 * (size_t)c->nrep);
     VMX_HIP(hipStreamSynchronize(c->stream));
     const size_t rb = c->nrep * sizeof(double);
-    VMX_HIP(hipMemcpy(c->mc_sigma.p, tmp.data(), rb, hipMemcpyHostToDevice));
-    VMX_HIP(hipMemcpy(c->mc_tot_moves.p, tmp.data() + c->nrep, rb, hipMemcpyHostToDevice));
-    VMX_HIP(hipMemcpy(c->mc_tot_rej.p, tmp.data() + 2 * (size_t)c->nrep, rb, hipMemcpyHostToDevice));
+    VMX_HIP(hipMemcpy(c->mc_state.p, tmp.data(), 3 * rb, hipMemcpyHostToDevice));
     get(tmp.data(), 24 * (size_t)c->n);
     VMX_TRY(vmx_set_spins(c, tmp.data(), tmp.data() + c->n, tmp.data() + 2 * (size_t)c->n));
     VMX_TRY(vmx_set_step(c, (int64_t)step));
@@ -2442,11 +2525,13 @@ int vmx_mc_sweep(vmx_ctx* c, int32_t nsweeps) {
 int vmx_mc_get_state(vmx_ctx* c, double* sigma, double* moves, double* rejects) {
     if (!c) return fail(VMX_ERR_ARG, "null context");
     VMX_TRY(c->use_device());
-    VMX_HIP(hipStreamSynchronize(c->stream));
-    const size_t b = c->nrep * sizeof(double);
-    if (sigma) VMX_HIP(hipMemcpy(sigma, c->mc_sigma.p, b, hipMemcpyDeviceToHost));
-    if (moves) VMX_HIP(hipMemcpy(moves, c->mc_tot_moves.p, b, hipMemcpyDeviceToHost));
-    if (rejects) VMX_HIP(hipMemcpy(rejects, c->mc_tot_rej.p, b, hipMemcpyDeviceToHost));
+    const size_t k = (size_t)c->nrep;
+    std::vector<double> v(3 * k);
+    const HostPipe::Seg seg{v.data(), c->mc_state.p, v.size() * sizeof(double)};
+    VMX_TRY(c->pipe.move(&seg, 1, true, c->stream));
+    if (sigma) std::copy(v.begin(), v.begin() + k, sigma);
+    if (moves) std::copy(v.begin() + k, v.begin() + 2 * k, moves);
+    if (rejects) std::copy(v.begin() + 2 * k, v.end(), rejects);
     return VMX_OK;
 }
 
@@ -2457,7 +2542,7 @@ int vmx_mc_set_sigma(vmx_ctx* c, int32_t replica, double sigma) {
     VMX_HIP(hipStreamSynchronize(c->stream));
     const int r0 = replica < 0 ? 0 : replica, r1 = replica < 0 ? c->nrep : replica + 1;
     for (int r = r0; r < r1; ++r)
-        VMX_HIP(hipMemcpy(c->mc_sigma.as<double>() + r, &sigma, sizeof(double), hipMemcpyHostToDevice));
+        VMX_HIP(hipMemcpy(c->mc_sigma() + r, &sigma, sizeof(double), hipMemcpyHostToDevice));
     return VMX_OK;
 }
 
@@ -2527,10 +2612,10 @@ int vmx_cmc_sweep(vmx_ctx* c, int32_t nsweeps) {
 int vmx_cmc_get_counts(vmx_ctx* c, double* counts) {
     if (!c || !counts) return fail(VMX_ERR_ARG, "null argument");
     VMX_TRY(c->use_device());
-    VMX_HIP(hipStreamSynchronize(c->stream));
     const size_t per = (size_t)kRejectSlots * kRejectStride;
     std::vector<double> slots((size_t)c->nrep * per);
-    VMX_HIP(hipMemcpy(slots.data(), c->cmc_counts.p, slots.size() * sizeof(double), hipMemcpyDeviceToHost));
+    const HostPipe::Seg seg{slots.data(), c->cmc_counts.p, slots.size() * sizeof(double)};
+    VMX_TRY(c->pipe.move(&seg, 1, true, c->stream));
     for (int r = 0; r < c->nrep; ++r)
         for (int k = 0; k < 3; ++k) {
             double t = 0.0;
@@ -2562,15 +2647,11 @@ int vmx_stats_add_magnetization(vmx_ctx* c, int32_t mask_size, const int32_t* ma
     st->nbins = mask_size;
     VMX_TRY(st->mask.alloc((size_t)c->n * sizeof(int)));
     VMX_HIP(hipMemcpy(st->mask.p, c->internal_ints(mask).data(), (size_t)c->n * sizeof(int), hipMemcpyHostToDevice));
-    VMX_TRY(st->cur.alloc(4 * (size_t)mask_size * sizeof(double)));
-    VMX_TRY(st->mean.alloc(4 * (size_t)mask_size * sizeof(double)));
-    VMX_HIP(hipMemset(st->cur.p, 0, 4 * (size_t)mask_size * sizeof(double)));
-    VMX_HIP(hipMemset(st->mean.p, 0, 4 * (size_t)mask_size * sizeof(double)));
+    VMX_TRY(st->res.alloc(st->bytes()));
+    VMX_HIP(hipMemset(st->res.p, 0, st->bytes()));
     VMX_TRY(st->empty_dev.alloc(std::max<size_t>(1, st->empty.size()) * sizeof(int)));
     if (!st->empty.empty())
         VMX_HIP(hipMemcpy(st->empty_dev.p, st->empty.data(), st->empty.size() * sizeof(int), hipMemcpyHostToDevice));
-    VMX_TRY(st->counter.alloc(sizeof(long long)));
-    VMX_HIP(hipMemset(st->counter.p, 0, sizeof(long long)));
     *handle = (int32_t)c->mags.size();
     c->mags.push_back(st.release());
     return VMX_OK;
@@ -2584,15 +2665,11 @@ int vmx_stats_add_energy(vmx_ctx* c, int32_t mask_size, const int32_t* mask, int
     st->nbins = mask_size;
     VMX_TRY(st->mask.alloc((size_t)c->n * sizeof(int)));
     VMX_HIP(hipMemcpy(st->mask.p, c->internal_ints(mask).data(), (size_t)c->n * sizeof(int), hipMemcpyHostToDevice));
-    VMX_TRY(st->cur.alloc(5 * (size_t)mask_size * sizeof(double)));
-    VMX_TRY(st->mean.alloc(5 * (size_t)mask_size * sizeof(double)));
-    VMX_HIP(hipMemset(st->cur.p, 0, 5 * (size_t)mask_size * sizeof(double)));
-    VMX_HIP(hipMemset(st->mean.p, 0, 5 * (size_t)mask_size * sizeof(double)));
+    VMX_TRY(st->res.alloc(st->bytes()));
+    VMX_HIP(hipMemset(st->res.p, 0, st->bytes()));
     VMX_TRY(st->empty_dev.alloc(std::max<size_t>(1, st->empty.size()) * sizeof(int)));
     if (!st->empty.empty())
         VMX_HIP(hipMemcpy(st->empty_dev.p, st->empty.data(), st->empty.size() * sizeof(int), hipMemcpyHostToDevice));
-    VMX_TRY(st->counter.alloc(sizeof(long long)));
-    VMX_HIP(hipMemset(st->counter.p, 0, sizeof(long long)));
     *handle = (int32_t)c->energies.size();
     c->energies.push_back(st.release());
     return VMX_OK;
@@ -2623,54 +2700,48 @@ int vmx_stats_update_noalloc(vmx_ctx* c) {
                                     : c->stats_update<float>(c->stats_scratch);
 }
 
+extern "C++" template <int W>
+static int read_statistic(vmx_ctx* c, const Statistic<W>& st, double* cur, double* mean, int64_t* counter) {
+    const size_t k = st.values();
+    std::vector<double> v(2 * k + 1);
+    const HostPipe::Seg seg{v.data(), st.res.p, st.bytes()};
+    VMX_TRY(c->pipe.move(&seg, 1, true, c->stream));
+    if (cur) std::copy(v.begin(), v.begin() + k, cur);
+    if (mean) std::copy(v.begin() + k, v.begin() + 2 * k, mean);
+    if (counter) {
+        long long n = 0;
+        std::memcpy(&n, &v[2 * k], sizeof n);
+        *counter = n;
+    }
+    return VMX_OK;
+}
+
 int vmx_stats_get_magnetization(vmx_ctx* c, int32_t handle, double* magnetization, double* mean_sum,
                                 int64_t* counter) {
     if (!c) return fail(VMX_ERR_ARG, "null context");
     if (handle < 0 || handle >= (int)c->mags.size()) return fail(VMX_ERR_ARG, "bad magnetization handle %d", handle);
     VMX_TRY(c->use_device());
-    VMX_HIP(hipStreamSynchronize(c->stream));
-    MagStat* st = c->mags[handle];
-    const size_t b = 4 * (size_t)st->nbins * sizeof(double);
-    if (magnetization) VMX_HIP(hipMemcpy(magnetization, st->cur.p, b, hipMemcpyDeviceToHost));
-    if (mean_sum) VMX_HIP(hipMemcpy(mean_sum, st->mean.p, b, hipMemcpyDeviceToHost));
-    if (counter) {
-        long long v = 0;
-        VMX_HIP(hipMemcpy(&v, st->counter.p, sizeof v, hipMemcpyDeviceToHost));
-        *counter = v;
-    }
-    return VMX_OK;
+    return read_statistic(c, *c->mags[handle], magnetization, mean_sum, counter);
 }
 
 int vmx_stats_get_energy(vmx_ctx* c, int32_t handle, double* energy, double* mean_sum, int64_t* counter) {
     if (!c) return fail(VMX_ERR_ARG, "null context");
     if (handle < 0 || handle >= (int)c->energies.size()) return fail(VMX_ERR_ARG, "bad energy handle %d", handle);
     VMX_TRY(c->use_device());
-    VMX_HIP(hipStreamSynchronize(c->stream));
-    EnergyStat* st = c->energies[handle];
-    const size_t b = 5 * (size_t)st->nbins * sizeof(double);
-    if (energy) VMX_HIP(hipMemcpy(energy, st->cur.p, b, hipMemcpyDeviceToHost));
-    if (mean_sum) VMX_HIP(hipMemcpy(mean_sum, st->mean.p, b, hipMemcpyDeviceToHost));
-    if (counter) {
-        long long v = 0;
-        VMX_HIP(hipMemcpy(&v, st->counter.p, sizeof v, hipMemcpyDeviceToHost));
-        *counter = v;
-    }
-    return VMX_OK;
+    return read_statistic(c, *c->energies[handle], energy, mean_sum, counter);
 }
 
 int vmx_stats_reset(vmx_ctx* c) {
     if (!c) return fail(VMX_ERR_ARG, "null context");
     VMX_TRY(c->use_device());
-    VMX_HIP(hipStreamSynchronize(c->stream));
-    for (MagStat* st : c->mags) {
-        VMX_HIP(hipMemset(st->mean.p, 0, 4 * (size_t)st->nbins * sizeof(double)));
-        VMX_HIP(hipMemset(st->counter.p, 0, sizeof(long long)));
-    }
-    for (EnergyStat* st : c->energies) {
-        VMX_HIP(hipMemset(st->mean.p, 0, 5 * (size_t)st->nbins * sizeof(double)));
-        VMX_HIP(hipMemset(st->counter.p, 0, sizeof(long long)));
-    }
-    VMX_HIP(hipDeviceSynchronize());
+    // running sums and counter lie together (a counter of zero has the bits of 0.0): one fill each, in
+    // order on the stream
+    auto clear = [&](double* mean, size_t values) {
+        hipLaunchKernelGGL((k_fill<double>), dim3(1), dim3(256), 0, c->stream, values + 1, mean, 0.0);
+    };
+    for (const MagStat* st : c->mags) clear(st->mean(), st->values());
+    for (const EnergyStat* st : c->energies) clear(st->mean(), st->values());
+    VMX_HIP(hipGetLastError());
     return VMX_OK;
 }
 
@@ -2692,17 +2763,11 @@ static int compute_fields_impl(vmx_ctx* c, const double* noise, double* h_spin, 
     }
     VMX_HIP(Ops<R>::spin_fields(L, c->et, c->am(), s, c->spins<R>(c->s_idx), c->arr3<R>(c->plainF)));
     VMX_HIP(Ops<R>::ext_fields(L, s, c->arr3<R>(c->plainE), nd, 0u));
-    const size_t nb = 3 * (size_t)c->n * sizeof(double);
-    double* st = c->staging.as<double>();
     for (int which = 0; which < 2; ++which) {
         double* dst = which == 0 ? h_spin : h_ext;
         if (!dst) continue;
         const DevBuf& src = which == 0 ? c->plainF : c->plainE;
-        VMX_HIP(Ops<R>::to_double(c->stream, 3 * c->n, src.as<R>(), st));
-        VMX_HIP(hipStreamSynchronize(c->stream));
-        std::vector<double> tmp(3 * (size_t)c->n);
-        VMX_HIP(hipMemcpy(tmp.data(), st, nb, hipMemcpyDeviceToHost));
-        c->to_caller(tmp.data(), dst, 3);
+        VMX_TRY(c->download(c->arr3<R>(src), dst, dst + c->n, dst + 2 * (size_t)c->n));
     }
     VMX_HIP(hipStreamSynchronize(c->stream));
     return VMX_OK;
@@ -2945,7 +3010,6 @@ int vmx_set_dipole(vmx_ctx* c, const vmx_dipole* d) {
     VMX_HIP(hipMemset(c->hdip.p, 0, 3 * (size_t)n * c->rsize()));
     VMX_TRY(D.hd_atom.alloc(3 * (size_t)n * sizeof(double)));
     VMX_HIP(hipMemset(D.hd_atom.p, 0, 3 * (size_t)n * sizeof(double)));
-    D.acell_h = acell;
     D.nc = nc; D.nl = nl; D.rate = d->update_rate; D.time = 0;
     D.on = 1;
     c->hdip_on = 1;
@@ -2970,19 +3034,19 @@ int vmx_get_dipole_field(vmx_ctx* c, double* bx, double* by, double* bz, double*
     if (!c) return fail(VMX_ERR_ARG, "null context");
     if (!c->dip.on) return fail(VMX_ERR_STATE, "no dipole field set (vmx_set_dipole)");
     VMX_TRY(c->use_device());
-    VMX_HIP(hipStreamSynchronize(c->stream));
-    const int n = c->n, nc = c->dip.nc;
-    std::vector<double> B(3 * (size_t)nc), H(3 * (size_t)nc);
-    VMX_HIP(hipMemcpy(B.data(), c->dip.B.p, B.size() * sizeof(double), hipMemcpyDeviceToHost));
-    VMX_HIP(hipMemcpy(H.data(), c->dip.Hd.p, H.size() * sizeof(double), hipMemcpyDeviceToHost));
     double* out[6] = {bx, by, bz, hx, hy, hz};
-    for (int i = 0; i < n; ++i) {
-        const int cell = c->dip.acell_h[c->q > 1 ? c->pi[i] : i];
-        for (int k = 0; k < 6; ++k) {
-            if (!out[k]) continue;
-            const std::vector<double>& src = k < 3 ? B : H;
-            out[k][i] = cell < 0 ? 0.0 : src[(size_t)(k % 3) * nc + cell];
-        }
+    const size_t n = (size_t)c->n;
+    double* st = c->staging.as<double>();
+    for (int f = 0; f < 2; ++f) {                  // B, then mu0 Hd
+        HostPipe::Seg seg[3];
+        int k = 0;
+        for (int x = 0; x < 3; ++x)
+            if (out[3 * f + x]) seg[k++] = HostPipe::Seg{out[3 * f + x], st + x * n, n * sizeof(double)};
+        if (!k) continue;
+        hipLaunchKernelGGL(k_dip_to_caller, dim3(c->launch().grid), dim3(c->block), 0, c->stream, c->sys<double>(),
+                           c->dip.nc, c->dip.acell.as<int>(), (f ? c->dip.Hd : c->dip.B).as<double>(), st);
+        VMX_HIP(hipGetLastError());
+        VMX_TRY(c->pipe.move(seg, k, true, c->stream));
     }
     return VMX_OK;
 }

@@ -94,9 +94,10 @@ struct Ops {
     static hipError_t fit_mz(hipStream_t st, int n, Spin3<R> S, double* out4);
     // Philox normals of `step` as double [3][n]
     static hipError_t thermal_noise(const Launch& L, const SysDev<R>& s, uint64_t step, double* out);
-    // conversions between the double host/staging layout and R device arrays
-    static hipError_t from_double(hipStream_t st, int n, const double* in, R* out);
-    static hipError_t to_double(hipStream_t st, int n, const R* in, double* out);
+    // three-component arrays between the device's atom order and the caller's ([3][n] doubles), over
+    // the one-atom block table
+    static hipError_t to_caller(const Launch& L, const SysDev<R>& s, Spin3<R> S, double* out);
+    static hipError_t from_caller(const Launch& L, const SysDev<R>& s, const double* in, Spin3<R> S);
 };
 
 extern template struct Ops<double>;

@@ -600,6 +600,13 @@ struct vmx_ctx {
     // can write S_next over S, and a step touches two spin arrays instead of three; the FP64
     // corrector that recomputes dS gathers S and cannot.
     bool corrector_in_place() const { return precision == VMX_FP32 || store_euler; }
+    // Tiles of the whole-step kernel (k_tile_step); ntiles == 0: the step takes two kernels.
+    int ntiles = 0;
+    bool tiles_made = false;      // or found to be out of question
+    int64_t steps_before_tiles = 0;
+    TileDev tile{};
+    DevBuf tile_buf;
+    int build_tiles(int64_t steps);
     DevBuf plainF, plainE, plainD;
     int store_euler = 1;          // fused FP64 step: the predictor keeps dS (FP32 keeps nothing)
     DevBuf euler_buf;             // 3N R
@@ -1015,6 +1022,7 @@ template <typename R>
 int vmx_ctx::heun_steps(int nsteps, const double* noise, double* kernel_ms) {
     const SysDev<R> s = sys<R>(), sf = sys_fused<R>();
     const Launch L = launch(), Lf = launch_fused();
+    VMX_TRY(build_tiles(nsteps));
     uint32_t off0 = 0;
     VMX_TRY(eager_step_off(nsteps, off0));
     const double* nd = nullptr;
@@ -1051,7 +1059,11 @@ int vmx_ctx::heun_steps(int nsteps, const double* noise, double* kernel_ms) {
         }
         const int p_idx = 3 - s_idx - o_idx;
         int nk = 0;
-        if (kernel == VMX_KERNEL_FUSED) {
+        if (kernel == VMX_KERNEL_FUSED && ntiles && !kernel_ms) {
+            VMX_HIP(Ops<R>::tile_step(stream, et, jm, wsel, STEP_HEUN, s, tile, ntiles, spins<R>(s_idx), spins<R>(o_idx),
+                                      nd, off0 + (uint32_t)k));
+            std::swap(s_idx, o_idx);
+        } else if (kernel == VMX_KERNEL_FUSED) {
             VMX_HIP(mark(0));
             VMX_HIP(Ops<R>::fused_predictor(Lf, et, am(), sf, spins<R>(s_idx), spins<R>(p_idx), euler<R>(),
                                             field<R>(), nd, off0 + (uint32_t)k));
@@ -1104,6 +1116,7 @@ template <typename R>
 int vmx_ctx::midpoint_steps(int nsteps, const double* noise) {
     const SysDev<R> s = sys<R>(), sf = sys_fused<R>();
     const Launch L = launch(), Lf = launch_fused();
+    VMX_TRY(build_tiles(nsteps));
     uint32_t off0 = 0;
     VMX_TRY(eager_step_off(nsteps, off0));
     const double* nd = nullptr;
@@ -1123,12 +1136,18 @@ int vmx_ctx::midpoint_steps(int nsteps, const double* noise) {
         } else if (normals64) {
             VMX_TRY(draw_fp64_normals(step + (uint64_t)k));
         }
-        const int p_idx = 3 - s_idx - o_idx;
-        VMX_HIP(Ops<R>::mid_predictor(Lf, et, am(), sf, spins<R>(s_idx), spins<R>(p_idx), field<R>(), nd,
-                                      off0 + (uint32_t)k));
-        // the midpoint corrector gathers only the midpoint: S_next overwrites S
-        VMX_HIP(Ops<R>::mid_corrector(L, et, am(), s, spins<R>(s_idx), spins<R>(p_idx), spins<R>(s_idx), field<R>(),
-                                      nd, off0 + (uint32_t)k));
+        if (ntiles) {
+            VMX_HIP(Ops<R>::tile_step(stream, et, jm, wsel, STEP_MIDPOINT, s, tile, ntiles, spins<R>(s_idx),
+                                      spins<R>(o_idx), nd, off0 + (uint32_t)k));
+            std::swap(s_idx, o_idx);
+        } else {
+            const int p_idx = 3 - s_idx - o_idx;
+            VMX_HIP(Ops<R>::mid_predictor(Lf, et, am(), sf, spins<R>(s_idx), spins<R>(p_idx), field<R>(), nd,
+                                          off0 + (uint32_t)k));
+            // the midpoint corrector gathers only the midpoint: S_next overwrites S
+            VMX_HIP(Ops<R>::mid_corrector(L, et, am(), s, spins<R>(s_idx), spins<R>(p_idx), spins<R>(s_idx), field<R>(),
+                                          nd, off0 + (uint32_t)k));
+        }
         if (dip.on && (dip.time + k + 1) % dip.rate == 0) VMX_TRY(dipole_refresh<R>());
     }
     if (timed) VMX_HIP(hipEventRecord(ev1, stream));
@@ -1148,12 +1167,18 @@ int vmx_ctx::capture_graph(int nsteps) {
     int si = s_idx, oi = o_idx;
     for (int k = 0; k < nsteps; ++k) {
         const int pi = 3 - si - oi;
-        hipError_t e = Ops<R>::fused_predictor(Lf, et, am(), sf, spins<R>(si), spins<R>(pi), euler<R>(), field<R>(),
-                                               nullptr, (uint32_t)k);
-        const int out = corrector_in_place() ? si : oi;
-        if (e == hipSuccess)
-            e = Ops<R>::fused_corrector(L, et, am(), s, spins<R>(si), spins<R>(pi), spins<R>(out), euler<R>(),
-                                        field<R>(), nullptr, (uint32_t)k);
+        const int out = corrector_in_place() && !ntiles ? si : oi;
+        hipError_t e;
+        if (ntiles) {
+            e = Ops<R>::tile_step(stream, et, jm, wsel, STEP_HEUN, s, tile, ntiles, spins<R>(si), spins<R>(out), nullptr,
+                                  (uint32_t)k);
+        } else {
+            e = Ops<R>::fused_predictor(Lf, et, am(), sf, spins<R>(si), spins<R>(pi), euler<R>(), field<R>(), nullptr,
+                                        (uint32_t)k);
+            if (e == hipSuccess)
+                e = Ops<R>::fused_corrector(L, et, am(), s, spins<R>(si), spins<R>(pi), spins<R>(out), euler<R>(),
+                                            field<R>(), nullptr, (uint32_t)k);
+        }
         if (e != hipSuccess) {
             hipGraph_t g;
             (void)hipStreamEndCapture(stream, &g);
@@ -2022,6 +2047,110 @@ static int build_topology(vmx_ctx* c, int request, const std::vector<int>& rowh,
     return VMX_OK;
 }
 
+// Tiles of the whole-step kernel.  Grown breadth first from the lowest unassigned atom, a tile takes
+// atoms while they and their halo fit its items (one per thread); a component that ends early is
+// followed by the next, so that tiles stay full.
+//
+// Where the line lies (us a step from a replayed graph, whole-step against two kernels, FP64 / FP32):
+//   SC   9^3 4.9/3.5 against 9.4/8.2    SC  33^3 8.6/5.9 against 9.9/8.3    SC  40^3 10.0/6.9 against 10.1/8.3
+//   BCC 16^3 5.7/4.1 against 10.2/8.9   BCC 28^3 9.5/7.0 against 10.8/9.0   BCC 32^3 12.8/10.6 against 10.9/8.8
+//   FCC 12^3 5.7/4.5 against 12.1/9.5   FCC 20^3 9.9/7.4 against 12.3/9.6   FCC 23^3 13.0/9.6 against 12.6/9.7
+// The whole step reads each item's record (slots of neighbour indices) and repeats the halo's
+// arithmetic, so the two meet at a number of slots, 400,000 = SC 40^3 = FCC 20^3.  CSR rows (no fixed
+// slot width) and the plain kernels keep their launches.
+// Items per tile: 128 where the tiles do not fill the CUs (SC 20^3 FP64 5.2 us; 256: 5.7), then larger
+// tiles, whose halo is smaller (SC 33^3 FP32: 128 5.9, 192 5.9, 256 6.3; FCC 20^3: 8.7, 7.4, 8.4;
+// SC 40^3: 8.0, 7.5, 6.9).
+constexpr int kTileMaxSlots = 400000;
+//
+// steps: the steps about to be taken.  Making the tiles takes the host 25-40 ns an atom, about n / 128
+// steps' worth of what they save, so a context makes them when it has been asked for that many steps in
+// all (both forms give the same spins).
+int vmx_ctx::build_tiles(int64_t steps) {
+    if (tiles_made) return VMX_OK;
+    const int W = zmax;
+    if (kernel != VMX_KERNEL_FUSED || tp == TP_CSR || (int64_t)n * W > kTileMaxSlots) {
+        tiles_made = true;
+        return VMX_OK;
+    }
+    steps_before_tiles += steps;
+    if (steps_before_tiles < n / 128) return VMX_OK;
+    const int B = n <= 12288 ? 128 : (n <= 40000 ? 192 : 256);
+    struct Atom { int tile, mark, tried; };      // its tile, the last tile and the last attempt that met it
+    std::vector<Atom> at(n, Atom{-1, -1, -1});
+    std::vector<int4> hdr;
+    std::vector<int> atom, halo, queue, fresh;   // atom: [tile][B]
+    atom.reserve(3 * (size_t)n + B);
+    int attempt = 0;
+    for (int r = 0; r < nrep; ++r) {
+        int next = rep_off_h[r];
+        const int end = rep_off_h[r + 1];
+        for (;;) {
+            while (next < end && at[next].tile >= 0) ++next;
+            if (next >= end) break;
+            const int id = (int)hdr.size();
+            const size_t base = atom.size();
+            halo.clear(); queue.clear();
+            int items = 0;
+            size_t head = 0;
+            for (;;) {
+                int a;
+                if (head < queue.size()) {
+                    a = queue[head++];
+                    if (at[a].tile >= 0) continue;
+                } else {
+                    while (next < end && at[next].tile >= 0) ++next;
+                    if (next >= end) break;
+                    a = next;
+                }
+                const int own = at[a].mark == id ? 0 : 1;
+                at[a].tried = ++attempt;
+                fresh.clear();
+                for (int e = rowh_[a]; e < rowh_[a + 1]; ++e) {
+                    Atom& b = at[colh_[e]];
+                    if (b.mark == id || b.tried == attempt) continue;   // an item, or listed twice in the row
+                    b.tried = attempt;
+                    fresh.push_back(colh_[e]);
+                }
+                const int add = own + (int)fresh.size();
+                if (items + add > B) break;      // a tile holds at least one atom: 1 + W <= 17 items
+                items += add;
+                at[a].tile = at[a].mark = id;
+                atom.push_back(a);
+                for (int b : fresh) {
+                    at[b].mark = id;
+                    halo.push_back(b);
+                    if (at[b].tile < 0) queue.push_back(b);
+                }
+            }
+            const int members = (int)(atom.size() - base);
+            for (int b : halo)
+                if (at[b].tile != id) atom.push_back(b);
+            if ((int)(atom.size() - base) != items || items > B)
+                return fail(VMX_ERR_STATE, "tile %d holds %zu items, counted %d", id, atom.size() - base, items);
+            atom.resize(base + B, atom[base]);
+            hdr.push_back(make_int4(members, items, r, 0));
+        }
+    }
+    // one allocation: headers, then the 4-byte, 2-byte and 1-byte arrays
+    const size_t ni = atom.size(), nh = hdr.size() * sizeof(int4), slots = (size_t)W * ni;
+    const size_t jb = jm == JM_UNIFORM ? 0 : (jm == JM_IDX16 ? sizeof(uint16_t) : sizeof(int));
+    const size_t o_atom = nh, o_local = o_atom + 4 * ni, o_nbr = o_local + 4 * ni, o_jid = o_nbr + 4 * slots,
+                 o_lnb = o_jid + jb * slots, o_type = o_lnb + 2 * slots, o_deg = o_type + ni;
+    VMX_TRY(tile_buf.alloc(o_deg + ni));
+    char* p = tile_buf.as<char>();
+    const HostPipe::Seg seg[2] = {{hdr.data(), p, nh}, {atom.data(), p + o_atom, 4 * ni}};
+    VMX_TRY(pipe.move(seg, 2, false, stream));
+    tile = TileDev{B, (int)ni, (int4*)p, (int*)(p + o_atom), (int*)(p + o_local), (uint8_t*)(p + o_type),
+                   (uint8_t*)(p + o_deg), (int*)(p + o_nbr), jb ? (void*)(p + o_jid) : nullptr, (uint16_t*)(p + o_lnb)};
+    VMX_HIP(precision == VMX_FP64 ? Ops<double>::tile_fill(stream, am(), sys<double>(), tile, (int)hdr.size())
+                                  : Ops<float>::tile_fill(stream, am(), sys<float>(), tile, (int)hdr.size()));
+    ntiles = (int)hdr.size();
+    tiles_made = true;
+    drop_graph();                                // recorded from the two kernels
+    return VMX_OK;
+}
+
 // ============================================================================================
 extern "C" {
 
@@ -2384,6 +2513,7 @@ int vmx_llg_heun_graph(vmx_ctx* c, int32_t nsteps, int32_t nrepeat) {
                                    "vmx_llg_heun");
     if (!(c->dt > 0.0)) return fail(VMX_ERR_STATE, "time step not set (vmx_set_time_step)");
     VMX_TRY(c->use_device());
+    VMX_TRY(c->build_tiles((int64_t)nsteps * nrepeat));
     if (!c->graph_exec || c->graph_key != c->graph_key_of(nsteps)) {
         VMX_TRY(c->precision == VMX_FP64 ? c->capture_graph<double>(nsteps) : c->capture_graph<float>(nsteps));
     }

@@ -559,13 +559,26 @@ __device__ __forceinline__ void ext_field(const SysDev<R>& s, int rep, int m, in
     ext_field(s, s.cond[rep * s.nmat + m], rep, i, local, step, noise, ex, ey, ez);
 }
 
+// x y + z, and x y - u v: one rounding fewer in FP32 (explicit fused operations, so that every kernel
+// that forms a Heun step's numbers rounds them alike, whatever the compiler fuses around them); in FP64
+// the products and sums round one by one, as the reference's do.
+__device__ __forceinline__ float mad(float x, float y, float z) { return __builtin_fmaf(x, y, z); }
+__device__ __forceinline__ double mad(double x, double y, double z) { return x * y + z; }
+__device__ __forceinline__ float mulsub(float x, float y, float u, float v) { return __builtin_fmaf(x, y, -(u * v)); }
+__device__ __forceinline__ double mulsub(double x, double y, double u, double v) { return x * y - u * v; }
+// x y + u v
+__device__ __forceinline__ float muladd(float x, float y, float u, float v) { return __builtin_fmaf(x, y, u * v); }
+__device__ __forceinline__ double muladd(double x, double y, double u, double v) { return x * y + u * v; }
+
 // ---- LLG right-hand side, src/simulate/LLGHeun.cpp:201-203 (term order kept) --------------
+// d = a (S x H) + b S x (S x H)
 template <typename R>
 __device__ __forceinline__ void llg_rhs(R a, R b, R S0, R S1, R S2, R H0, R H1, R H2,
                                         R& d0, R& d1, R& d2) {
-    d0 = (a) * (S1 * H2 - S2 * H1) + (b) * (S1 * (S0 * H1 - S1 * H0) - S2 * (S2 * H0 - S0 * H2));
-    d1 = (a) * (S2 * H0 - S0 * H2) + (b) * (S2 * (S1 * H2 - S2 * H1) - S0 * (S0 * H1 - S1 * H0));
-    d2 = (a) * (S0 * H1 - S1 * H0) + (b) * (S0 * (S2 * H0 - S0 * H2) - S1 * (S1 * H2 - S2 * H1));
+    const R g0 = mulsub(S1, H2, S2, H1), g1 = mulsub(S2, H0, S0, H2), g2 = mulsub(S0, H1, S1, H0);
+    d0 = muladd(a, g0, b, mulsub(S1, g2, S2, g1));
+    d1 = muladd(a, g1, b, mulsub(S2, g0, S0, g2));
+    d2 = muladd(a, g2, b, mulsub(S0, g1, S1, g0));
 }
 
 __device__ __forceinline__ double inv_norm(double x, double y, double z) {
@@ -573,6 +586,11 @@ __device__ __forceinline__ double inv_norm(double x, double y, double z) {
 }
 __device__ __forceinline__ float inv_norm(float x, float y, float z) {
     return __builtin_amdgcn_rsqf(x * x + y * y + z * z);
+}
+// the Heun step's, with explicit fused operations in FP32
+__device__ __forceinline__ double step_inv_norm(double x, double y, double z) { return inv_norm(x, y, z); }
+__device__ __forceinline__ float step_inv_norm(float x, float y, float z) {
+    return __builtin_amdgcn_rsqf(mad(z, z, muladd(y, y, x, x)));
 }
 // a / b through the hardware reciprocal (about 1 ulp) in FP32, where b is of order one; an exact
 // division in FP64.
@@ -586,6 +604,38 @@ __device__ __forceinline__ double rcp_div(double a, double b) { return a / b; }
 // reference's order, which is what makes its results equal to the reference bit for bit.
 template <typename R> struct FoldEuler { static constexpr bool value = false; };
 template <> struct FoldEuler<float> { static constexpr bool value = true; };
+
+// The two stages of a Heun step at one atom, from its spin s, field h (spin field + external field)
+// and material: S' = |s + dt d| with d = f(s, h), and S_next from the predicted spin p and the field at
+// it (LLGHeun.cpp:201-217, 257-270).  e: the kept d (FP64; unread in FP32).
+template <typename R>
+__device__ __forceinline__ void heun_predict(const SysDev<R>& s, const MatConst<R>& mc, R sx, R sy, R sz, R hx, R hy,
+                                             R hz, R& d0, R& d1, R& d2, R& px, R& py, R& pz) {
+    llg_rhs(mc.one_opa2, mc.alpha_opa2, sx, sy, sz, hx, hy, hz, d0, d1, d2);
+    const R n0 = mad(d0, s.dt, sx), n1 = mad(d1, s.dt, sy), n2 = mad(d2, s.dt, sz);
+    const R r = step_inv_norm(n0, n1, n2);
+    px = n0 * r; py = n1 * r; pz = n2 * r;
+}
+template <typename R>
+__device__ __forceinline__ void heun_correct(const SysDev<R>& s, const MatConst<R>& mc, R sx, R sy, R sz, R px, R py,
+                                             R pz, R hx, R hy, R hz, R e0, R e1, R e2, R& o0, R& o1, R& o2) {
+    R h0, h1, h2, n0, n1, n2;
+    llg_rhs(mc.one_opa2, mc.alpha_opa2, px, py, pz, hx, hy, hz, h0, h1, h2);
+    if constexpr (FoldEuler<R>::value) {
+        // A = S + dt/2 dS from S and S' = (S + dt dS) / |S + dt dS|: dS is orthogonal to S, so
+        // the norm is |S|^2 / (S . S') and A = (S + N S') / 2
+        const R N = rcp_div(mad(sz, sz, muladd(sy, sy, sx, sx)), mad(sz, pz, muladd(sy, py, sx, px)));
+        n0 = muladd(s.half_dt, h0, R(0.5), mad(N, px, sx));
+        n1 = muladd(s.half_dt, h1, R(0.5), mad(N, py, sy));
+        n2 = muladd(s.half_dt, h2, R(0.5), mad(N, pz, sz));
+    } else {
+        n0 = sx + s.half_dt * (e0 + h0);
+        n1 = sy + s.half_dt * (e1 + h1);
+        n2 = sz + s.half_dt * (e2 + h2);
+    }
+    const R r = step_inv_norm(n0, n1, n2);
+    o0 = n0 * r; o1 = n1 * r; o2 = n2 * r;
+}
 
 // Atoms per thread of the fused predictors: a workgroup of B threads takes FusedAtoms * B
 // consecutive atoms of its block-table entry (thread t: t, t + B, ...).  The loads of every
@@ -739,10 +789,8 @@ k_fused_predictor(SysDev<R> s, Spin3<R> S, Spin3<R> P, Spin3<R> D, Spin3<R> E, c
         const Cond<R>& c = FusedLds<R>::cond(s)[m[u]];
         R ex, ey, ez;
         ext_from_normals(s, c, i, gx[u], gy[u], gz[u], ex, ey, ez);
-        R d0, d1, d2;
-        llg_rhs(mc.one_opa2, mc.alpha_opa2, sx[u], sy[u], sz[u], fx + ex, fy + ey, fz + ez, d0, d1, d2);
-        R n0 = sx[u] + d0 * s.dt, n1 = sy[u] + d1 * s.dt, n2 = sz[u] + d2 * s.dt;
-        const R r = inv_norm(n0, n1, n2);
+        R d0, d1, d2, p0, p1, p2;
+        heun_predict(s, mc, sx[u], sy[u], sz[u], fx + ex, fy + ey, fz + ez, d0, d1, d2, p0, p1, p2);
         if (ok[u]) {
             if constexpr (!FoldEuler<R>::value) {
                 if (D.x) { D.x[i] = d0; D.y[i] = d1; D.z[i] = d2; }
@@ -750,7 +798,7 @@ k_fused_predictor(SysDev<R> s, Spin3<R> S, Spin3<R> P, Spin3<R> D, Spin3<R> E, c
             if (E.x) {
                 E.x[i] = ex; E.y[i] = ey; E.z[i] = ez;
             }
-            P.x[i] = n0 * r; P.y[i] = n1 * r; P.z[i] = n2 * r;
+            P.x[i] = p0; P.y[i] = p1; P.z[i] = p2;
         }
     }
 }
@@ -820,19 +868,8 @@ k_fused_corrector(SysDev<R> s, Spin3Alias<R> S, Spin3<R> P, Spin3Alias<R> O, Spi
             const Cond<R>& c = FusedLds<R>::cond(s)[m[u]];
             ext_from_normals(s, c, i, gx[u], gy[u], gz[u], ex, ey, ez);
         }
-        R h0, h1, h2;
-        llg_rhs(mc.one_opa2, mc.alpha_opa2, px[u], py[u], pz[u], fx + ex, fy + ey, fz + ez, h0, h1, h2);
-        R n0, n1, n2;
-        if (fold) {
-            // A = S + dt/2 dS from S and S' = (S + dt dS) / |S + dt dS|: dS is orthogonal to S, so
-            // the norm is |S|^2 / (S . S') and A = (S + N S') / 2
-            const R N = rcp_div(ax[u] * ax[u] + ay[u] * ay[u] + az[u] * az[u],
-                                ax[u] * px[u] + ay[u] * py[u] + az[u] * pz[u]);
-            n0 = R(0.5) * (ax[u] + N * px[u]) + s.half_dt * h0;
-            n1 = R(0.5) * (ay[u] + N * py[u]) + s.half_dt * h1;
-            n2 = R(0.5) * (az[u] + N * pz[u]) + s.half_dt * h2;
-        } else {
-            R e0, e1, e2;
+        R e0 = R(0), e1 = R(0), e2 = R(0);
+        if (!fold) {
             if (keep) {
                 e0 = dx[u]; e1 = dy[u]; e2 = dz[u];
             } else {
@@ -845,13 +882,12 @@ k_fused_corrector(SysDev<R> s, Spin3Alias<R> S, Spin3<R> P, Spin3Alias<R> O, Spi
                 }
                 llg_rhs(mc.one_opa2, mc.alpha_opa2, ax[u], ay[u], az[u], gx + ex, gy + ey, gz + ez, e0, e1, e2);
             }
-            n0 = ax[u] + s.half_dt * (e0 + h0);
-            n1 = ay[u] + s.half_dt * (e1 + h1);
-            n2 = az[u] + s.half_dt * (e2 + h2);
         }
-        const R r = inv_norm(n0, n1, n2);
+        R o0, o1, o2;
+        heun_correct(s, mc, ax[u], ay[u], az[u], px[u], py[u], pz[u], fx + ex, fy + ey, fz + ez, e0, e1, e2, o0, o1,
+                     o2);
         if (ok[u]) {
-            O.x[i] = n0 * r; O.y[i] = n1 * r; O.z[i] = n2 * r;
+            O.x[i] = o0; O.y[i] = o1; O.z[i] = o2;
         }
     }
 }
@@ -1001,6 +1037,142 @@ k_mid_corrector(SysDev<R> s, Spin3Alias<R> S, Spin3<R> P, Spin3Alias<R> O, Spin3
             O.x[i] = o0; O.y[i] = o1; O.z[i] = o2;
         }
     }
+}
+
+// ======================= whole-step kernel: one launch per step for small systems ============
+// A system that leaves most of the chip idle is bound by its launches' dependent memory round trips,
+// not by its arithmetic: on SC 20^3 in FP64 the predictor and the corrector each took 4.75 us for 8000
+// atoms.  Here a workgroup owns a tile of atoms and forms the predicted spins of the tile and of its
+// halo (every neighbour of a tile atom outside the tile) itself, one atom per thread, leaves them in
+// LDS, and corrects the tile's atoms from there: a step is one launch with two levels of global loads
+// (the item's record; the spins) instead of two launches with three each, and a tile atom's thermal
+// field, spin and Euler derivative stay in its thread's registers.  The price is that halo atoms are
+// predicted by every tile that touches them (1.0-1.8 halo atoms per tile atom at 256 items a tile).
+// Every atom's arithmetic is that of the two-kernel step, in the same order.
+struct TileDev {
+    int block;                               // items per tile = threads per workgroup
+    int ni;                                  // tiles * block: stride of the slot arrays
+    const int4* __restrict__ hdr;            // [tile] {tile atoms, items, replica, 0}
+    int* __restrict__ atom;                  // [ni] the item's atom (tile atoms first, then the halo; past the
+                                             //      items: a tile atom, never stored)
+    int* __restrict__ local;                 // [ni] its caller index within the replica (Philox counter)
+    uint8_t* __restrict__ type;              // [ni]
+    uint8_t* __restrict__ deg;               // [ni]
+    int* __restrict__ nbr;                   // [W][ni] neighbours (internal atom index; padding: in bounds)
+    void* __restrict__ jid;                  // [W][ni] J table index (16/32-bit J modes)
+    uint16_t* __restrict__ lnb;              // [W][ni] tile atoms: the neighbours' items within the tile
+};
+enum { STEP_HEUN = 0, STEP_MIDPOINT = 1 };
+
+// Fills the slot arrays from the tiles' atoms (hdr, atom) and the context's own rows, once per context.
+// Both runs of items are sorted first (each item's rank is the number of smaller ones in its run, read
+// from LDS by all lanes at once), so that neighbouring threads load and store neighbouring atoms and a
+// neighbour's item is found by bisection.
+template <typename R, int AM>
+__global__ void __launch_bounds__(512) k_tile_fill(SysDev<R> s, TileDev t) {
+    if constexpr (Access<AM>::TP != TP_CSR) {
+        constexpr int W = Access<AM>::W, JM = Access<AM>::JM;
+        int* const given = vmx_lds;              // the tile's atoms as given, then sorted
+        int* const items = vmx_lds + t.block;
+        const int tid = (int)threadIdx.x;
+        const size_t e = (size_t)blockIdx.x * (size_t)t.block + (size_t)tid;
+        const int4 h = t.hdr[blockIdx.x];
+        given[tid] = t.atom[e];
+        __syncthreads();
+        if (tid < h.y) {
+            const int first = tid < h.x ? 0 : h.x, last = tid < h.x ? h.x : h.y, mine = given[tid];
+            int rank = first;
+            for (int k = first; k < last; ++k) rank += given[k] < mine ? 1 : 0;
+            items[rank] = mine;
+        }
+        __syncthreads();
+        const int i = items[tid < h.y ? tid : 0];
+        t.atom[e] = i;
+        RowIdx<AM> r;
+        row_index(s, i, row_head<R, AM>(s, i), s.pat_off, r);
+        t.local[e] = caller_local(s, h.z, i - s.rep_off[h.z]);
+        t.type[e] = s.type[i];
+        t.deg[e] = (uint8_t)r.deg;
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            const size_t o = (size_t)k * t.ni + e;
+            const int j = k < r.deg ? r.j[k] : i;
+            t.nbr[o] = j;
+            if (JM == JM_IDX16) ((uint16_t*)t.jid)[o] = (uint16_t)r.jd[k];
+            if (JM == JM_IDX32) ((int*)t.jid)[o] = r.jd[k];
+            int item = 0;
+            if (tid < h.x) {                     // j is a tile atom or in the halo: search both runs
+                int lo = 0, hi = h.x;
+                while (lo < hi) { const int mid = (lo + hi) >> 1; if (items[mid] < j) lo = mid + 1; else hi = mid; }
+                if (lo < h.x && items[lo] == j) {
+                    item = lo;
+                } else {
+                    lo = h.x; hi = h.y;
+                    while (lo < hi) { const int mid = (lo + hi) >> 1; if (items[mid] < j) lo = mid + 1; else hi = mid; }
+                    item = lo < h.y ? lo : 0;
+                }
+            }
+            t.lnb[o] = (uint16_t)item;
+        }
+    }
+}
+
+// AM: an ELL access mode (slot width and J mode), whatever layout the context's own rows have.
+template <typename R, int ET, int AM, int STEP>
+__global__ void __launch_bounds__(512)
+k_tile_step(SysDev<R> s, TileDev t, Spin3<R> S, Spin3<R> O, const double* __restrict__ noise, uint32_t step_off) {
+    constexpr int W = Access<AM>::W, JM = Access<AM>::JM;
+    R* const lx = reinterpret_cast<R*>(vmx_lds);
+    R* const ly = lx + t.block;
+    R* const lz = ly + t.block;
+    const int tid = (int)threadIdx.x;
+    const size_t e = (size_t)blockIdx.x * (size_t)t.block + (size_t)tid;
+    const int i = t.atom[e], local = t.local[e];
+    RowIdx<AM> r;
+    r.deg = s.full_rows ? W : (int)t.deg[e];
+    int q[W];
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+        r.j[k] = t.nbr[(size_t)k * t.ni + e];
+        if (JM == JM_IDX16) r.jd[k] = ((const uint16_t*)t.jid)[(size_t)k * t.ni + e];
+        if (JM == JM_IDX32) r.jd[k] = ((const int*)t.jid)[(size_t)k * t.ni + e];
+        q[k] = t.lnb[(size_t)k * t.ni + e];
+    }
+    const int m = s.nmat == 1 ? 0 : (int)t.type[e];
+    const int4 h = t.hdr[blockIdx.x];
+    const uint64_t step = *s.step_base + step_off;
+    const SpinRsrc<R> rs(s, S.x, S.y, S.z);
+    R sx, sy, sz;
+    rs.load(i, sx, sy, sz);
+    RowSpins<R, AM> v;
+    row_load(rs, r, v);
+    R gx = R(0), gy = R(0), gz = R(0);       // while the gathers are in flight
+    if (s.fld & FLD_THERMAL) unit_normals(s, h.z, i, local, step, noise, gx, gy, gz);
+    const MatConst<R>& mc = s.mat[m];
+    const Cond<R>& c = s.cond[h.z * s.nmat + m];
+    const UniformJ<R, ET> ju(s, JM);
+    R fx, fy, fz, ex, ey, ez, px, py, pz, d0 = R(0), d1 = R(0), d2 = R(0);
+    row_field<R, ET, AM>(s, r, v, ju.v, mc, sx, sy, sz, fx, fy, fz);
+    ext_from_normals(s, c, i, gx, gy, gz, ex, ey, ez);
+    if constexpr (STEP == STEP_HEUN) {
+        heun_predict(s, mc, sx, sy, sz, fx + ex, fy + ey, fz + ez, d0, d1, d2, px, py, pz);
+    } else {
+        R o0, o1, o2;
+        cayley(mc.alpha, midpoint_beta(s, mc), sx, sy, sz, fx + ex, fy + ey, fz + ez, sx, sy, sz, o0, o1, o2);
+        px = (sx + o0) * R(0.5); py = (sy + o1) * R(0.5); pz = (sz + o2) * R(0.5);
+    }
+    lx[tid] = px; ly[tid] = py; lz[tid] = pz;
+    __syncthreads();
+    if (tid >= h.x) return;
+#pragma unroll
+    for (int k = 0; k < W; ++k) { v.x[k] = lx[q[k]]; v.y[k] = ly[q[k]]; v.z[k] = lz[q[k]]; }
+    row_field<R, ET, AM>(s, r, v, ju.v, mc, px, py, pz, fx, fy, fz);
+    R o0, o1, o2;
+    if constexpr (STEP == STEP_HEUN)
+        heun_correct(s, mc, sx, sy, sz, px, py, pz, fx + ex, fy + ey, fz + ez, d0, d1, d2, o0, o1, o2);
+    else
+        cayley(mc.alpha, midpoint_beta(s, mc), px, py, pz, fx + ex, fy + ey, fz + ez, sx, sy, sz, o0, o1, o2);
+    O.x[i] = o0; O.y[i] = o1; O.z[i] = o2;
 }
 
 // ======================= plain kernels: the reference dataflow ==============================

@@ -33,6 +33,12 @@ struct Ops {
                                     Spin3<R> E, const double* noise, uint32_t step_off);
     static hipError_t mid_corrector(const Launch& L, int et, int jm, const SysDev<R>& s, Spin3<R> S, Spin3<R> P,
                                     Spin3<R> O, Spin3<R> E, const double* noise, uint32_t step_off);
+    // a whole Heun (STEP_HEUN) or midpoint (STEP_MIDPOINT) step: O from S, one workgroup per tile.
+    // jm, wsel: the rows' J mode and slot width (kSlotWidths)
+    static hipError_t tile_step(hipStream_t st, int et, int jm, int wsel, int kind, const SysDev<R>& s, const TileDev& t,
+                                int ntiles, Spin3<R> S, Spin3<R> O, const double* noise, uint32_t step_off);
+    // fills the tiles' slot arrays from the system's rows
+    static hipError_t tile_fill(hipStream_t st, int am, const SysDev<R>& s, const TileDev& t, int ntiles);
     // plain Heun step
     static hipError_t spin_fields(const Launch& L, int et, int jm, const SysDev<R>& s, Spin3<R> S, Spin3<R> F);
     static hipError_t ext_fields(const Launch& L, const SysDev<R>& s, Spin3<R> E, const double* noise,

@@ -358,14 +358,15 @@ typedef struct vmx_fit_params {
 } vmx_fit_params;
 
 /* Runs nsteps steps from spins0 [3][N] and writes <m_z> after every record_every steps to
- * mz [nsteps/record_every].  Keeps a checkpoint every checkpoint_every steps for the adjoint.
+ * mz [nsteps/record_every].  While the predicted and corrected spins of every step fit 8 GiB of
+ * device memory, all are kept for the adjoint; else a checkpoint every checkpoint_every steps.
  * h: per-site field [3][N] or NULL.  nsteps must be a multiple of record_every. */
 int vmx_fit_forward(vmx_ctx* ctx, const vmx_fit_params* p, const double* h, const double* spins0,
                     int32_t nsteps, int32_t record_every, int32_t checkpoint_every, double* mz);
 
 /* Discrete adjoint of the last vmx_fit_forward: given dL/d<m_z> [nsteps/record_every], writes
- * grad = {dL/dJ, dL/dku2, dL/dalpha} and, if dL_dh is not NULL, dL/dh_i [3][N].  Segments between
- * checkpoints are recomputed forward, then swept backward (hand-written adjoint kernels). */
+ * grad = {dL/dJ, dL/dku2, dL/dalpha} and, if dL_dh is not NULL, dL/dh_i [3][N].  The steps are swept backward
+ * over the kept trajectory, or over segments recomputed from the checkpoints (hand-written adjoint kernels). */
 int vmx_fit_backward(vmx_ctx* ctx, const double* dL_dmz, double* grad, double* dL_dh);
 
 /* Chooses the workgroup size (64, 128, 256, 512) and whether workgroups are remapped to give

@@ -255,14 +255,6 @@ using EnergyStat = Statistic<5>;
 __global__ void k_advance_step(unsigned long long* base, unsigned int n) { *base += n; }
 __global__ void k_set_step(unsigned long long* base, unsigned long long v) { *base = v; }
 
-// adds dL/dS_z (the same for every atom) to the adjoint of a recorded state
-template <typename R>
-__global__ void k_lam_inject(int n, R* __restrict__ lz, const R* __restrict__ inj) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const R v = *inj;
-    if (i < n && v != R(0)) lz[i] += v;
-}
-
 template <typename R>
 __global__ void k_fill(size_t n, R* __restrict__ a, R v) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
@@ -987,27 +979,43 @@ struct vmx_ctx {
     int mc_sweeps(int nsweeps);
     int colour();
 
-    // deterministic fitting trajectory and its adjoint
+    // Deterministic fitting trajectory and its adjoint.  A segment of G steps lies in `seg`: states
+    // S_0 .. S_G, then (keepP) the predicted P_0 .. P_{G-1}.  While every S and P of the trajectory fits
+    // kFitResident, they are kept (traj: per segment S_1 .. S_G, P_0 .. P_{G-1}) and the backward pass
+    // recomputes nothing; else the forward pass keeps a checkpoint every K steps and the backward pass
+    // recomputes a segment of K before it steps back over it.  Segments of equal length replay graphs
+    // whose kernels read the parameters from device memory, so one recording serves every call until a
+    // buffer moves.
     struct Fit {
         bool ready = false;
         int nsteps = 0, record_every = 1, K = 100, nrec = 0;
         double J = 0, k = 0, alpha = 0, gamma_rel = 1, H[3] = {0, 0, 0};
         bool has_h = false;
-        DevBuf ckpt, seg, P, lam, lH1, lPd, lT, H0, sumS, lH0, lSp, dh, nhat, h, acc, mz;
-        // backward: dL/dm_z injections per step (inj[q], zero between records) and the slice of
-        // the segment being replayed (inj_seg[K]); the graph of one full segment, captured by
-        // each backward call (its kernels take that call's buffers and parameters) and replayed
-        // for every full segment
+        bool resident = false, keepP = false;
+        int G = 1;                // steps of a full segment
+        DevBuf prm, traj, ckpt, seg, P, lH1, lPd, lT, H0, sumS, lH0, lSp, dh, nhat, h, acc, mz;
+        // backward: dL/dm_z injections per step (inj[q], zero between records) and the slice of the
+        // segment being replayed (inj_seg[G])
         DevBuf inj, inj_seg;
-        hipGraph_t graph = nullptr;
-        hipGraphExec_t graph_exec = nullptr;
-        void drop_graph() {
-            if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
-            if (graph) (void)hipGraphDestroy(graph);
-            graph_exec = nullptr;
-            graph = nullptr;
-        }
+        struct Replay {           // a recorded segment and the addresses its kernels hold
+            hipGraph_t graph = nullptr;
+            hipGraphExec_t exec = nullptr;
+            std::vector<const void*> key;
+            void drop() {
+                if (exec) (void)hipGraphExecDestroy(exec);
+                if (graph) (void)hipGraphDestroy(graph);
+                exec = nullptr;
+                graph = nullptr;
+                key.clear();
+            }
+        } fwd, bwd;
+        void drop_graph() { fwd.drop(); bwd.drop(); }
     } fit;
+    template <typename F>
+    int fit_replay(Fit::Replay& r, const std::vector<const void*>& key, F&& record);
+    static constexpr size_t kFitResident = (size_t)8 << 30;   // bytes: 3 % of this device's memory
+    static constexpr int kFitSegment = 50;                    // steps of a recorded segment
+    static constexpr int kFitParts = 8;                       // partial sums of a recorded state's S_z
     bool symmetric_checked = false, symmetric = false;
     template <typename R>
     FitPrm<R> fit_prm() const;
@@ -1683,139 +1691,188 @@ FitPrm<R> vmx_ctx::fit_prm() const {
     return p;
 }
 
+// Replays r, recorded anew when the addresses it holds (key) have changed.
+template <typename F>
+int vmx_ctx::fit_replay(Fit::Replay& r, const std::vector<const void*>& key, F&& record) {
+    if (!r.exec || r.key != key) {
+        r.drop();
+        VMX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+        const hipError_t e = record();
+        const hipError_t ec = hipStreamEndCapture(stream, &r.graph);
+        if (e != hipSuccess || ec != hipSuccess) {
+            r.drop();
+            return fail(VMX_ERR_HIP, "fitting segment capture failed: %s", hipGetErrorString(e != hipSuccess ? e : ec));
+        }
+        const hipError_t ei = hipGraphInstantiate(&r.exec, r.graph, nullptr, nullptr, 0);
+        if (ei != hipSuccess) {
+            r.exec = nullptr;
+            r.drop();
+            return fail(VMX_ERR_HIP, "fitting segment graph failed: %s", hipGetErrorString(ei));
+        }
+        r.key = key;
+    }
+    VMX_HIP(hipGraphLaunch(r.exec, stream));
+    return VMX_OK;
+}
+
 template <typename R>
 int vmx_ctx::fit_forward(const double* h, const double* spins0, double* mz_out) {
-    const size_t N3 = 3 * (size_t)n;
-    const int nck = fit.nsteps / fit.K + 1;
-    VMX_TRY(fit.ckpt.alloc((size_t)nck * N3 * sizeof(R)));
-    VMX_TRY(fit.seg.alloc((size_t)(fit.K + 1) * N3 * sizeof(R)));
-    VMX_TRY(fit.P.alloc(N3 * sizeof(R)));
-    VMX_TRY(fit.h.alloc(N3 * sizeof(R)));
-    VMX_TRY(fit.mz.alloc((size_t)4 * std::max(fit.nrec, 1) * sizeof(double)));
+    const size_t N3 = 3 * (size_t)n, sb = N3 * sizeof(R);   // reals and bytes of a state
+    fit.ready = false;
+    VMX_HIP(hipStreamSynchronize(stream));         // a buffer that grows is freed: nothing may use it
+    const int Gr = std::min(fit.nsteps, kFitSegment);
+    const size_t all = 2 * (size_t)((fit.nsteps + Gr - 1) / Gr) * Gr * sb;
+    fit.resident = all <= kFitResident && fit.traj.alloc(all) == VMX_OK;
+    if (!fit.resident) (void)hipGetLastError();    // no room for the trajectory: checkpoints
+    fit.G = fit.resident ? Gr : std::min(fit.K, fit.nsteps);
+    fit.keepP = fit.resident || 2 * (size_t)fit.G * sb <= kFitResident;
+    const int G = fit.G, nseg = (fit.nsteps + G - 1) / G;
+    VMX_TRY(fit.ckpt.alloc((size_t)(fit.resident ? 1 : nseg) * sb));
+    VMX_TRY(fit.seg.alloc((size_t)(fit.keepP ? 2 * G + 1 : G + 1) * sb));
+    if (!fit.keepP) VMX_TRY(fit.P.alloc(sb));
+    VMX_TRY(fit.h.alloc(sb));
+    const int parts = std::max(1, std::min(kFitParts, n / 4096));
+    VMX_TRY(fit.mz.alloc((size_t)parts * std::max(fit.nrec, 1) * sizeof(double)));
+    VMX_TRY(fit.prm.alloc(sizeof(FitPrm<R>)));
     fit.has_h = h != nullptr;
     R* ck = fit.ckpt.as<R>();
-    auto state = [&](R* base) { return Spin3<R>{base, base + n, base + 2 * (size_t)n}; };
-    if (h) VMX_TRY(upload3(h, h + n, h + 2 * (size_t)n, arr3<R>(fit.h)));
-    VMX_TRY(upload3(spins0, spins0 + n, spins0 + 2 * (size_t)n, state(ck)));
-    VMX_HIP(hipMemsetAsync(fit.mz.p, 0, (size_t)4 * std::max(fit.nrec, 1) * sizeof(double), stream));
-    const SysDev<R> s = sys<R>();
-    const FitPrm<R> p = fit_prm<R>();
-    const Spin3<R> hh = fit.has_h ? arr3<R>(fit.h) : Spin3<R>{nullptr, nullptr, nullptr};
     R* seg = fit.seg.as<R>();
-    R* cur = seg;
-    R* nxt = seg + N3;
-    VMX_HIP(hipMemcpyAsync(cur, ck, N3 * sizeof(R), hipMemcpyDeviceToDevice, stream));
-    for (int q = 0; q < fit.nsteps; ++q) {
-        VMX_HIP(Ops<R>::fit_predictor(stream, am(), s, p, hh, state(cur), arr3<R>(fit.P)));
-        VMX_HIP(Ops<R>::fit_corrector(stream, am(), s, p, hh, state(cur), arr3<R>(fit.P), state(nxt)));
-        std::swap(cur, nxt);
-        if ((q + 1) % fit.K == 0)
-            VMX_HIP(hipMemcpyAsync(ck + (size_t)((q + 1) / fit.K) * N3, cur, N3 * sizeof(R), hipMemcpyDeviceToDevice,
-                                   stream));
-        if ((q + 1) % fit.record_every == 0)
-            VMX_HIP(Ops<R>::fit_mz(stream, n, state(cur), fit.mz.as<double>() + 4 * (size_t)((q + 1) / fit.record_every - 1)));
+    auto state = [&](R* base) { return Spin3<R>{base, base + n, base + 2 * (size_t)n}; };
+    const FitPrm<R> p = fit_prm<R>();
+    const HostPipe::Seg ps{const_cast<FitPrm<R>*>(&p), fit.prm.p, sizeof p};
+    VMX_TRY(pipe.move(&ps, 1, false, stream));
+    if (h) VMX_TRY(upload3(h, h + n, h + 2 * (size_t)n, arr3<R>(fit.h)));
+    VMX_TRY(upload3(spins0, spins0 + n, spins0 + 2 * (size_t)n, state(seg)));
+    const SysDev<R> s = sys<R>();
+    const Spin3<R> hh = fit.has_h ? arr3<R>(fit.h) : Spin3<R>{nullptr, nullptr, nullptr};
+    const FitPrm<R>* pp = fit.prm.as<FitPrm<R>>();
+    auto segment = [&](int len) -> hipError_t {
+        for (int t = 0; t < len; ++t) {
+            R* a = seg + (size_t)t * N3;
+            const Spin3<R> P = fit.keepP ? state(seg + (size_t)(G + 1 + t) * N3) : arr3<R>(fit.P);
+            hipError_t e = Ops<R>::fit_predictor(stream, am(), s, pp, hh, state(a), P);
+            if (e == hipSuccess) e = Ops<R>::fit_corrector(stream, am(), s, pp, hh, state(a), P, state(a + N3));
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    };
+    const std::vector<const void*> key = {seg, fit.P.p, hh.x, pp, (const void*)(intptr_t)(2 * G + (fit.keepP ? 1 : 0))};
+    const bool replay = fit.nsteps / G >= 2;
+    for (int c = 0; c < nseg; ++c) {
+        const int start = c * G, len = std::min(G, fit.nsteps - start);
+        if (c) VMX_HIP(hipMemcpyAsync(seg, seg + (size_t)G * N3, sb, hipMemcpyDeviceToDevice, stream));
+        if (!fit.resident || c == 0)
+            VMX_HIP(hipMemcpyAsync(ck + (size_t)c * N3, seg, sb, hipMemcpyDeviceToDevice, stream));
+        if (replay && len == G) VMX_TRY(fit_replay(fit.fwd, key, [&] { return segment(G); }));
+        else VMX_HIP(segment(len));
+        if (fit.resident)
+            VMX_HIP(hipMemcpyAsync(fit.traj.as<R>() + (size_t)c * 2 * G * N3, seg + N3,
+                                   (size_t)(len == G ? 2 * G : G + len) * sb, hipMemcpyDeviceToDevice, stream));
+        // recorded states: those after a multiple of record_every steps
+        const int first = (start / fit.record_every + 1) * fit.record_every;
+        if (first <= start + len)
+            VMX_HIP(Ops<R>::fit_mz(stream, n, seg + (size_t)(first - start) * N3 + 2 * (size_t)n,
+                                   (size_t)fit.record_every * N3, (start + len - first) / fit.record_every + 1, parts,
+                                   fit.mz.as<double>() + (size_t)(first / fit.record_every - 1) * parts));
     }
-    std::vector<double> mzh((size_t)4 * std::max(fit.nrec, 1));
-    VMX_HIP(hipStreamSynchronize(stream));
-    VMX_HIP(hipMemcpy(mzh.data(), fit.mz.p, mzh.size() * sizeof(double), hipMemcpyDeviceToHost));
-    for (int r = 0; r < fit.nrec; ++r) mz_out[r] = mzh[4 * (size_t)r] / n;
+    std::vector<double> mzh((size_t)parts * std::max(fit.nrec, 1));
+    const HostPipe::Seg ms{mzh.data(), fit.mz.p, mzh.size() * sizeof(double)};
+    VMX_TRY(pipe.move(&ms, 1, true, stream));
+    for (int r = 0; r < fit.nrec; ++r) {
+        double t = 0.0;
+        for (int k = 0; k < parts; ++k) t += mzh[(size_t)r * parts + k];
+        mz_out[r] = t / n;
+    }
     fit.ready = true;
     return VMX_OK;
 }
 
 template <typename R>
 int vmx_ctx::fit_backward(const double* dmz, double* grad, double* dh_out) {
-    const size_t N3 = 3 * (size_t)n;
-    for (DevBuf* b : {&fit.lam, &fit.lH1, &fit.lPd, &fit.lT, &fit.H0, &fit.sumS, &fit.lH0, &fit.lSp, &fit.dh})
-        VMX_TRY(b->alloc(N3 * sizeof(R)));
+    const size_t N3 = 3 * (size_t)n, sb = N3 * sizeof(R);
+    const int G = fit.G, nseg = (fit.nsteps + G - 1) / G;
+    for (DevBuf* b : {&fit.lH1, &fit.lPd, &fit.lT, &fit.H0, &fit.sumS, &fit.lH0, &fit.lSp, &fit.dh})
+        VMX_TRY(b->alloc(sb));
     VMX_TRY(fit.nhat.alloc((size_t)n * sizeof(R)));
-    const int nwg = (n + 255) / 256;   // workgroups of the backward kernels: one slot of 4 sums each
-    VMX_TRY(fit.acc.alloc((size_t)4 * nwg * sizeof(double)));
+    const int nwave = (n + 255) / 256 * 4;   // wavefronts of the backward kernels: one slot of 4 sums each
+    VMX_TRY(fit.acc.alloc((size_t)4 * nwave * sizeof(double)));
     const SysDev<R> s = sys<R>();
-    const FitPrm<R> p = fit_prm<R>();
     const Spin3<R> hh = fit.has_h ? arr3<R>(fit.h) : Spin3<R>{nullptr, nullptr, nullptr};
+    const FitPrm<R>* pp = fit.prm.as<FitPrm<R>>();
     auto state = [&](R* base) { return Spin3<R>{base, base + n, base + 2 * (size_t)n}; };
-    const int fill_grid = (int)std::min<size_t>((N3 + 255) / 256, 4096);
-    hipLaunchKernelGGL((k_fill<R>), dim3(fill_grid), dim3(256), 0, stream, N3, fit.lam.as<R>(), (R)0);
-    hipLaunchKernelGGL((k_fill<R>), dim3(fill_grid), dim3(256), 0, stream, N3, fit.dh.as<R>(), (R)0);
-    hipLaunchKernelGGL((k_fill<double>), dim3(std::min(nwg, 1024)), dim3(64), 0, stream, (size_t)4 * nwg,
+    auto clear = [&](DevBuf& b, size_t count) {
+        hipLaunchKernelGGL((k_fill<R>), dim3((int)std::min<size_t>((count + 255) / 256, 4096)), dim3(256), 0, stream,
+                           count, b.as<R>(), (R)0);
+    };
+    clear(fit.lH0, N3);
+    clear(fit.lSp, N3);
+    clear(fit.dh, N3);
+    hipLaunchKernelGGL((k_fill<double>), dim3(std::min(nwave / 4, 1024)), dim3(256), 0, stream, (size_t)4 * nwave,
                        fit.acc.as<double>(), 0.0);
     VMX_HIP(hipGetLastError());
     R* ck = fit.ckpt.as<R>();
     R* seg = fit.seg.as<R>();
-    const Spin3<R> lam = arr3<R>(fit.lam);
-    const int nseg = (fit.nsteps + fit.K - 1) / fit.K;
     // dL/dm_z enters lambda_z after step q when q + 1 is a recorded step (zero elsewhere)
     {
         std::vector<R> inj((size_t)fit.nsteps, R(0));
         for (int q = 0; q < fit.nsteps; ++q)
             if ((q + 1) % fit.record_every == 0) inj[q] = (R)(dmz[(q + 1) / fit.record_every - 1] / n);
-        VMX_TRY(upload(fit.inj, inj));
-        VMX_TRY(fit.inj_seg.alloc((size_t)fit.K * sizeof(R)));
+        VMX_TRY(fit.inj.alloc(inj.size() * sizeof(R)));
+        const HostPipe::Seg is{inj.data(), fit.inj.p, inj.size() * sizeof(R)};
+        VMX_TRY(pipe.move(&is, 1, false, stream));
+        VMX_TRY(fit.inj_seg.alloc((size_t)G * sizeof(R)));
     }
-    // One segment: recompute its states from the checkpoint in seg[0], then step back over them.
-    // inj: the segment's injections (inj[t] after local step t).  The same sequence for every
-    // full segment, so it is captured once and replayed.
+    // One segment: its states recomputed from the checkpoint in seg[0] unless the trajectory was kept,
+    // then the steps back over them.  inj: the segment's injections (inj[t] after local step t).
     auto segment = [&](int len, const R* inj) -> hipError_t {
-        for (int t = 0; t < len; ++t) {
+        hipError_t e = hipSuccess;
+        auto P = [&](int t) { return fit.keepP ? state(seg + (size_t)(G + 1 + t) * N3) : arr3<R>(fit.P); };
+        for (int t = 0; t < len && !fit.resident && e == hipSuccess; ++t) {
             R* a = seg + (size_t)t * N3;
-            hipError_t e = Ops<R>::fit_predictor(stream, am(), s, p, hh, state(a), arr3<R>(fit.P));
-            if (e == hipSuccess) e = Ops<R>::fit_corrector(stream, am(), s, p, hh, state(a), arr3<R>(fit.P),
-                                                          state(a + N3));
-            if (e != hipSuccess) return e;
+            e = Ops<R>::fit_predictor(stream, am(), s, pp, hh, state(a), P(t));
+            if (e == hipSuccess) e = Ops<R>::fit_corrector(stream, am(), s, pp, hh, state(a), P(t), state(a + N3));
         }
-        for (int t = len - 1; t >= 0; --t) {
-            hipLaunchKernelGGL((k_lam_inject<R>), dim3((n + 255) / 256), dim3(256), 0, stream, n, lam.z, inj + t);
-            hipError_t e = hipGetLastError();
-            R* a = seg + (size_t)t * N3;
-            if (e == hipSuccess) e = Ops<R>::fit_predictor(stream, am(), s, p, hh, state(a), arr3<R>(fit.P));
+        for (int t = len - 1; t >= 0 && e == hipSuccess; --t) {
+            const Spin3<R> S = state(seg + (size_t)t * N3);
+            if (!fit.keepP) e = Ops<R>::fit_predictor(stream, am(), s, pp, hh, S, P(t));
             if (e == hipSuccess)
-                e = Ops<R>::adj_b1(stream, am(), s, p, hh, state(a), arr3<R>(fit.P), lam, arr3<R>(fit.lH1),
-                                   arr3<R>(fit.lPd), arr3<R>(fit.lT), arr3<R>(fit.H0), arr3<R>(fit.sumS),
-                                   fit.nhat.as<R>(), fit.acc.as<double>());
+                e = Ops<R>::adj_a(stream, am(), s, pp, hh, S, P(t), arr3<R>(fit.lH0), arr3<R>(fit.lSp), inj + t,
+                                  arr3<R>(fit.lH1), arr3<R>(fit.lPd), arr3<R>(fit.lT), arr3<R>(fit.H0),
+                                  arr3<R>(fit.sumS), fit.nhat.as<R>(), fit.acc.as<double>());
             if (e == hipSuccess)
-                e = Ops<R>::adj_b2(stream, am(), s, p, state(a), arr3<R>(fit.P), arr3<R>(fit.lH1), arr3<R>(fit.lPd),
-                                   arr3<R>(fit.lT), arr3<R>(fit.H0), arr3<R>(fit.sumS), fit.nhat.as<R>(),
-                                   arr3<R>(fit.lH0), arr3<R>(fit.lSp), arr3<R>(fit.dh), fit.acc.as<double>());
-            if (e == hipSuccess) e = Ops<R>::adj_b3(stream, am(), s, p, arr3<R>(fit.lH0), arr3<R>(fit.lSp), lam, (R)0);
-            if (e != hipSuccess) return e;
+                e = Ops<R>::adj_b(stream, am(), s, pp, S, P(t), arr3<R>(fit.lH1), arr3<R>(fit.lPd), arr3<R>(fit.lT),
+                                  arr3<R>(fit.H0), arr3<R>(fit.sumS), fit.nhat.as<R>(), arr3<R>(fit.lH0),
+                                  arr3<R>(fit.lSp), arr3<R>(fit.dh), fit.acc.as<double>());
         }
-        return hipSuccess;
+        return e;
     };
-    // full segments replay one graph when there are at least two of them
-    const int nfull = fit.nsteps / fit.K;
-    const bool use_graph = nfull >= 2;
-    if (use_graph) {
-        fit.drop_graph();
-        VMX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        const hipError_t e = segment(fit.K, fit.inj_seg.as<R>());
-        hipGraph_t g = nullptr;
-        const hipError_t ec = hipStreamEndCapture(stream, &g);
-        if (e != hipSuccess || ec != hipSuccess) {
-            if (g) (void)hipGraphDestroy(g);
-            return fail(VMX_ERR_HIP, "adjoint segment capture failed: %s",
-                        hipGetErrorString(e != hipSuccess ? e : ec));
-        }
-        fit.graph = g;
-        VMX_HIP(hipGraphInstantiate(&fit.graph_exec, fit.graph, nullptr, nullptr, 0));
-    }
+    // the buffers are never freed while the context lives except to grow, which changes an address here
+    const std::vector<const void*> key = {seg, fit.P.p, hh.x, pp, fit.lH0.p, fit.lSp.p, fit.lH1.p, fit.lPd.p, fit.lT.p,
+                                          fit.H0.p, fit.sumS.p, fit.nhat.p, fit.dh.p, fit.acc.p, fit.inj_seg.p,
+                                          (const void*)(intptr_t)(4 * G + (fit.resident ? 2 : 0) + (fit.keepP ? 1 : 0))};
+    const bool replay = fit.nsteps / G >= 2;
     for (int c = nseg - 1; c >= 0; --c) {
-        const int start = c * fit.K, end = std::min(start + fit.K, fit.nsteps);
-        VMX_HIP(hipMemcpyAsync(seg, ck + (size_t)c * N3, N3 * sizeof(R), hipMemcpyDeviceToDevice, stream));
-        if (use_graph && end - start == fit.K) {
-            VMX_HIP(hipMemcpyAsync(fit.inj_seg.p, fit.inj.as<R>() + start, (size_t)fit.K * sizeof(R),
+        const int start = c * G, len = std::min(G, fit.nsteps - start);
+        if (!fit.resident || c == 0)
+            VMX_HIP(hipMemcpyAsync(seg, ck + (size_t)c * N3, sb, hipMemcpyDeviceToDevice, stream));
+        if (fit.resident) {
+            const R* tr = fit.traj.as<R>() + (size_t)c * 2 * G * N3;
+            if (c) VMX_HIP(hipMemcpyAsync(seg, tr - (size_t)(G + 1) * N3, sb, hipMemcpyDeviceToDevice, stream));
+            VMX_HIP(hipMemcpyAsync(seg + N3, tr, (size_t)(len == G ? 2 * G : G + len) * sb, hipMemcpyDeviceToDevice, stream));
+        }
+        if (replay && len == G) {
+            VMX_HIP(hipMemcpyAsync(fit.inj_seg.p, fit.inj.as<R>() + start, (size_t)G * sizeof(R),
                                    hipMemcpyDeviceToDevice, stream));
-            VMX_HIP(hipGraphLaunch(fit.graph_exec, stream));
+            VMX_TRY(fit_replay(fit.bwd, key, [&] { return segment(G, fit.inj_seg.as<R>()); }));
         } else {
-            VMX_HIP(segment(end - start, fit.inj.as<R>() + start));
+            VMX_HIP(segment(len, fit.inj.as<R>() + start));
         }
     }
-    VMX_HIP(hipStreamSynchronize(stream));
-    fit.drop_graph();   // its replays have finished
-    std::vector<double> part((size_t)4 * nwg);
-    VMX_HIP(hipMemcpy(part.data(), fit.acc.p, part.size() * sizeof(double), hipMemcpyDeviceToHost));
+    std::vector<double> part((size_t)4 * nwave);
+    const HostPipe::Seg as{part.data(), fit.acc.p, part.size() * sizeof(double)};
+    VMX_TRY(pipe.move(&as, 1, true, stream));
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int w = 0; w < nwg; ++w)
+    for (int w = 0; w < nwave; ++w)
         for (int k = 0; k < 4; ++k) acc[k] += part[4 * (size_t)w + k];
     // a = -gamma/(1+alpha^2), b = alpha a
     const double al = fit.alpha, g = fit.gamma_rel;

@@ -84,20 +84,19 @@ struct Ops {
                                      const int* gather, const int* rep_blk, int nrep, double* partial, double* M);
     // M[r] += the sum of the cmc_pairs partials dM[range[r] .. range[r+1]], in a fixed order
     static hipError_t moment_add(hipStream_t st, const int* range, int nrep, const double* dM, double* M);
-    // deterministic fitting step and its adjoint (isotropic uniform exchange); grids of 256
-    static hipError_t fit_predictor(hipStream_t st, int am, const SysDev<R>& s, const FitPrm<R>& p, Spin3<R> h,
+    // deterministic fitting step and its adjoint (isotropic uniform exchange); grids of 256; p: device
+    static hipError_t fit_predictor(hipStream_t st, int am, const SysDev<R>& s, const FitPrm<R>* p, Spin3<R> h,
                                     Spin3<R> S, Spin3<R> P);
-    static hipError_t fit_corrector(hipStream_t st, int am, const SysDev<R>& s, const FitPrm<R>& p, Spin3<R> h,
+    static hipError_t fit_corrector(hipStream_t st, int am, const SysDev<R>& s, const FitPrm<R>* p, Spin3<R> h,
                                     Spin3<R> S, Spin3<R> P, Spin3<R> O);
-    static hipError_t adj_b1(hipStream_t st, int am, const SysDev<R>& s, const FitPrm<R>& p, Spin3<R> h,
-                             Spin3<R> S, Spin3<R> P, Spin3<R> lam, Spin3<R> lH1, Spin3<R> lPd, Spin3<R> lT,
-                             Spin3<R> H0, Spin3<R> sumS, R* nhat, double* acc);
-    static hipError_t adj_b2(hipStream_t st, int am, const SysDev<R>& s, const FitPrm<R>& p, Spin3<R> S,
-                             Spin3<R> P, Spin3<R> lH1, Spin3<R> lPd, Spin3<R> lT, Spin3<R> H0, Spin3<R> sumS,
-                             const R* nhat, Spin3<R> lH0, Spin3<R> lSp, Spin3<R> dh, double* acc);
-    static hipError_t adj_b3(hipStream_t st, int am, const SysDev<R>& s, const FitPrm<R>& p, Spin3<R> lH0,
-                             Spin3<R> lSp, Spin3<R> lam, R inj);
-    static hipError_t fit_mz(hipStream_t st, int n, Spin3<R> S, double* out4);
+    static hipError_t adj_a(hipStream_t st, int am, const SysDev<R>& s, const FitPrm<R>* p, Spin3<R> h, Spin3<R> S,
+                            Spin3<R> P, Spin3<R> lH0, Spin3<R> lSp, const R* inj, Spin3<R> lH1, Spin3<R> lPd,
+                            Spin3<R> lT, Spin3<R> H0, Spin3<R> sumS, R* nhat, double* acc);
+    static hipError_t adj_b(hipStream_t st, int am, const SysDev<R>& s, const FitPrm<R>* p, Spin3<R> S, Spin3<R> P,
+                            Spin3<R> lH1, Spin3<R> lPd, Spin3<R> lT, Spin3<R> H0, Spin3<R> sumS, const R* nhat,
+                            Spin3<R> lH0, Spin3<R> lSp, Spin3<R> dh, double* acc);
+    // sums of S_z of `records` states, the first's z array at z, stride reals apart: out[record][part]
+    static hipError_t fit_mz(hipStream_t st, int n, const R* z, size_t stride, int records, int parts, double* out);
     // Philox normals of `step` as double [3][n]
     static hipError_t thermal_noise(const Launch& L, const SysDev<R>& s, uint64_t step, double* out);
     // three-component arrays between the device's atom order and the caller's ([3][n] doubles), over

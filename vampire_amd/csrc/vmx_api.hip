@@ -558,6 +558,7 @@ struct vmx_ctx {
     int n = 0, nmat = 0, nrep = 1;
     int64_t nnz = 0;
     int et = 0, jm = 0, K = 1;
+    int njt = 0;                                     // entries of the exchange table
     int tp = TP_CSR, zmax = 0, npat = 0, wsel = 0;   // zmax: row stride W for ELL / stencil
     int full_rows = 0;                               // ELL / stencil: every row has W neighbours
     // internal atom order: with lattice period q > 1 atoms are stored basis-major inside each
@@ -815,6 +816,9 @@ struct vmx_ctx {
         // the whole staging area stays within 64 KiB
         s.pat_lds = (tp == TP_PAT && (size_t)npat * zmax * sizeof(int) <= 16384 &&
                      fused_lds_bytes<R>(nmat, npat, zmax, 1) <= 65536) ? 1 : 0;
+        // and an exchange table of up to 8 KiB, while the whole stays within 64 KiB
+        s.njt_lds = (jm == JM_IDX16 && (size_t)njt * K * sizeof(R) <= 8192 &&
+                     fused_lds_bytes<R>(nmat, npat, zmax, s.pat_lds, (size_t)njt * K) <= 65536) ? njt : 0;
         s.am = am();
         s.q = q;
         s.rep_m = rep_m.as<int>();
@@ -2397,6 +2401,7 @@ int vmx_create(const vmx_system* sys, const vmx_options* opt, vmx_ctx** out) {
     if (c->tp == TP_PAT && c->jm == JM_IDX16) c->idx16_ = idx16;
     c->rowh_.swap(rowh);
     c->colh_.swap(colh);
+    c->njt = (int)std::min<size_t>(table.size() / K, 1u << 30);
     VMX_TRY(c->jtab.alloc(table.size() * rs));
     if (c->precision == VMX_FP64) {
         VMX_HIP(hipMemcpy(c->jtab.p, table.data(), table.size() * sizeof(double), hipMemcpyHostToDevice));

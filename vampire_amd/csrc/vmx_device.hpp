@@ -81,6 +81,8 @@ struct SysDev {
     int full_rows;                           // ELL / stencil: every row has exactly W neighbours
     int npat;                                // stencils in the table
     int pat_lds;                             // 1: fused kernels stage the stencil offsets in LDS
+    int njt_lds;                             // entries of the exchange table that the step kernels stage in LDS
+                                             // (16-bit J ids; 0: the table stays in memory)
     int am;                                  // access mode the arrays below were built for
     int q;                                   // basis-major atom order with period q (1: caller's order)
     const int* __restrict__ rep_m;           // [nrep] replica size / q
@@ -342,20 +344,26 @@ __device__ __forceinline__ void row_load(const SpinRsrc<R>& rs, const RowIdx<AM>
     for (int k = 0; k < Access<AM>::W; ++k) rs.load(r.j[k], v.x[k], v.y[k], v.z[k]);
 }
 
+// jt: the exchange table, in memory or staged in LDS.
 template <typename R, int ET, int AM, typename F>
 __device__ __forceinline__ void row_sum(const SysDev<R>& s, const RowIdx<AM>& r, const RowSpins<R, AM>& v,
-                                        const R* ju, F&& f) {
+                                        const R* ju, const R* jt, F&& f) {
     constexpr int K = (ET == ET_ISO) ? 1 : (ET == ET_VEC ? 3 : 9);
     constexpr int JM = Access<AM>::JM, W = Access<AM>::W;
     if (s.full_rows) {
 #pragma unroll
-        for (int k = 0; k < W; ++k) f(v.x[k], v.y[k], v.z[k], JM == JM_UNIFORM ? ju : s.jtab + (size_t)K * r.jd[k]);
+        for (int k = 0; k < W; ++k) f(v.x[k], v.y[k], v.z[k], JM == JM_UNIFORM ? ju : jt + (size_t)K * r.jd[k]);
     } else {
 #pragma unroll
         for (int k = 0; k < W; ++k) {
-            if (k < r.deg) f(v.x[k], v.y[k], v.z[k], JM == JM_UNIFORM ? ju : s.jtab + (size_t)K * r.jd[k]);
+            if (k < r.deg) f(v.x[k], v.y[k], v.z[k], JM == JM_UNIFORM ? ju : jt + (size_t)K * r.jd[k]);
         }
     }
+}
+template <typename R, int ET, int AM, typename F>
+__device__ __forceinline__ void row_sum(const SysDev<R>& s, const RowIdx<AM>& r, const RowSpins<R, AM>& v,
+                                        const R* ju, F&& f) {
+    row_sum<R, ET, AM>(s, r, v, ju, s.jtab, f);
 }
 
 // Calls f(Sx, Sy, Sz, J) for every neighbour of atom i in row order, with its spin and a pointer
@@ -464,15 +472,15 @@ __device__ __forceinline__ void spin_field(const SysDev<R>& s, const R* __restri
 // FP64 kernels need fewer registers and keep more wavefronts per SIMD in flight.
 template <typename R, int ET, int AM, int Parts>
 __device__ __forceinline__ void row_gather_field(const SysDev<R>& s, const SpinRsrc<R>& rs, const RowIdx<AM>& r,
-                                                 const R* ju, const MatConst<R>& mc, R sx, R sy, R sz, R& fx,
-                                                 R& fy, R& fz);
+                                                 const R* ju, const R* jt, const MatConst<R>& mc, R sx, R sy, R sz,
+                                                 R& fx, R& fy, R& fz);
 
 template <typename R, int ET, int AM>
 __device__ __forceinline__ void row_field(const SysDev<R>& s, const RowIdx<AM>& r, const RowSpins<R, AM>& v,
-                                          const R* ju, const MatConst<R>& mc, R sx, R sy, R sz, R& fx, R& fy,
-                                          R& fz) {
+                                          const R* ju, const R* jt, const MatConst<R>& mc, R sx, R sy, R sz, R& fx,
+                                          R& fy, R& fz) {
     R hx = R(0), hy = R(0), hz = R(0);
-    row_sum<R, ET, AM>(s, r, v, ju, [&](const R Sx, const R Sy, const R Sz, const R* J) {
+    row_sum<R, ET, AM>(s, r, v, ju, jt, [&](const R Sx, const R Sy, const R Sz, const R* J) {
         exchange_term<R, ET>(J, Sx, Sy, Sz, hx, hy, hz);
     });
     add_anisotropy(s.ani, mc, sx, sy, sz, hx, hy, hz, fx, fy, fz);
@@ -480,8 +488,8 @@ __device__ __forceinline__ void row_field(const SysDev<R>& s, const RowIdx<AM>& 
 
 template <typename R, int ET, int AM, int Parts>
 __device__ __forceinline__ void row_gather_field(const SysDev<R>& s, const SpinRsrc<R>& rs, const RowIdx<AM>& r,
-                                                 const R* ju, const MatConst<R>& mc, R sx, R sy, R sz, R& fx,
-                                                 R& fy, R& fz) {
+                                                 const R* ju, const R* jt, const MatConst<R>& mc, R sx, R sy, R sz,
+                                                 R& fx, R& fy, R& fz) {
     constexpr int W = Access<AM>::W;
     if constexpr (Parts > 1 && sizeof(R) == 8 && W >= 8) {
         constexpr int K = (ET == ET_ISO) ? 1 : (ET == ET_VEC ? 3 : 9);
@@ -497,8 +505,8 @@ __device__ __forceinline__ void row_gather_field(const SysDev<R>& s, const SpinR
             for (int k = 0; k < H; ++k) {
                 const int slot = part * H + k;
                 if (slot < W && (s.full_rows || slot < r.deg))
-                    exchange_term<R, ET>(JM == JM_UNIFORM ? ju : s.jtab + (size_t)K * r.jd[slot], vx[k], vy[k],
-                                         vz[k], hx, hy, hz);
+                    exchange_term<R, ET>(JM == JM_UNIFORM ? ju : jt + (size_t)K * r.jd[slot], vx[k], vy[k], vz[k], hx,
+                                         hy, hz);
             }
             if (part + 1 < Parts) __builtin_amdgcn_sched_barrier(0);   // the next part's loads stay here
         }
@@ -506,7 +514,7 @@ __device__ __forceinline__ void row_gather_field(const SysDev<R>& s, const SpinR
     } else {
         RowSpins<R, AM> rv;
         row_load(rs, r, rv);
-        row_field<R, ET, AM>(s, r, rv, ju, mc, sx, sy, sz, fx, fy, fz);
+        row_field<R, ET, AM>(s, r, rv, ju, jt, mc, sx, sy, sz, fx, fy, fz);
     }
 }
 
@@ -683,6 +691,13 @@ struct FusedLds {
     static __device__ __forceinline__ int pat_off(const SysDev<R>& s) {
         return ((s.nmat * (kMatInts + kCondInts)) + 3) & ~3;   // 16-byte aligned for int4 reads
     }
+    // exchange table (after the stencil offsets): ints from the start, 16-byte aligned
+    static __device__ __forceinline__ int jt_off(const SysDev<R>& s) {
+        return pat_off(s) + ((s.pat_lds ? s.npat * s.zmax + 3 : 0) & ~3);
+    }
+    static __device__ __forceinline__ const R* jt(const SysDev<R>& s) {
+        return reinterpret_cast<const R*>(vmx_lds + jt_off(s));
+    }
     static __device__ __forceinline__ const MatConst<R>* mat() { return reinterpret_cast<const MatConst<R>*>(vmx_lds); }
     static __device__ __forceinline__ const Cond<R>* cond(const SysDev<R>& s) {
         return reinterpret_cast<const Cond<R>*>(vmx_lds + cond_off(s));
@@ -690,10 +705,10 @@ struct FusedLds {
 };
 // bytes of dynamic LDS the fused kernels need (host and device agree on this layout)
 template <typename R>
-__host__ __device__ inline size_t fused_lds_bytes(int nmat, int npat, int zmax, int pat_lds) {
+__host__ __device__ inline size_t fused_lds_bytes(int nmat, int npat, int zmax, int pat_lds, size_t jt_reals = 0) {
     const size_t rec = (size_t)nmat * ((sizeof(MatConst<R>) + sizeof(Cond<R>)) / sizeof(int));
-    const size_t pat = pat_lds ? (size_t)npat * (size_t)zmax : 0;
-    return (((rec + 3) & ~(size_t)3) + pat) * sizeof(int);
+    const size_t pat = pat_lds ? ((size_t)npat * (size_t)zmax + 3) & ~(size_t)3 : 0;
+    return (((rec + 3) & ~(size_t)3) + pat) * sizeof(int) + jt_reals * sizeof(R);
 }
 // Thermal unit normals of a thread's atoms, formed before the LDS tables are staged: they depend
 // only on the atom and the step, so their arithmetic runs while the own-data loads are in flight.
@@ -709,18 +724,23 @@ __device__ __forceinline__ void early_normals(const SysDev<R>& s, int rep, const
     }
 }
 
-template <typename R, int AM>
+// KJ: reals of an exchange table entry when the table is staged too (the step kernels), else 0.
+template <typename R, int AM, int KJ = 0>
 __device__ __forceinline__ void stage_fused(const SysDev<R>& s, int rep) {
     using L = FusedLds<R>;
     const int* __restrict__ mat = reinterpret_cast<const int*>(s.mat);
     const int* __restrict__ cond = reinterpret_cast<const int*>(s.cond + rep * s.nmat);
     const int nm = s.nmat * L::kMatInts, nc = s.nmat * L::kCondInts;
     const int np = (Access<AM>::TP == TP_PAT && s.pat_lds) ? s.npat * Access<AM>::W : 0;
-    const int rec = nm + nc, base = L::pat_off(s), total = rec + np;
+    const int nj = Access<AM>::JM == JM_IDX16 ? s.njt_lds * KJ * (int)(sizeof(R) / sizeof(int)) : 0;
+    const int* __restrict__ jt = reinterpret_cast<const int*>(s.jtab);
+    const int rec = nm + nc, base = L::pat_off(s), jbase = L::jt_off(s), offs = rec + np, total = offs + nj;
     // one pass over the three tables with two loads in flight per thread: every wait for these
     // loads also waits for the own-data loads issued before, so fewer rounds mean fewer waits
-    auto src = [&](int k) { return k < nm ? mat[k] : (k < rec ? cond[k - nm] : s.pat_off[k - rec]); };
-    auto dst = [&](int k) { return k < rec ? k : base + (k - rec); };
+    auto src = [&](int k) {
+        return k < nm ? mat[k] : (k < rec ? cond[k - nm] : (k < offs ? s.pat_off[k - rec] : jt[k - offs]));
+    };
+    auto dst = [&](int k) { return k < rec ? k : (k < offs ? base + (k - rec) : jbase + (k - offs)); };
     const int bd = (int)blockDim.x;
     for (int k0 = (int)threadIdx.x; k0 < total; k0 += 2 * bd) {
         const int k1 = k0 + bd;
@@ -737,6 +757,19 @@ __device__ __forceinline__ void fused_row_index(const SysDev<R>& s, int i, int h
         row_index(s, i, head, vmx_lds + FusedLds<R>::pat_off(s), r);
     else
         row_index(s, i, head, s.pat_off, r);
+}
+
+// The spin field of a staged row in the step kernels.  A table of up to 8 KiB of exchange entries is read
+// from LDS: an edge's entry is 1, 3 or 9 reals, and through the texture path the 9 of a tensor cost three
+// times the neighbour's spin (diluted film of 472,014 atoms, 28 tensors, FP32: predictor 16.0 -> 13.4 us,
+// corrector 15.5 -> 12.8; the step with its temperature set before it 32.6 -> 26.3).
+template <typename R, int ET, int AM, int Parts>
+__device__ __forceinline__ void step_field(const SysDev<R>& s, const SpinRsrc<R>& rs, const RowIdx<AM>& r, const R* ju,
+                                           const MatConst<R>& mc, R sx, R sy, R sz, R& fx, R& fy, R& fz) {
+    if (Access<AM>::JM == JM_IDX16 && s.njt_lds)
+        row_gather_field<R, ET, AM, Parts>(s, rs, r, ju, FusedLds<R>::jt(s), mc, sx, sy, sz, fx, fy, fz);
+    else
+        row_gather_field<R, ET, AM, Parts>(s, rs, r, ju, s.jtab, mc, sx, sy, sz, fx, fy, fz);
 }
 
 // Predictor: S' = |S + dt f(S, H_spin(S) + H_ext)|, written to P.  With D.x set the FP64 Euler
@@ -771,7 +804,7 @@ k_fused_predictor(SysDev<R> s, Spin3<R> S, Spin3<R> P, Spin3<R> D, Spin3<R> E, c
     const uint64_t step = *s.step_base + step_off;
     R gx[U], gy[U], gz[U];
     early_normals<R, U>(s, rep, b, idx, step, noise, true, gx, gy, gz);
-    stage_fused<R, AM>(s, rep);
+    stage_fused<R, AM, UniformJ<R, ET>::K>(s, rep);
     if (!ok[0]) return;
     const UniformJ<R, ET> ju(s, Access<AM>::JM);
 #pragma unroll
@@ -782,7 +815,7 @@ k_fused_predictor(SysDev<R> s, Spin3<R> S, Spin3<R> P, Spin3<R> D, Spin3<R> E, c
         if constexpr (kStaged) {
             RowIdx<AM> ri;
             fused_row_index(s, i, head[u], ri);
-            row_gather_field<R, ET, AM, 2>(s, rs, ri, ju.v, mc, sx[u], sy[u], sz[u], fx, fy, fz);
+            step_field<R, ET, AM, 2>(s, rs, ri, ju.v, mc, sx[u], sy[u], sz[u], fx, fy, fz);
         } else {
             spin_field<R, ET, AM>(s, S.x, S.y, S.z, i, m[u], sx[u], sy[u], sz[u], fx, fy, fz);
         }
@@ -845,7 +878,7 @@ k_fused_corrector(SysDev<R> s, Spin3Alias<R> S, Spin3<R> P, Spin3Alias<R> O, Spi
     const uint64_t step = *s.step_base + step_off;
     R gx[U], gy[U], gz[U];                        // unless H_ext is read back
     early_normals<R, U>(s, rep, b, idx, step, noise, E.x == nullptr, gx, gy, gz);
-    stage_fused<R, AM>(s, rep);      // own data above is in flight meanwhile
+    stage_fused<R, AM, UniformJ<R, ET>::K>(s, rep);      // own data above is in flight meanwhile
     if (!ok[0]) return;
     const UniformJ<R, ET> ju(s, Access<AM>::JM);
     constexpr int parts = CorrectorParts<R>::value;
@@ -857,7 +890,7 @@ k_fused_corrector(SysDev<R> s, Spin3Alias<R> S, Spin3<R> P, Spin3Alias<R> O, Spi
         R fx, fy, fz;
         if constexpr (kStaged) {
             fused_row_index(s, i, head[u], ri);
-            row_gather_field<R, ET, AM, parts>(s, rp, ri, ju.v, mc, px[u], py[u], pz[u], fx, fy, fz);
+            step_field<R, ET, AM, parts>(s, rp, ri, ju.v, mc, px[u], py[u], pz[u], fx, fy, fz);
         } else {
             spin_field<R, ET, AM>(s, P.x, P.y, P.z, i, m[u], px[u], py[u], pz[u], fx, fy, fz);
         }
@@ -876,7 +909,7 @@ k_fused_corrector(SysDev<R> s, Spin3Alias<R> S, Spin3<R> P, Spin3Alias<R> O, Spi
                 R gx, gy, gz;
                 if constexpr (kStaged) {
                     const SpinRsrc<R> rs(s, S.x, S.y, S.z);
-                    row_gather_field<R, ET, AM, parts>(s, rs, ri, ju.v, mc, ax[u], ay[u], az[u], gx, gy, gz);
+                    step_field<R, ET, AM, parts>(s, rs, ri, ju.v, mc, ax[u], ay[u], az[u], gx, gy, gz);
                 } else {
                     spin_field<R, ET, AM>(s, S.x, S.y, S.z, i, m[u], ax[u], ay[u], az[u], gx, gy, gz);
                 }
@@ -946,7 +979,7 @@ k_mid_predictor(SysDev<R> s, Spin3<R> S, Spin3<R> P, Spin3<R> E, const double* _
     const uint64_t step = *s.step_base + step_off;
     R gx[U], gy[U], gz[U];
     early_normals<R, U>(s, rep, b, idx, step, noise, true, gx, gy, gz);
-    stage_fused<R, AM>(s, rep);
+    stage_fused<R, AM, UniformJ<R, ET>::K>(s, rep);
     if (!ok[0]) return;
     const UniformJ<R, ET> ju(s, Access<AM>::JM);
 #pragma unroll
@@ -957,7 +990,7 @@ k_mid_predictor(SysDev<R> s, Spin3<R> S, Spin3<R> P, Spin3<R> E, const double* _
         if constexpr (kStaged) {
             RowIdx<AM> ri;
             fused_row_index(s, i, head[u], ri);
-            row_gather_field<R, ET, AM, 2>(s, rs, ri, ju.v, mc, sx[u], sy[u], sz[u], fx, fy, fz);
+            step_field<R, ET, AM, 2>(s, rs, ri, ju.v, mc, sx[u], sy[u], sz[u], fx, fy, fz);
         } else {
             spin_field<R, ET, AM>(s, S.x, S.y, S.z, i, m[u], sx[u], sy[u], sz[u], fx, fy, fz);
         }
@@ -1007,7 +1040,7 @@ k_mid_corrector(SysDev<R> s, Spin3Alias<R> S, Spin3<R> P, Spin3Alias<R> O, Spin3
     const uint64_t step = *s.step_base + step_off;
     R gx[U], gy[U], gz[U];                        // unless H_ext is read back
     early_normals<R, U>(s, rep, b, idx, step, noise, E.x == nullptr, gx, gy, gz);
-    stage_fused<R, AM>(s, rep);
+    stage_fused<R, AM, UniformJ<R, ET>::K>(s, rep);
     if (!ok[0]) return;
     const UniformJ<R, ET> ju(s, Access<AM>::JM);
 #pragma unroll
@@ -1018,7 +1051,7 @@ k_mid_corrector(SysDev<R> s, Spin3Alias<R> S, Spin3<R> P, Spin3Alias<R> O, Spin3
         if constexpr (kStaged) {
             RowIdx<AM> ri;
             fused_row_index(s, i, head[u], ri);
-            row_gather_field<R, ET, AM, CorrectorParts<R>::value>(s, rp, ri, ju.v, mc, px[u], py[u], pz[u], fx, fy,
+            step_field<R, ET, AM, CorrectorParts<R>::value>(s, rp, ri, ju.v, mc, px[u], py[u], pz[u], fx, fy,
                                                                   fz);
         } else {
             spin_field<R, ET, AM>(s, P.x, P.y, P.z, i, m[u], px[u], py[u], pz[u], fx, fy, fz);
@@ -1152,7 +1185,7 @@ k_tile_step(SysDev<R> s, TileDev t, Spin3<R> S, Spin3<R> O, const double* __rest
     const Cond<R>& c = s.cond[h.z * s.nmat + m];
     const UniformJ<R, ET> ju(s, JM);
     R fx, fy, fz, ex, ey, ez, px, py, pz, d0 = R(0), d1 = R(0), d2 = R(0);
-    row_field<R, ET, AM>(s, r, v, ju.v, mc, sx, sy, sz, fx, fy, fz);
+    row_field<R, ET, AM>(s, r, v, ju.v, s.jtab, mc, sx, sy, sz, fx, fy, fz);
     ext_from_normals(s, c, i, gx, gy, gz, ex, ey, ez);
     if constexpr (STEP == STEP_HEUN) {
         heun_predict(s, mc, sx, sy, sz, fx + ex, fy + ey, fz + ez, d0, d1, d2, px, py, pz);
@@ -1166,7 +1199,7 @@ k_tile_step(SysDev<R> s, TileDev t, Spin3<R> S, Spin3<R> O, const double* __rest
     if (tid >= h.x) return;
 #pragma unroll
     for (int k = 0; k < W; ++k) { v.x[k] = lx[q[k]]; v.y[k] = ly[q[k]]; v.z[k] = lz[q[k]]; }
-    row_field<R, ET, AM>(s, r, v, ju.v, mc, px, py, pz, fx, fy, fz);
+    row_field<R, ET, AM>(s, r, v, ju.v, s.jtab, mc, px, py, pz, fx, fy, fz);
     R o0, o1, o2;
     if constexpr (STEP == STEP_HEUN)
         heun_correct(s, mc, sx, sy, sz, px, py, pz, fx + ex, fy + ey, fz + ez, d0, d1, d2, o0, o1, o2);

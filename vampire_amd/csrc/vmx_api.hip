@@ -781,6 +781,11 @@ struct vmx_ctx {
         if (device >= 0) VMX_HIP(hipSetDevice(device));
         return VMX_OK;
     }
+    // for calls whose kernels read the condition table
+    int use_device_and_conditions() {
+        VMX_TRY(use_device());
+        return flush_conditions();
+    }
 
     template <typename R>
     Spin3<R> spins(int idx) const {
@@ -969,6 +974,12 @@ struct vmx_ctx {
         }
         VMX_TRY(cond.alloc(cv.size() * sizeof(Cond<R>)));
         const size_t b = cv.size() * sizeof(Cond<R>);
+        cond_next.n = 0;
+        if (b <= sizeof cond_next.w && b % sizeof(uint32_t) == 0) {
+            std::memcpy(cond_next.w, cv.data(), b);          // carried by the next launch that needs them
+            cond_next.n = (int)(b / sizeof(uint32_t));
+            return VMX_OK;
+        }
         if (b % 4 == 0 && b <= sizeof(ArgWords)) {
             ArgWords v;
             std::memcpy(v.w, cv.data(), b);
@@ -979,6 +990,25 @@ struct vmx_ctx {
         }
         if (ring.bytes < b) return fail(VMX_ERR_STATE, "condition table exceeds staging");
         return ring.copy(cond.p, cv.data(), b, stream);
+    }
+    // Conditions the device table does not hold yet (n = 0: none).
+    CondArg cond_next{};
+    // hands them to a launch that writes them to the table
+    CondArg take_conditions() {
+        const CondArg a = cond_next;
+        cond_next.n = 0;
+        return a;
+    }
+    // writes them now, for launches that read the table
+    int flush_conditions() {
+        if (!cond_next.n) return VMX_OK;
+        ArgWords v;
+        const int words = cond_next.n;
+        std::memcpy(v.w, cond_next.w, (size_t)words * sizeof(uint32_t));
+        hipLaunchKernelGGL(k_put_words, dim3(1), dim3(kArgWords), 0, stream, cond.as<uint32_t>(), v, words);
+        VMX_HIP(hipGetLastError());
+        cond_next.n = 0;
+        return VMX_OK;
     }
     int upload_conditions_any() {
         return precision == VMX_FP64 ? upload_conditions<double>() : upload_conditions<float>();
@@ -1062,6 +1092,7 @@ int vmx_ctx::heun_steps(int nsteps, const double* noise, double* kernel_ms) {
     const SysDev<R> s = sys<R>(), sf = sys_fused<R>();
     const Launch L = launch(), Lf = launch_fused();
     VMX_TRY(build_tiles(nsteps));
+    if (kernel == VMX_KERNEL_PLAIN) VMX_TRY(flush_conditions());
     uint32_t off0 = 0;
     VMX_TRY(eager_step_off(nsteps, off0));
     const double* nd = nullptr;
@@ -1100,12 +1131,12 @@ int vmx_ctx::heun_steps(int nsteps, const double* noise, double* kernel_ms) {
         int nk = 0;
         if (kernel == VMX_KERNEL_FUSED && ntiles && !kernel_ms) {
             VMX_HIP(Ops<R>::tile_step(stream, et, jm, wsel, STEP_HEUN, s, tile, ntiles, spins<R>(s_idx), spins<R>(o_idx),
-                                      nd, off0 + (uint32_t)k));
+                                      nd, off0 + (uint32_t)k, take_conditions()));
             std::swap(s_idx, o_idx);
         } else if (kernel == VMX_KERNEL_FUSED) {
             VMX_HIP(mark(0));
             VMX_HIP(Ops<R>::fused_predictor(Lf, et, am(), sf, spins<R>(s_idx), spins<R>(p_idx), euler<R>(),
-                                            field<R>(), nd, off0 + (uint32_t)k));
+                                            field<R>(), nd, off0 + (uint32_t)k, take_conditions()));
             VMX_HIP(mark(1));
             const int out = corrector_in_place() ? s_idx : o_idx;
             VMX_HIP(Ops<R>::fused_corrector(L, et, am(), s, spins<R>(s_idx), spins<R>(p_idx), spins<R>(out),
@@ -1156,6 +1187,7 @@ int vmx_ctx::midpoint_steps(int nsteps, const double* noise) {
     const SysDev<R> s = sys<R>(), sf = sys_fused<R>();
     const Launch L = launch(), Lf = launch_fused();
     VMX_TRY(build_tiles(nsteps));
+    if (kernel == VMX_KERNEL_PLAIN) VMX_TRY(flush_conditions());
     uint32_t off0 = 0;
     VMX_TRY(eager_step_off(nsteps, off0));
     const double* nd = nullptr;
@@ -1177,12 +1209,12 @@ int vmx_ctx::midpoint_steps(int nsteps, const double* noise) {
         }
         if (ntiles) {
             VMX_HIP(Ops<R>::tile_step(stream, et, jm, wsel, STEP_MIDPOINT, s, tile, ntiles, spins<R>(s_idx),
-                                      spins<R>(o_idx), nd, off0 + (uint32_t)k));
+                                      spins<R>(o_idx), nd, off0 + (uint32_t)k, take_conditions()));
             std::swap(s_idx, o_idx);
         } else {
             const int p_idx = 3 - s_idx - o_idx;
             VMX_HIP(Ops<R>::mid_predictor(Lf, et, am(), sf, spins<R>(s_idx), spins<R>(p_idx), field<R>(), nd,
-                                          off0 + (uint32_t)k));
+                                          off0 + (uint32_t)k, take_conditions()));
             // the midpoint corrector gathers only the midpoint: S_next overwrites S
             VMX_HIP(Ops<R>::mid_corrector(L, et, am(), s, spins<R>(s_idx), spins<R>(p_idx), spins<R>(s_idx), field<R>(),
                                           nd, off0 + (uint32_t)k));
@@ -1210,10 +1242,10 @@ int vmx_ctx::capture_graph(int nsteps) {
         hipError_t e;
         if (ntiles) {
             e = Ops<R>::tile_step(stream, et, jm, wsel, STEP_HEUN, s, tile, ntiles, spins<R>(si), spins<R>(out), nullptr,
-                                  (uint32_t)k);
+                                  (uint32_t)k, CondArg{});
         } else {
             e = Ops<R>::fused_predictor(Lf, et, am(), sf, spins<R>(si), spins<R>(pi), euler<R>(), field<R>(), nullptr,
-                                        (uint32_t)k);
+                                        (uint32_t)k, CondArg{});
             if (e == hipSuccess)
                 e = Ops<R>::fused_corrector(L, et, am(), s, spins<R>(si), spins<R>(pi), spins<R>(out), euler<R>(),
                                             field<R>(), nullptr, (uint32_t)k);
@@ -2601,7 +2633,7 @@ int vmx_llg_heun_graph(vmx_ctx* c, int32_t nsteps, int32_t nrepeat) {
         return fail(VMX_ERR_STATE, "graph replay draws the normals in the step kernels; fp64_normals needs "
                                    "vmx_llg_heun");
     if (!(c->dt > 0.0)) return fail(VMX_ERR_STATE, "time step not set (vmx_set_time_step)");
-    VMX_TRY(c->use_device());
+    VMX_TRY(c->use_device_and_conditions());
     VMX_TRY(c->build_tiles((int64_t)nsteps * nrepeat));
     if (!c->graph_exec || c->graph_key != c->graph_key_of(nsteps)) {
         VMX_TRY(c->precision == VMX_FP64 ? c->capture_graph<double>(nsteps) : c->capture_graph<float>(nsteps));
@@ -2737,7 +2769,7 @@ int vmx_mc_sweep(vmx_ctx* c, int32_t nsweeps) {
     if (c->hdip_on && !c->dip.on)
         return fail(VMX_ERR_STATE, "an uploaded dipole field has no demag field for the Metropolis energy; "
                                    "use vmx_set_dipole or clear it");
-    VMX_TRY(c->use_device());
+    VMX_TRY(c->use_device_and_conditions());
     return c->precision == VMX_FP64 ? c->mc_sweeps<double>(nsweeps) : c->mc_sweeps<float>(nsweeps);
 }
 
@@ -2824,7 +2856,7 @@ int vmx_cmc_sweep(vmx_ctx* c, int32_t nsweeps) {
     if (c->dip.on || c->hdip_on)
         return fail(VMX_ERR_STATE, "constrained Monte Carlo does not refresh a dipole field; clear it first");
     if (nsweeps == 0) return VMX_OK;
-    VMX_TRY(c->use_device());
+    VMX_TRY(c->use_device_and_conditions());
     return c->precision == VMX_FP64 ? c->cmc_sweeps<double>(nsweeps) : c->cmc_sweeps<float>(nsweeps);
 }
 
@@ -2899,7 +2931,7 @@ int vmx_stats_update(vmx_ctx* c) {
     if (c->hdip_on && !c->dip.on && !c->energies.empty())
         return fail(VMX_ERR_STATE, "an uploaded dipole field has no demag field for the magnetostatic energy; "
                                    "use vmx_set_dipole or clear it");
-    VMX_TRY(c->use_device());
+    VMX_TRY(c->use_device_and_conditions());
     return c->precision == VMX_FP64 ? c->stats_update<double>() : c->stats_update<float>();
 }
 
@@ -2914,7 +2946,7 @@ int vmx_stats_update_noalloc(vmx_ctx* c) {
                                  "no-allocation update holds at most %zu (fewer mask bins, or vmx_stats_update)",
                     need, kStatsScratchBytes);
     if (!c->stats_scratch) return fail(VMX_ERR_STATE, "no statistics scratch on this context's device");
-    VMX_TRY(c->use_device());
+    VMX_TRY(c->use_device_and_conditions());
     return c->precision == VMX_FP64 ? c->stats_update<double>(c->stats_scratch)
                                     : c->stats_update<float>(c->stats_scratch);
 }
@@ -2994,7 +3026,7 @@ static int compute_fields_impl(vmx_ctx* c, const double* noise, double* h_spin, 
 
 int vmx_compute_fields(vmx_ctx* c, const double* noise, double* h_spin, double* h_ext) {
     if (!c) return fail(VMX_ERR_ARG, "null context");
-    VMX_TRY(c->use_device());
+    VMX_TRY(c->use_device_and_conditions());
     return c->precision == VMX_FP64 ? compute_fields_impl<double>(c, noise, h_spin, h_ext)
                                     : compute_fields_impl<float>(c, noise, h_spin, h_ext);
 }
@@ -3041,7 +3073,7 @@ int vmx_time_kernels(vmx_ctx* c, int32_t nsteps, double* avg_ms, int32_t* nkerne
     if (!c || !avg_ms || !nkernels) return fail(VMX_ERR_ARG, "null argument");
     if (nsteps <= 0) return fail(VMX_ERR_ARG, "nsteps must be positive");
     if (!(c->dt > 0.0)) return fail(VMX_ERR_STATE, "time step not set (vmx_set_time_step)");
-    VMX_TRY(c->use_device());
+    VMX_TRY(c->use_device_and_conditions());
     *nkernels = c->kernel == VMX_KERNEL_FUSED ? 2 : 5;
     return c->precision == VMX_FP64 ? c->heun_steps<double>(nsteps, nullptr, avg_ms)
                                     : c->heun_steps<float>(nsteps, nullptr, avg_ms);
@@ -3105,7 +3137,7 @@ int vmx_autotune(vmx_ctx* c, int32_t steps_per_trial, int32_t* chosen) {
     if (!c) return fail(VMX_ERR_ARG, "null context");
     if (steps_per_trial <= 0) return fail(VMX_ERR_ARG, "steps_per_trial must be positive");
     if (!(c->dt > 0.0)) return fail(VMX_ERR_STATE, "time step not set (vmx_set_time_step)");
-    VMX_TRY(c->use_device());
+    VMX_TRY(c->use_device_and_conditions());
     // the trials read the dipole field but must not refresh it or advance its clock
     struct PauseDipole {
         vmx_ctx* c;

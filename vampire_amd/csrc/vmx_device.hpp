@@ -71,6 +71,17 @@ struct Cond {                // per (replica, material); rewritten when conditio
     R cmc_delta;             // width of the constrained Monte Carlo angle move (cmc.cpp:320-325)
 };
 
+// Conditions that changed since the device table was last written, carried by the launch that first needs
+// them (a step's predictor, or the whole step): n words of the table, all of it, or n = 0: the device
+// table holds.  That launch reads them from its arguments and one of its workgroups writes them to the
+// table for the launches after it, so setting the temperature before every step costs no launch (a launch
+// of its own was 3 us on the device and 4.6 on the host, which a small system's step of 4-5 us waits for).
+constexpr int kCondWords = 48;
+struct CondArg {
+    int n, pad;
+    uint32_t w[kCondWords];
+};
+
 template <typename R>
 struct SysDev {
     int n;                                   // atoms over all replicas
@@ -710,6 +721,24 @@ __host__ __device__ inline size_t fused_lds_bytes(int nmat, int npat, int zmax, 
     const size_t pat = pat_lds ? ((size_t)npat * (size_t)zmax + 3) & ~(size_t)3 : 0;
     return (((rec + 3) & ~(size_t)3) + pat) * sizeof(int) + jt_reals * sizeof(R);
 }
+// the table's words from the launch's arguments to the device table (one workgroup)
+template <typename R>
+__device__ __forceinline__ void keep_conditions(const SysDev<R>& s, const CondArg& ca) {
+    uint32_t* t = reinterpret_cast<uint32_t*>(const_cast<Cond<R>*>(s.cond));
+    for (int k = (int)threadIdx.x; k < ca.n; k += (int)blockDim.x) t[k] = ca.w[k];
+}
+// record idx of the table
+template <typename R>
+__device__ __forceinline__ Cond<R> condition(const SysDev<R>& s, const CondArg& ca, int idx) {
+    if (ca.n == 0) return s.cond[idx];
+    constexpr int words = (int)(sizeof(Cond<R>) / sizeof(uint32_t)), records = kCondWords / words;
+    Cond<R> c;
+    __builtin_memcpy(&c, ca.w, sizeof c);
+#pragma unroll
+    for (int k = 1; k < records; ++k)
+        if (idx == k) __builtin_memcpy(&c, ca.w + k * words, sizeof c);
+    return c;
+}
 // Thermal unit normals of a thread's atoms, formed before the LDS tables are staged: they depend
 // only on the atom and the step, so their arithmetic runs while the own-data loads are in flight.
 template <typename R, int U>
@@ -725,8 +754,9 @@ __device__ __forceinline__ void early_normals(const SysDev<R>& s, int rep, const
 }
 
 // KJ: reals of an exchange table entry when the table is staged too (the step kernels), else 0.
+// ca: the launch's conditions, or null when the device table holds.
 template <typename R, int AM, int KJ = 0>
-__device__ __forceinline__ void stage_fused(const SysDev<R>& s, int rep) {
+__device__ __forceinline__ void stage_fused(const SysDev<R>& s, int rep, const CondArg* ca = nullptr) {
     using L = FusedLds<R>;
     const int* __restrict__ mat = reinterpret_cast<const int*>(s.mat);
     const int* __restrict__ cond = reinterpret_cast<const int*>(s.cond + rep * s.nmat);
@@ -738,6 +768,7 @@ __device__ __forceinline__ void stage_fused(const SysDev<R>& s, int rep) {
     // one pass over the three tables with two loads in flight per thread: every wait for these
     // loads also waits for the own-data loads issued before, so fewer rounds mean fewer waits
     auto src = [&](int k) {
+        if (ca && ca->n && k >= nm && k < rec) return (int)ca->w[rep * nc + k - nm];
         return k < nm ? mat[k] : (k < rec ? cond[k - nm] : (k < offs ? s.pat_off[k - rec] : jt[k - offs]));
     };
     auto dst = [&](int k) { return k < rec ? k : (k < offs ? base + (k - rec) : jbase + (k - offs)); };
@@ -782,7 +813,7 @@ __device__ __forceinline__ void step_field(const SysDev<R>& s, const SpinRsrc<R>
 template <typename R, int ET, int AM>
 __global__ void __launch_bounds__(512)
 k_fused_predictor(SysDev<R> s, Spin3<R> S, Spin3<R> P, Spin3<R> D, Spin3<R> E, const double* __restrict__ noise,
-                  uint32_t step_off) {
+                  uint32_t step_off, CondArg ca) {
     constexpr int U = FusedAtoms<R>::value;
     constexpr bool kStaged = Access<AM>::TP != TP_CSR;
     const int lb = logical_block(s.xcd_remap);
@@ -804,7 +835,8 @@ k_fused_predictor(SysDev<R> s, Spin3<R> S, Spin3<R> P, Spin3<R> D, Spin3<R> E, c
     const uint64_t step = *s.step_base + step_off;
     R gx[U], gy[U], gz[U];
     early_normals<R, U>(s, rep, b, idx, step, noise, true, gx, gy, gz);
-    stage_fused<R, AM, UniformJ<R, ET>::K>(s, rep);
+    stage_fused<R, AM, UniformJ<R, ET>::K>(s, rep, &ca);
+    if (lb == 0 && ca.n) keep_conditions(s, ca);
     if (!ok[0]) return;
     const UniformJ<R, ET> ju(s, Access<AM>::JM);
 #pragma unroll
@@ -957,7 +989,7 @@ __device__ __forceinline__ R midpoint_beta(const SysDev<R>& s, const MatConst<R>
 template <typename R, int ET, int AM>
 __global__ void __launch_bounds__(512)
 k_mid_predictor(SysDev<R> s, Spin3<R> S, Spin3<R> P, Spin3<R> E, const double* __restrict__ noise,
-                uint32_t step_off) {
+                uint32_t step_off, CondArg ca) {
     constexpr int U = FusedAtoms<R>::value;
     constexpr bool kStaged = Access<AM>::TP != TP_CSR;
     const int lb = logical_block(s.xcd_remap);
@@ -979,7 +1011,8 @@ k_mid_predictor(SysDev<R> s, Spin3<R> S, Spin3<R> P, Spin3<R> E, const double* _
     const uint64_t step = *s.step_base + step_off;
     R gx[U], gy[U], gz[U];
     early_normals<R, U>(s, rep, b, idx, step, noise, true, gx, gy, gz);
-    stage_fused<R, AM, UniformJ<R, ET>::K>(s, rep);
+    stage_fused<R, AM, UniformJ<R, ET>::K>(s, rep, &ca);
+    if (lb == 0 && ca.n) keep_conditions(s, ca);
     if (!ok[0]) return;
     const UniformJ<R, ET> ju(s, Access<AM>::JM);
 #pragma unroll
@@ -1153,7 +1186,8 @@ __global__ void __launch_bounds__(512) k_tile_fill(SysDev<R> s, TileDev t) {
 // AM: an ELL access mode (slot width and J mode), whatever layout the context's own rows have.
 template <typename R, int ET, int AM, int STEP>
 __global__ void __launch_bounds__(512)
-k_tile_step(SysDev<R> s, TileDev t, Spin3<R> S, Spin3<R> O, const double* __restrict__ noise, uint32_t step_off) {
+k_tile_step(SysDev<R> s, TileDev t, Spin3<R> S, Spin3<R> O, const double* __restrict__ noise, uint32_t step_off,
+            CondArg ca) {
     constexpr int W = Access<AM>::W, JM = Access<AM>::JM;
     R* const lx = reinterpret_cast<R*>(vmx_lds);
     R* const ly = lx + t.block;
@@ -1182,7 +1216,8 @@ k_tile_step(SysDev<R> s, TileDev t, Spin3<R> S, Spin3<R> O, const double* __rest
     R gx = R(0), gy = R(0), gz = R(0);       // while the gathers are in flight
     if (s.fld & FLD_THERMAL) unit_normals(s, h.z, i, local, step, noise, gx, gy, gz);
     const MatConst<R>& mc = s.mat[m];
-    const Cond<R>& c = s.cond[h.z * s.nmat + m];
+    const Cond<R> c = condition(s, ca, h.z * s.nmat + m);
+    if (blockIdx.x == 0 && ca.n) keep_conditions(s, ca);
     const UniformJ<R, ET> ju(s, JM);
     R fx, fy, fz, ex, ey, ez, px, py, pz, d0 = R(0), d1 = R(0), d2 = R(0);
     row_field<R, ET, AM>(s, r, v, ju.v, s.jtab, mc, sx, sy, sz, fx, fy, fz);

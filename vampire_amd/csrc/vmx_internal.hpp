@@ -23,20 +23,22 @@ struct Ops {
     // D: Euler derivative (FP64) or S + dt/2 dS (FP32) kept by the predictor for the corrector;
     // E: external field kept the same way.  All-null arrays make the corrector recompute them.
     static hipError_t fused_predictor(const Launch& L, int et, int jm, const SysDev<R>& s, Spin3<R> S,
-                                      Spin3<R> P, Spin3<R> D, Spin3<R> E, const double* noise, uint32_t step_off);
+                                      Spin3<R> P, Spin3<R> D, Spin3<R> E, const double* noise, uint32_t step_off,
+                                      const CondArg& ca);
     static hipError_t fused_corrector(const Launch& L, int et, int jm, const SysDev<R>& s, Spin3<R> S,
                                       Spin3<R> P, Spin3<R> O, Spin3<R> D, Spin3<R> E, const double* noise,
                                       uint32_t step_off);
     // LLG midpoint step: predictor writes the midpoint P from S (E: H_ext kept, or null);
     // corrector writes O from S and P
     static hipError_t mid_predictor(const Launch& L, int et, int jm, const SysDev<R>& s, Spin3<R> S, Spin3<R> P,
-                                    Spin3<R> E, const double* noise, uint32_t step_off);
+                                    Spin3<R> E, const double* noise, uint32_t step_off, const CondArg& ca);
     static hipError_t mid_corrector(const Launch& L, int et, int jm, const SysDev<R>& s, Spin3<R> S, Spin3<R> P,
                                     Spin3<R> O, Spin3<R> E, const double* noise, uint32_t step_off);
     // a whole Heun (STEP_HEUN) or midpoint (STEP_MIDPOINT) step: O from S, one workgroup per tile.
     // jm, wsel: the rows' J mode and slot width (kSlotWidths)
     static hipError_t tile_step(hipStream_t st, int et, int jm, int wsel, int kind, const SysDev<R>& s, const TileDev& t,
-                                int ntiles, Spin3<R> S, Spin3<R> O, const double* noise, uint32_t step_off);
+                                int ntiles, Spin3<R> S, Spin3<R> O, const double* noise, uint32_t step_off,
+                                const CondArg& ca);
     // fills the tiles' slot arrays from the system's rows
     static hipError_t tile_fill(hipStream_t st, int am, const SysDev<R>& s, const TileDev& t, int ntiles);
     // plain Heun step

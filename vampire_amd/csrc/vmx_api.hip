@@ -248,6 +248,7 @@ struct Statistic {
     double* cur() const { return res.as<double>(); }
     double* mean() const { return cur() + values(); }
     long long* counter() const { return reinterpret_cast<long long*>(mean() + values()); }
+    StatOut out() const { return StatOut{cur(), mean(), counter(), empty_dev.as<int>(), (int)empty.size()}; }
 };
 using MagStat = Statistic<4>;
 using EnergyStat = Statistic<5>;
@@ -259,96 +260,6 @@ template <typename R>
 __global__ void k_fill(size_t n, R* __restrict__ a, R v) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
         a[i] = v;
-}
-
-// Reduces the workgroup partials in block order, then normalises (magnetization.cpp:150-178).
-// Sum over the nblk per-workgroup partials [nblk][W] of every value k < W, handed to put(k, sum).
-// With fewer values than threads, each value's partials are split over blockDim / W threads whose
-// sub-sums are then added in thread order: the whole block works and the order is fixed, so the
-// result is the same on every run.  With many values, one thread per value.
-template <typename F>
-__device__ void reduce_partials(int nblk, const double* __restrict__ partial, int W, F&& put) {
-    __shared__ double red[256];                   // the finish kernels run one block of 256 threads
-    const int per = (int)blockDim.x / W;
-    if (per >= 2) {
-        const int k = (int)threadIdx.x % W, j = (int)threadIdx.x / W;
-        double a = 0.0;
-        if (j < per) {
-#pragma unroll 8
-            for (int b = j; b < nblk; b += per) a += partial[(size_t)b * W + k];
-        }
-        red[threadIdx.x] = a;
-        __syncthreads();
-        if ((int)threadIdx.x < W) {
-            double t = 0.0;
-            for (int q = 0; q < per; ++q) t += red[q * W + (int)threadIdx.x];
-            put((int)threadIdx.x, t);
-        }
-    } else {
-        for (int k = threadIdx.x; k < W; k += blockDim.x) {
-            double acc = 0.0;
-            for (int b = 0; b < nblk; ++b) acc += partial[(size_t)b * W + k];
-            put(k, acc);
-        }
-    }
-}
-
-__global__ void k_mag_finish(int nblk, const double* __restrict__ partial, int nbins, double* cur,
-                             double* mean, const int* __restrict__ empty, int nempty,
-                             long long* counter) {
-    const int W = 4 * nbins;
-    reduce_partials(nblk, partial, W, [&](int k, double v) { cur[k] = v; });
-    __threadfence_block();
-    __syncthreads();
-    for (int id = threadIdx.x; id < nbins - 1; id += blockDim.x) {
-        const double msat = cur[4 * id + 3];
-        const double magm = sqrt(cur[4 * id + 0] * cur[4 * id + 0] + cur[4 * id + 1] * cur[4 * id + 1] +
-                                 cur[4 * id + 2] * cur[4 * id + 2]);
-        cur[4 * id + 0] = cur[4 * id + 0] / magm;
-        cur[4 * id + 1] = cur[4 * id + 1] / magm;
-        cur[4 * id + 2] = cur[4 * id + 2] / magm;
-        cur[4 * id + 3] = magm / msat;
-    }
-    __threadfence_block();
-    __syncthreads();
-    for (int e = threadIdx.x; e < nempty; e += blockDim.x) {
-        const int id = empty[e];
-        cur[4 * id + 0] = 0.0; cur[4 * id + 1] = 0.0; cur[4 * id + 2] = 0.0; cur[4 * id + 3] = 0.0;
-    }
-    __threadfence_block();
-    __syncthreads();
-    for (int k = threadIdx.x; k < W; k += blockDim.x) mean[k] += cur[k];
-    if (threadIdx.x == 0) *counter += 1;
-}
-
-// Energies [5][nbins]: total, exchange, anisotropy, applied, magnetostatic
-// (src/statistics/energy.cpp:141-258; the magnetostatic term is zero without a device dipole field).
-__global__ void k_energy_finish(int nblk, const double* __restrict__ partial, int nbins, double* cur,
-                                double* mean, const int* __restrict__ empty, int nempty,
-                                long long* counter) {
-    const int W = 4 * nbins;
-    reduce_partials(nblk, partial, W, [&](int k, double v) {
-        const int id = k / 4, term = k % 4;     // term: exchange, anisotropy, applied, magnetostatic
-        cur[(size_t)(1 + term) * nbins + id] = v;
-    });
-    for (int id = threadIdx.x; id < nbins; id += blockDim.x) cur[id] = 0.0;
-    __threadfence_block();
-    __syncthreads();
-    const int ms = nbins - 1;
-    for (int id = threadIdx.x; id < ms; id += blockDim.x) {
-        cur[(size_t)1 * nbins + id] = 0.5 * cur[(size_t)1 * nbins + id];
-        cur[(size_t)4 * nbins + id] = 0.5 * cur[(size_t)4 * nbins + id];
-        cur[id] = cur[(size_t)1 * nbins + id] + cur[(size_t)2 * nbins + id] + cur[(size_t)3 * nbins + id] +
-                  cur[(size_t)4 * nbins + id];
-        for (int t = 0; t < 5; ++t) mean[(size_t)t * nbins + id] += cur[(size_t)t * nbins + id];
-    }
-    __threadfence_block();
-    __syncthreads();
-    for (int e = threadIdx.x; e < nempty; e += blockDim.x) {
-        const int id = empty[e];
-        for (int t = 0; t < 5; ++t) cur[(size_t)t * nbins + id] = 0.0;
-    }
-    if (threadIdx.x == 0) *counter += 1;
 }
 
 // Adaptive cone width after a sweep (src/montecarlo/mc.cpp:112-120) and running totals.  A
@@ -635,7 +546,7 @@ struct vmx_ctx {
     DevBuf euler_buf;             // 3N R
     int store_field = 0;          // fused step: predictor keeps H_ext for the corrector
     DevBuf field_buf;             // 3N R
-    DevBuf mm, atom_rep;
+    DevBuf mm;
     DevBuf mm_tab;                   // [nmat] each material's moment, when every atom has its material's
     // the moments the statistics read: the per-material table when it describes every atom
     Moments moments() const {
@@ -1265,11 +1176,14 @@ int vmx_ctx::capture_graph(int nsteps) {
     return VMX_OK;
 }
 
-// Workgroups of the partial-sum kernels.  Each thread walks its atoms with a grid stride, one
-// dependent memory round trip per atom, so masks with few bins get eight workgroups per CU
-// (2048); masks with many bins keep 512, which bounds the partials k_*_finish reduces.
+// Workgroups of the statistics kernels.  Up to 65,536 atoms every thread has one atom at most and the
+// launch is one round trip; beyond, a thread takes several, so that the workgroups' reductions and their
+// partials stay few: one workgroup per 1024 atoms between 256 and eight per CU (2048) (472,014 atoms, three
+// bins: 1844 workgroups of one atom a thread 20.6 us and 8.9 us to finish, 460 6.4 and 4.2).  Masks with
+// many bins keep 512 at most, which bounds their partials.
 int vmx_ctx::stats_grid(int nbins) const {
-    return std::max(1, std::min((n + 255) / 256, nbins <= 16 ? 2048 : 512));
+    if (nbins > 16) return std::max(1, std::min((n + 255) / 256, 512));
+    return n <= 65536 ? std::max(1, (n + 255) / 256) : std::min(2048, std::max(256, n / 1024));
 }
 // Bytes of workgroup partials the largest registered statistic needs.
 size_t vmx_ctx::stats_partial_bytes() const {
@@ -1292,20 +1206,14 @@ int vmx_ctx::stats_update(double* fixed) {
     }
     for (MagStat* st : mags) {
         const int grid = stats_grid(st->nbins);
-        VMX_HIP(Ops<R>::mag_partial(grid, stream, n, S, st->mask.as<int>(), moments(), st->nbins, part));
-        hipLaunchKernelGGL(k_mag_finish, dim3(1), dim3(256), 0, stream, grid, part, st->nbins,
-                           st->cur(), st->mean(), st->empty_dev.as<int>(), (int)st->empty.size(), st->counter());
-        VMX_HIP(hipGetLastError());
+        VMX_HIP(Ops<R>::magnetization(grid, stream, n, S, st->mask.as<int>(), moments(), st->nbins, part, st->out()));
     }
     if (!energies.empty()) {
         const SysDev<R> s = sys<R>();
         for (EnergyStat* st : energies) {
             const int grid = stats_grid(st->nbins);
-            VMX_HIP(Ops<R>::energy_partial(grid, stream, et, am(), s, S, st->mask.as<int>(), moments(),
-                                           nrep > 1 ? atom_rep.as<int>() : nullptr, st->nbins, part));
-            hipLaunchKernelGGL(k_energy_finish, dim3(1), dim3(256), 0, stream, grid, part, st->nbins,
-                               st->cur(), st->mean(), st->empty_dev.as<int>(), (int)st->empty.size(), st->counter());
-            VMX_HIP(hipGetLastError());
+            VMX_HIP(Ops<R>::energy(grid, stream, et, am(), s, (block + 63) / 64, S, st->mask.as<int>(), moments(), st->nbins, part,
+                                   st->out()));
         }
     }
     return VMX_OK;
@@ -2460,10 +2368,6 @@ int vmx_create(const vmx_system* sys, const vmx_options* opt, vmx_ctx** out) {
     }
     VMX_TRY(c->rep_off.alloc((nrep + 1) * sizeof(int)));
     VMX_HIP(hipMemcpy(c->rep_off.p, roff.data(), (nrep + 1) * sizeof(int), hipMemcpyHostToDevice));
-    if (nrep > 1) {   // replica of every atom (the energy statistics' applied field); replicas keep
-                      // their atom ranges in the internal order
-        VMX_TRY(upload(c->atom_rep, atom_rep_h));
-    }
     VMX_TRY(scratch_on_current_device(&c->stats_scratch));
     {
         std::vector<int> rep_m(nrep);

@@ -1301,15 +1301,36 @@ k_plain_corrector(SysDev<R> s, Spin3<R> S, Spin3<R> P, Spin3<R> F, Spin3<R> E, S
     S.x[i] = n0 * r; S.y[i] = n1 * r; S.z[i] = n2 * r;
 }
 
+// ---- sums over a wavefront in registers -----------------------------------------------------------
+// v of the lane that the DPP control CTRL reads from (rows in MASK; zero elsewhere)
+template <int CTRL, int MASK>
+__device__ __forceinline__ double dpp_from(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, MASK, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, MASK, 0xf, true);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+// The wavefront's sum of v, in lane 63 (a fixed order: within rows of 16 lanes by shifts, then rows 0 + 1
+// and 2 + 3, then both).  Stays in registers where shuffles pass through the LDS.
+__device__ __forceinline__ double wave_sum63(double v) {
+    v += dpp_from<0x111, 0xf>(v);            // row_shr:1, 2, 4, 8
+    v += dpp_from<0x112, 0xf>(v);
+    v += dpp_from<0x114, 0xf>(v);
+    v += dpp_from<0x118, 0xf>(v);
+    v += dpp_from<0x142, 0xa>(v);            // row_bcast:15 into rows 1 and 3
+    v += dpp_from<0x143, 0xc>(v);            // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 // ======================= statistics ==========================================================
 // Per-mask sums in FP64.  Each thread keeps a register accumulator for the mask id of its
 // current run of atoms and flushes it into the workgroup's LDS histogram when the id changes,
 // so a system-wide mask (one id) costs one LDS atomic per thread.  Each workgroup writes its
-// histogram to partial[block][nbins*W]; k_stats_finish reduces the partials in block order.
+// histogram to partial[block][nbins*W]; the finish reduces the partials in block order.
 
 // Fixed-order reduction of the threads' register histograms acc[MAXB][4] (bins < nbins <= MAXB)
-// into partial[block][nbins*4]: wavefront shuffles, then the wavefronts in order.  Workgroups of at
-// most 256 threads; every thread of the workgroup calls it.
+// into partial[block][nbins*4]: each wavefront in registers, then the wavefronts in order.  Workgroups
+// of at most 256 threads; every thread of the workgroup calls it.
 template <int MAXB>
 __device__ __forceinline__ void reduce_hist_regs(const double (&acc)[MAXB][4], int nbins,
                                                  double* __restrict__ partial) {
@@ -1319,9 +1340,8 @@ __device__ __forceinline__ void reduce_hist_regs(const double (&acc)[MAXB][4], i
     for (int b = 0; b < MAXB; ++b) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            double v = acc[b][c];
-            for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-            if (lane == 0) red[w][4 * b + c] = v;
+            const double v = wave_sum63(acc[b][c]);
+            if (lane == 63) red[w][4 * b + c] = v;
         }
     }
     __syncthreads();
@@ -1332,6 +1352,152 @@ __device__ __forceinline__ void reduce_hist_regs(const double (&acc)[MAXB][4], i
         for (int q = 0; q < nw; ++q) t += red[q][threadIdx.x];
         partial[(size_t)blockIdx.x * W + threadIdx.x] = t;
     }
+}
+
+// ---- the end of a statistic: one workgroup over the partials -----------------------------------------
+// (Taken over by the last workgroup of the partials' own launch instead, told by a ticket, it cost more:
+// with agent-scope fences each workgroup writes back and invalidates its XCD's L2, 4M atoms 18 + 6 us ->
+// 64; with stores and loads past the L2 the ticket's address serialises 2048 workgroups, 50 us, and three
+// workgroups of 729 atoms still take 7.0 against 3.0 + 3.0.)
+struct StatOut {
+    double* cur;                 // latest values
+    double* mean;                // running sums
+    long long* counter;          // updates
+    const int* empty;            // mask ids (< nbins - 1) without atoms
+    int nempty;
+};
+
+// Sum over the nblk per-workgroup partials [nblk][W] of every value k < W, handed to put(k, sum).
+// With fewer values than threads, each value's partials are split over blockDim / W threads whose
+// sub-sums are then added in thread order: the whole workgroup works and the order is fixed, so the
+// result is the same on every run.  With many values, one thread per value.  Loads go eight at a time
+// before any is added.
+template <typename F>
+__device__ __forceinline__ void reduce_partials(int nblk, const double* __restrict__ partial, int W, F&& put) {
+    __shared__ double red[256];              // workgroups of 256 threads
+    auto sum = [&](int k, int first, int step) {
+        double a = 0.0;
+        int b = first;
+        for (; b + 7 * step < nblk; b += 8 * step) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = partial[(size_t)(b + u * step) * W + k];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) a += v[u];
+        }
+        double v[7];
+#pragma unroll
+        for (int u = 0; u < 7; ++u) v[u] = partial[(size_t)(b + u * step < nblk ? b + u * step : 0) * W + k];
+#pragma unroll
+        for (int u = 0; u < 7; ++u)
+            if (b + u * step < nblk) a += v[u];
+        return a;
+    };
+    const int per = (int)blockDim.x / W;
+    if (per >= 2) {
+        const int k = (int)threadIdx.x % W, j = (int)threadIdx.x / W;
+        red[threadIdx.x] = j < per ? sum(k, j, per) : 0.0;
+        __syncthreads();
+        if ((int)threadIdx.x < W) {
+            double t = 0.0;
+            for (int q = 0; q < per; ++q) t += red[q * W + (int)threadIdx.x];
+            put((int)threadIdx.x, t);
+        }
+    } else {
+        for (int k = threadIdx.x; k < W; k += blockDim.x) put(k, sum(k, 0, 1));
+    }
+    __threadfence_block();
+    __syncthreads();
+}
+
+// The values of a statistic while they are formed: in LDS for masks of few bins (each step on them is then
+// no round trip to memory), else where the caller reads them.
+constexpr int kStatLdsValues = 80;           // 16 bins of 5 energies
+__device__ __forceinline__ double* stat_lds() {
+    __shared__ double v[kStatLdsValues];
+    return v;
+}
+
+// Magnetisation from the partials, normalised (magnetization.cpp:150-178).
+__device__ __forceinline__ void mag_finish(int nblk, const double* __restrict__ partial, int nbins, const StatOut& o) {
+    const int W = 4 * nbins;
+    auto form = [&](double* cur) {
+        reduce_partials(nblk, partial, W, [&](int k, double v) { cur[k] = v; });
+        for (int id = threadIdx.x; id < nbins - 1; id += blockDim.x) {
+            const double msat = cur[4 * id + 3];
+            const double magm = sqrt(cur[4 * id + 0] * cur[4 * id + 0] + cur[4 * id + 1] * cur[4 * id + 1] +
+                                     cur[4 * id + 2] * cur[4 * id + 2]);
+            cur[4 * id + 0] = cur[4 * id + 0] / magm;
+            cur[4 * id + 1] = cur[4 * id + 1] / magm;
+            cur[4 * id + 2] = cur[4 * id + 2] / magm;
+            cur[4 * id + 3] = magm / msat;
+        }
+        __threadfence_block();
+        __syncthreads();
+        for (int e = threadIdx.x; e < o.nempty; e += blockDim.x) {
+            const int id = o.empty[e];
+            cur[4 * id + 0] = 0.0; cur[4 * id + 1] = 0.0; cur[4 * id + 2] = 0.0; cur[4 * id + 3] = 0.0;
+        }
+        __threadfence_block();
+        __syncthreads();
+    };
+    const long long count = threadIdx.x == 0 ? *o.counter : 0;
+    if (W <= kStatLdsValues) {
+        const int k = (int)threadIdx.x;
+        const double mean = k < W ? o.mean[k] : 0.0;
+        double* cur = stat_lds();
+        form(cur);
+        if (k < W) { o.cur[k] = cur[k]; o.mean[k] = mean + cur[k]; }
+    } else {
+        form(o.cur);
+        for (int k = threadIdx.x; k < W; k += blockDim.x) o.mean[k] += o.cur[k];
+    }
+    if (threadIdx.x == 0) *o.counter = count + 1;
+}
+
+// Energies [5][nbins]: total, exchange, anisotropy, applied, magnetostatic
+// (src/statistics/energy.cpp:141-258; the magnetostatic term is zero without a device dipole field).
+__device__ __forceinline__ void energy_finish(int nblk, const double* __restrict__ partial, int nbins, const StatOut& o) {
+    const int V = 5 * nbins, ms = nbins - 1;
+    // the running sums take every bin but the last, before the bins without atoms are cleared
+    auto form = [&](double* cur, auto&& add) {
+        for (int id = threadIdx.x; id < nbins; id += blockDim.x) cur[id] = 0.0;
+        reduce_partials(nblk, partial, 4 * nbins, [&](int k, double v) {
+            const int id = k / 4, term = k % 4;     // term: exchange, anisotropy, applied, magnetostatic
+            cur[(size_t)(1 + term) * nbins + id] = v;
+        });
+        for (int id = threadIdx.x; id < ms; id += blockDim.x) {
+            cur[(size_t)1 * nbins + id] = 0.5 * cur[(size_t)1 * nbins + id];
+            cur[(size_t)4 * nbins + id] = 0.5 * cur[(size_t)4 * nbins + id];
+            cur[id] = cur[(size_t)1 * nbins + id] + cur[(size_t)2 * nbins + id] + cur[(size_t)3 * nbins + id] +
+                      cur[(size_t)4 * nbins + id];
+        }
+        __threadfence_block();
+        __syncthreads();
+        add();
+        __threadfence_block();
+        __syncthreads();
+        for (int e = threadIdx.x; e < o.nempty; e += blockDim.x) {
+            const int id = o.empty[e];
+            for (int t = 0; t < 5; ++t) cur[(size_t)t * nbins + id] = 0.0;
+        }
+        __threadfence_block();
+        __syncthreads();
+    };
+    const long long count = threadIdx.x == 0 ? *o.counter : 0;
+    if (V <= kStatLdsValues) {
+        const int k = (int)threadIdx.x;
+        const double mean = k < V ? o.mean[k] : 0.0;
+        double* cur = stat_lds();
+        form(cur, [&] { if (k < V && k % nbins < ms) o.mean[k] = mean + cur[k]; });
+        if (k < V) o.cur[k] = cur[k];
+    } else {
+        form(o.cur, [&] {
+            for (int k = threadIdx.x; k < V; k += blockDim.x)
+                if (k % nbins < ms) o.mean[k] += o.cur[k];
+        });
+    }
+    if (threadIdx.x == 0) *o.counter = count + 1;
 }
 
 // Each atom's moment (mu_B) for the statistics: per atom, or, when every atom's moment is its
@@ -1348,18 +1514,13 @@ struct Moments {
 // atom to its bin with predicated adds, so the cost does not depend on how often the id changes
 // along the atoms (a random alloy's material mask changes at nearly every atom).  The workgroup
 // then reduces its threads' sums in a fixed order (wavefront shuffles, then the wavefronts in
-// order) into partial[block][nbins*4], the layout k_mag_partial writes.
+// order) into partial[block][nbins*4], the layout k_mag_hist writes.
 template <typename R, int MAXB>
 __global__ void __launch_bounds__(256)
-k_mag_partial_regs(int n, Spin3<R> S, const int* __restrict__ mask, Moments mo, int nbins,
-                   double* __restrict__ partial) {
+k_mag_regs(int n, Spin3<R> S, const int* __restrict__ mask, Moments mo, int nbins, double* __restrict__ partial) {
     double acc[MAXB][4];
 #pragma unroll
     for (int b = 0; b < MAXB; ++b) { acc[b][0] = 0.0; acc[b][1] = 0.0; acc[b][2] = 0.0; acc[b][3] = 0.0; }
-    // with up to four bins, four of the thread's atoms are loaded before any is added (then added
-    // in the same order as one at a time), so each wavefront has four atoms' loads in flight; with
-    // eight the histogram's 64 registers leave no room, and atoms go one at a time
-    constexpr int U = MAXB >= 8 ? 1 : 4;
     auto add = [&](int id, double m, R x, R y, R z) {
         const double v0 = (double)x * m, v1 = (double)y * m, v2 = (double)z * m;
 #pragma unroll
@@ -1371,27 +1532,32 @@ k_mag_partial_regs(int n, Spin3<R> S, const int* __restrict__ mask, Moments mo, 
             acc[b][3] += hit ? m : 0.0;
         }
     };
-    if constexpr (U == 1) {
-        for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-            add(MAXB == 1 ? 0 : mask[i], mo.at(i), S.x[i], S.y[i], S.z[i]);
-    } else {
-        const int stride = (int)(gridDim.x * blockDim.x);
-        int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-        for (; (long long)i + (U - 1) * (long long)stride < n; i += U * stride) {
-            int id[U];
-            double m[U];
-            R x[U], y[U], z[U];
+    // a one-bin mask holds 0 everywhere: not read
+    const int stride = (int)(gridDim.x * blockDim.x), first = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (n <= stride) {                   // one atom a thread
+        if (first < n) add(MAXB == 1 ? 0 : mask[first], mo.at(first), S.x[first], S.y[first], S.z[first]);
+        reduce_hist_regs<MAXB>(acc, nbins, partial);
+        return;
+    }
+    // U of the thread's atoms are loaded before any is added (in order), so that a wavefront has that many
+    // atoms' loads in flight; with eight bins the histogram's 64 registers leave room for two.  Past the end
+    // the last atom is loaded and added to no bin, so the remainder is one more round, not one per atom.
+    constexpr int U = MAXB >= 8 ? 2 : (MAXB == 4 ? 4 : 8);
+    for (long long i = first; i < n; i += (long long)U * stride) {
+        int id[U];
+        double m[U];
+        R x[U], y[U], z[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int k = i + u * stride;
-                id[u] = MAXB == 1 ? 0 : mask[k];   // a one-bin mask holds 0 everywhere: not read
-                m[u] = mo.at(k);
-                x[u] = S.x[k]; y[u] = S.y[k]; z[u] = S.z[k];
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) add(id[u], m[u], x[u], y[u], z[u]);
+        for (int u = 0; u < U; ++u) {
+            const long long at = i + (long long)u * stride;
+            const int k = at < n ? (int)at : n - 1;
+            id[u] = MAXB == 1 ? 0 : mask[k];
+            if (at >= n) id[u] = -1;
+            m[u] = mo.at(k);
+            x[u] = S.x[k]; y[u] = S.y[k]; z[u] = S.z[k];
         }
-        for (; i < n; i += stride) add(MAXB == 1 ? 0 : mask[i], mo.at(i), S.x[i], S.y[i], S.z[i]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) add(id[u], m[u], x[u], y[u], z[u]);
     }
     reduce_hist_regs<MAXB>(acc, nbins, partial);
 }
@@ -1399,9 +1565,8 @@ k_mag_partial_regs(int n, Spin3<R> S, const int* __restrict__ mask, Moments mo, 
 // W = 4: sum(m s_x), sum(m s_y), sum(m s_z), sum(m)   (magnetization.cpp:141-147)
 template <typename R>
 __global__ void __launch_bounds__(256)
-k_mag_partial(int n, Spin3<R> S, const int* __restrict__ mask, Moments mo, int nbins,
-              double* __restrict__ partial) {
-    extern __shared__ double hist[];
+k_mag_hist(int n, Spin3<R> S, const int* __restrict__ mask, Moments mo, int nbins, double* __restrict__ partial) {
+    double* const hist = reinterpret_cast<double*>(vmx_lds);
     for (int k = threadIdx.x; k < 4 * nbins; k += blockDim.x) hist[k] = 0.0;
     __syncthreads();
     int cur = -1;
@@ -1426,8 +1591,8 @@ k_mag_partial(int n, Spin3<R> S, const int* __restrict__ mask, Moments mo, int n
         atomicAdd(&hist[4 * cur + 2], a2); atomicAdd(&hist[4 * cur + 3], a3);
     }
     __syncthreads();
-    double* out = partial + (size_t)blockIdx.x * 4 * nbins;
-    for (int k = threadIdx.x; k < 4 * nbins; k += blockDim.x) out[k] = hist[k];
+    double* mine = partial + (size_t)blockIdx.x * 4 * nbins;
+    for (int k = threadIdx.x; k < 4 * nbins; k += blockDim.x) mine[k] = hist[k];
 }
 
 // Single-spin energies (tesla): exchange (src/exchange/energy.cpp:27-104), anisotropy
@@ -1542,67 +1707,92 @@ __device__ __forceinline__ R magnetostatic_energy(const SysDev<R>& s, int i, R s
 }
 
 // W = 4: exchange, anisotropy, applied, magnetostatic, each times m_i (energy.cpp:155-203); the
-// last is zero without a device dipole field
+// last is zero without a device dipole field.  A workgroup takes a contiguous run of the block table's
+// 64-atom units (units per entry; with XCD remapping, of its XCD's stretch), a wavefront a unit, so the rows it gathers lie in its own L2, the replica and its
+// conditions come with the entry, and the stencil offsets are staged in LDS.  Bound by the gathers, like a
+// step's field (FP32: 4M FCC atoms 67 -> 56 us, 472,014-atom film 26.5 -> 22.7; FP64 1M FCC 42.8 -> 36.7).
 template <typename R, int ET, int AM>
 __global__ void __launch_bounds__(256)
-k_energy_partial(SysDev<R> s, Spin3<R> S, const int* __restrict__ mask, Moments mo,
-                 const int* __restrict__ atom_rep, int nbins, double* __restrict__ partial) {
-    if (nbins <= 4) {                // few bins: register histograms, as k_mag_partial_regs
-        double acc[4][4];
-#pragma unroll
-        for (int b = 0; b < 4; ++b) { acc[b][0] = 0.0; acc[b][1] = 0.0; acc[b][2] = 0.0; acc[b][3] = 0.0; }
-        for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < s.n; i += gridDim.x * blockDim.x) {
-            const int id = mask[i];
-            const R sx = S.x[i], sy = S.y[i], sz = S.z[i];
-            const int m = s.type[i];
-            const int rep = atom_rep ? atom_rep[i] : 0;
-            const double w = mo.at(i);
-            const double e0 = (double)exchange_energy<R, ET, AM>(s, S.x, S.y, S.z, i, sx, sy, sz) * w;
-            const double e1 = (double)anisotropy_energy(s, m, sx, sy, sz) * w;
-            const double e2 = (double)applied_energy(s.cond[rep * s.nmat + m], sx, sy, sz) * w;
-            const double e3 = s.hd ? (double)magnetostatic_energy(s, i, sx, sy, sz) * w : 0.0;
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const bool hit = id == b;
-                acc[b][0] += hit ? e0 : 0.0;
-                acc[b][1] += hit ? e1 : 0.0;
-                acc[b][2] += hit ? e2 : 0.0;
-                acc[b][3] += hit ? e3 : 0.0;
-            }
-        }
-        reduce_hist_regs<4>(acc, nbins, partial);
-        return;
-    }
-    extern __shared__ double hist[];
-    for (int k = threadIdx.x; k < 4 * nbins; k += blockDim.x) hist[k] = 0.0;
+k_energy(SysDev<R> s, int units, Spin3<R> S, const int* __restrict__ mask, Moments mo, int nbins,
+         double* __restrict__ partial) {
+    constexpr int TP = Access<AM>::TP, W = Access<AM>::W;
+    const bool few = nbins <= 4;     // few bins: register histograms, as k_mag_regs
+    double* const hist = reinterpret_cast<double*>(vmx_lds);
+    int* const offs = vmx_lds + (few ? 0 : 8 * nbins);
+    if (TP == TP_PAT && s.pat_lds)
+        for (int k = threadIdx.x; k < s.npat * W; k += blockDim.x) offs[k] = s.pat_off[k];
+    if (!few)
+        for (int k = threadIdx.x; k < 4 * nbins; k += blockDim.x) hist[k] = 0.0;
     __syncthreads();
+    double acc[4][4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) { acc[b][0] = 0.0; acc[b][1] = 0.0; acc[b][2] = 0.0; acc[b][3] = 0.0; }
+    const UniformJ<R, ET> ju(s, Access<AM>::JM);
+    const SpinRsrc<R> rs(s, S.x, S.y, S.z);
+    const bool remap = s.xcd_remap && (gridDim.x & 7) == 0;
+    const long long lb = logical_block(remap ? 1 : 0);
+    const long long all = (long long)s.nblocks * units;
+    const long long u0 = lb * all / gridDim.x, u1 = (lb + 1) * all / gridDim.x;
     int cur = -1;
     double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < s.n; i += gridDim.x * blockDim.x) {
-        const int id = mask[i];
-        if (id != cur) {
-            if (cur >= 0) {
-                atomicAdd(&hist[4 * cur + 0], a0); atomicAdd(&hist[4 * cur + 1], a1);
-                atomicAdd(&hist[4 * cur + 2], a2); atomicAdd(&hist[4 * cur + 3], a3);
+    for (long long u = u0 + (threadIdx.x >> 6); u < u1; u += blockDim.x >> 6) {
+        const int entry = (int)(u / units);
+        const int4 b = s.blk[entry];
+        const int i = b.x + 64 * (int)(u - (long long)entry * units) + (int)__lane_id();
+        if (i < b.z) {
+            const int head = row_head<R, AM>(s, i);
+            const int id = mask[i];
+            R sx, sy, sz;
+            rs.load(i, sx, sy, sz);
+            const int m = s.type[i];
+            const double w = mo.at(i);
+            R ex;
+            if constexpr (TP == TP_CSR) {
+                ex = exchange_energy<R, ET, AM>(s, S.x, S.y, S.z, i, sx, sy, sz);
+            } else {
+                RowIdx<AM> r;
+                if (TP == TP_PAT && s.pat_lds) row_index(s, i, head, offs, r);
+                else row_index(s, i, head, s.pat_off, r);
+                RowSpins<R, AM> v;
+                row_load(rs, r, v);
+                ex = row_exchange_energy<R, ET, AM>(s, r, v, ju.v, sx, sy, sz);
             }
-            cur = id; a0 = a1 = a2 = a3 = 0.0;
+            const double t0 = (double)ex * w;
+            const double t1 = (double)anisotropy_energy(s, m, sx, sy, sz) * w;
+            const double t2 = (double)applied_energy(s.cond[b.y * s.nmat + m], sx, sy, sz) * w;
+            const double t3 = s.hd ? (double)magnetostatic_energy(s, i, sx, sy, sz) * w : 0.0;
+            if (few) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const bool hit = id == k;
+                    acc[k][0] += hit ? t0 : 0.0;
+                    acc[k][1] += hit ? t1 : 0.0;
+                    acc[k][2] += hit ? t2 : 0.0;
+                    acc[k][3] += hit ? t3 : 0.0;
+                }
+                continue;
+            }
+            if (id != cur) {
+                if (cur >= 0) {
+                    atomicAdd(&hist[4 * cur + 0], a0); atomicAdd(&hist[4 * cur + 1], a1);
+                    atomicAdd(&hist[4 * cur + 2], a2); atomicAdd(&hist[4 * cur + 3], a3);
+                }
+                cur = id; a0 = a1 = a2 = a3 = 0.0;
+            }
+            a0 += t0; a1 += t1; a2 += t2; a3 += t3;
         }
-        const R sx = S.x[i], sy = S.y[i], sz = S.z[i];
-        const int m = s.type[i];
-        const int rep = atom_rep ? atom_rep[i] : 0;
-        const double w = mo.at(i);
-        a0 += (double)exchange_energy<R, ET, AM>(s, S.x, S.y, S.z, i, sx, sy, sz) * w;
-        a1 += (double)anisotropy_energy(s, m, sx, sy, sz) * w;
-        a2 += (double)applied_energy(s.cond[rep * s.nmat + m], sx, sy, sz) * w;
-        if (s.hd) a3 += (double)magnetostatic_energy(s, i, sx, sy, sz) * w;
     }
-    if (cur >= 0) {
-        atomicAdd(&hist[4 * cur + 0], a0); atomicAdd(&hist[4 * cur + 1], a1);
-        atomicAdd(&hist[4 * cur + 2], a2); atomicAdd(&hist[4 * cur + 3], a3);
+    if (few) {
+        reduce_hist_regs<4>(acc, nbins, partial);
+    } else {
+        if (cur >= 0) {
+            atomicAdd(&hist[4 * cur + 0], a0); atomicAdd(&hist[4 * cur + 1], a1);
+            atomicAdd(&hist[4 * cur + 2], a2); atomicAdd(&hist[4 * cur + 3], a3);
+        }
+        __syncthreads();
+        double* mine = partial + (size_t)blockIdx.x * 4 * nbins;
+        for (int k = threadIdx.x; k < 4 * nbins; k += blockDim.x) mine[k] = hist[k];
     }
-    __syncthreads();
-    double* out = partial + (size_t)blockIdx.x * 4 * nbins;
-    for (int k = threadIdx.x; k < 4 * nbins; k += blockDim.x) out[k] = hist[k];
 }
 
 // ======================= checkerboard Metropolis =============================================

@@ -737,6 +737,8 @@ struct vmx_ctx {
                      fused_lds_bytes<R>(nmat, npat, zmax, s.pat_lds, (size_t)njt * K) <= 65536) ? njt : 0;
         s.am = am();
         s.q = q;
+        s.span = nrep == 1 ? block : 0;
+        s.cells = n / q;
         s.rep_m = rep_m.as<int>();
         s.row = row.as<int>(); s.col = col.as<int>();
         s.jidx = jm == JM_UNIFORM ? nullptr : jidx.p;
@@ -782,6 +784,7 @@ struct vmx_ctx {
     SysDev<R> sys_fused() const {
         SysDev<R> s = sys<R>();
         s.blk = blk_fused.as<int4>();
+        s.span *= fused_atoms();
         s.nblocks = nblocks_fused;
         return s;
     }

@@ -96,6 +96,9 @@ struct SysDev {
                                              // (16-bit J ids; 0: the table stays in memory)
     int am;                                  // access mode the arrays below were built for
     int q;                                   // basis-major atom order with period q (1: caller's order)
+    int span;                                // one replica: cells per entry of blk, which block_entry then
+                                             // computes instead of loading; 0: several replicas
+    int cells;                               // one replica: n / q
     const int* __restrict__ rep_m;           // [nrep] replica size / q
     const int* __restrict__ row;             // CSR: [n+1]
     const int* __restrict__ col;             // CSR: [nnz]; ELL: [zmax][n]
@@ -237,6 +240,19 @@ __device__ __forceinline__ int caller_local(const SysDev<R>& s, int rep, int p) 
     int b = 0;
     while (p >= m) { p -= m; ++b; }   // at most q - 1 iterations
     return p * s.q + b;
+}
+
+// Entry lb of the block table in a step kernel.  ELL rows of one replica: from the launch's arguments, so
+// that the row's three levels of loads (indices, ids, neighbours) do not wait for a fourth (472,014-atom
+// film FP32 25.2 -> 23.8 us a step).  Stencil rows have one level fewer, and there the division and the
+// registers cost what the load does (4M FCC 77.9 -> 78.4, 2.7M-atom batch 47.4 -> 47.8): they load it.
+template <typename R, int AM>
+__device__ __forceinline__ int4 block_entry(const SysDev<R>& s, int lb) {
+    if (Access<AM>::TP != TP_ELL || s.span == 0) return s.blk[lb];
+    int chunk = lb, basis = 0;
+    if (s.q > 1) { chunk = lb / s.q; basis = lb - chunk * s.q; }
+    const int c0 = chunk * s.span, first = basis * s.cells + c0;
+    return make_int4(first, 0, first + min(s.span, s.cells - c0), 0);
 }
 
 // i: internal atom index; local: the caller's replica-local index (keys the Philox counter)
@@ -818,7 +834,7 @@ k_fused_predictor(SysDev<R> s, Spin3<R> S, Spin3<R> P, Spin3<R> D, Spin3<R> E, c
     constexpr bool kStaged = Access<AM>::TP != TP_CSR;
     const int lb = logical_block(s.xcd_remap);
     if (lb >= s.nblocks) return;                 // whole workgroup
-    const int4 b = s.blk[lb];
+    const int4 b = block_entry<R, AM>(s, lb);
     int idx[U];
     bool ok[U];
     fused_atoms<U>(b, idx, ok);
@@ -884,7 +900,7 @@ k_fused_corrector(SysDev<R> s, Spin3Alias<R> S, Spin3<R> P, Spin3Alias<R> O, Spi
     constexpr bool kStaged = Access<AM>::TP != TP_CSR;
     const int lb = logical_block(s.xcd_remap);
     if (lb >= s.nblocks) return;                 // whole workgroup
-    const int4 b = s.blk[lb];
+    const int4 b = block_entry<R, AM>(s, lb);
     int idx[U];
     bool ok[U];
     fused_atoms<U>(b, idx, ok);
@@ -994,7 +1010,7 @@ k_mid_predictor(SysDev<R> s, Spin3<R> S, Spin3<R> P, Spin3<R> E, const double* _
     constexpr bool kStaged = Access<AM>::TP != TP_CSR;
     const int lb = logical_block(s.xcd_remap);
     if (lb >= s.nblocks) return;
-    const int4 b = s.blk[lb];
+    const int4 b = block_entry<R, AM>(s, lb);
     int idx[U];
     bool ok[U];
     fused_atoms<U>(b, idx, ok);
@@ -1053,7 +1069,7 @@ k_mid_corrector(SysDev<R> s, Spin3Alias<R> S, Spin3<R> P, Spin3Alias<R> O, Spin3
     constexpr bool kStaged = Access<AM>::TP != TP_CSR;
     const int lb = logical_block(s.xcd_remap);
     if (lb >= s.nblocks) return;
-    const int4 b = s.blk[lb];
+    const int4 b = block_entry<R, AM>(s, lb);
     int idx[U];
     bool ok[U];
     fused_atoms<U>(b, idx, ok);

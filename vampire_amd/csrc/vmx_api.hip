@@ -621,7 +621,12 @@ struct vmx_ctx {
     int cmc_move = 0;                      // 0: cone of the replica's Metropolis width; 1: angle move
     template <typename R>
     int cmc_sweeps(int nsweeps);
-    int cmc_permutations(uint64_t sw);
+    int cmc_permutations(uint64_t sw, int nsweeps);
+    // Rounds sum the partials of the round before themselves (CmcMoment) while a replica has at most
+    // kCmcFoldPartials of them, two loads a thread; the first colour without pairs ends a replica's rounds.
+    bool cmc_fold = false;
+    static constexpr int kCmcFoldPartials = 512;
+    static constexpr size_t kCmcPermBytes = (size_t)1 << 20;   // permutations made ahead of their sweeps
     int colour_order(const std::vector<int>& c, const std::vector<int>& lau, int nc);
     template <typename R>
     SysDev<R> sys_colour_order() const;
@@ -1400,8 +1405,18 @@ int vmx_ctx::colour() {
     VMX_TRY(upload(cmc_tab, ctab));
     VMX_TRY(upload(cmc_range, crange));
     VMX_TRY(upload(cmc_mlen, cmlen));
-    VMX_TRY(cmc_perm.alloc(2 * (size_t)nc * nrep * sizeof(int4)));
-    VMX_TRY(cmc_dm.alloc(3 * std::max<size_t>(ctab.size(), 1) * sizeof(double)));
+    VMX_TRY(cmc_perm.alloc(std::max(2 * (size_t)nc * nrep * sizeof(int4), kCmcPermBytes)));
+    VMX_TRY(cmc_dm.alloc(2 * 3 * std::max<size_t>(ctab.size(), 1) * sizeof(double)));   // per round
+    cmc_fold = true;
+    for (int r = 0; r < nrep; ++r) {
+        bool done = false;
+        for (int k = 0; k < nc; ++k) {
+            const int parts = crange[(size_t)k * (nrep + 1) + r + 1] - crange[(size_t)k * (nrep + 1) + r];
+            if (parts > kCmcFoldPartials || (parts > 0 && done)) cmc_fold = false;
+            done = done || parts == 0;
+        }
+        if ((rep_off_h[r + 1] - rep_off_h[r]) / 64 / q + 2 * q > 8 * kCmcFoldPartials) cmc_fold = false;
+    }
     ncolours = nc;
     coloured = true;
     return VMX_OK;
@@ -1552,14 +1567,15 @@ int vmx_ctx::mc_sweeps(int nsweeps) {
     return VMX_OK;
 }
 
-// The permutations of every (colour, round, replica) of sweep sw into cmc_perm: for a table of up
-// to 1 KiB (a few replicas) formed here with the device's own integer arithmetic and written by a
-// one-workgroup launch whose arguments carry it; else by k_cmc_perm, one thread per entry.  The
-// device kernel is a chain of dependent divisions (≈ 10 µs), longer than a small system's round.
-int vmx_ctx::cmc_permutations(uint64_t sw) {
+// The permutations of every (colour, round, replica) of the nsweeps sweeps from sw on into cmc_perm.  One
+// sweep's table of up to 1 KiB (a few replicas) is formed here with the device's own integer arithmetic and
+// written by a one-workgroup launch whose arguments carry it; else by k_cmc_perm, one thread per entry.  The
+// device kernel is a chain of dependent divisions (7-10 us whatever the number of entries), longer than a
+// small system's round, so it makes many sweeps' at once.
+int vmx_ctx::cmc_permutations(uint64_t sw, int nsweeps) {
     const size_t count = 2 * (size_t)ncolours * nrep;
-    if (count * sizeof(int4) > sizeof(ArgWords)) {
-        VMX_HIP(Ops<float>::cmc_perm(stream, rep_key.as<uint2>(), nrep, ncolours, cmc_mlen.as<int>(), sw,
+    if (nsweeps > 1 || count * sizeof(int4) > sizeof(ArgWords)) {
+        VMX_HIP(Ops<float>::cmc_perm(stream, rep_key.as<uint2>(), nrep, ncolours, cmc_mlen.as<int>(), sw, nsweeps,
                                      cmc_perm.as<int4>()));
         return VMX_OK;
     }
@@ -1597,7 +1613,7 @@ int vmx_ctx::cmc_sweeps(int nsweeps) {
         VMX_TRY(upload(cmc_frame, f));
         cmc_frame_dirty = false;
     }
-    VMX_TRY(cmc_M.alloc(3 * (size_t)nrep * sizeof(double)));
+    VMX_TRY(cmc_M.alloc(2 * 3 * (size_t)nrep * sizeof(double)));   // folded rounds alternate
     VMX_TRY(cmc_part.alloc(3 * (size_t)nblocks * sizeof(double)));
     const SysDev<R> s = sys<R>();
     const Spin3<R> S = spins<R>(s_idx);
@@ -1620,24 +1636,34 @@ int vmx_ctx::cmc_sweeps(int nsweeps) {
     const int* plidx = ordered ? mco_lidx.as<int>() : nullptr;
     const double* pmm = ordered ? mco_mm.as<double>() : mm.as<double>();
     const int* gather = ordered ? mco_invp.as<int>() : nullptr;
+    const size_t nperm = 2 * (size_t)ncolours * nrep, ndm = 3 * (size_t)cmc_tab_start[ncolours];
+    const int ahead = (int)std::max<size_t>(1, std::min<size_t>(64, cmc_perm.bytes / (nperm * sizeof(int4))));
+    double* const dm0 = cmc_dm.as<double>();
     for (int w = 0; w < nsweeps; ++w) {
         if (last < 0) { ++sweep; continue; }
-        VMX_TRY(cmc_permutations(sweep));
+        if (w % ahead == 0) VMX_TRY(cmc_permutations(sweep, std::min(ahead, nsweeps - w)));
         VMX_HIP(Ops<R>::replica_moment(stream, s, C, moments(), gather, rep_blk.as<int>(), nrep,
-                                       cmc_part.as<double>(), cmc_M.as<double>()));
+                                       cmc_part.as<double>(), cmc_M.as<double>(), !cmc_fold));
+        // folded: a round starts from the sums before it; the sweep's first from the full sum's partials
+        CmcMoment mom{cmc_M.as<double>(), nullptr, nullptr, nullptr};
+        if (cmc_fold) mom = CmcMoment{nullptr, cmc_part.as<double>(), rep_blk.as<int>(), cmc_M.as<double>()};
         for (int k = 0; k <= last; ++k) {
             const int ntab = cmc_tab_start[k + 1] - cmc_tab_start[k];
             if (ntab == 0) continue;
-            double* dm = cmc_dm.as<double>() + 3 * (size_t)cmc_tab_start[k];
+            const int* range = cmc_range.as<int>() + (size_t)k * (nrep + 1);
             for (int round = 0; round < 2; ++round) {
+                double* dm = dm0 + (size_t)round * ndm + 3 * (size_t)cmc_tab_start[k];
                 VMX_HIP(Ops<R>::cmc_pairs(stream, et, am(), so, C, pmm, plist, plidx,
                                           cmc_tab.as<int4>() + cmc_tab_start[k], ntab,
-                                          cmc_perm.as<int4>() + (size_t)(2 * k + round) * nrep,
-                                          cmc_frame.as<CmcFrame<R>>(), cmc_M.as<double>(), mc_sigma(),
-                                          cmc_move, round, sweep, cmc_counts.as<double>(), dm));
-                if (k < last || round == 0)
-                    VMX_HIP(Ops<R>::moment_add(stream, cmc_range.as<int>() + (size_t)k * (nrep + 1), nrep, dm,
-                                               cmc_M.as<double>()));
+                                          cmc_perm.as<int4>() + (size_t)(w % ahead) * nperm + (size_t)(2 * k + round) * nrep,
+                                          cmc_frame.as<CmcFrame<R>>(), mom, mc_sigma(), cmc_move, round, sweep,
+                                          cmc_counts.as<double>(), dm));
+                if (cmc_fold) {
+                    double* other = cmc_M.as<double>() + (mom.M_out == cmc_M.as<double>() ? 3 * (size_t)nrep : 0);
+                    mom = CmcMoment{mom.M_out, dm, range, other};
+                } else if (k < last || round == 0) {
+                    VMX_HIP(Ops<R>::moment_add(stream, range, nrep, dm, cmc_M.as<double>()));
+                }
             }
         }
         ++sweep;   // a constrained sweep advances sim::time like a Heun step (sim.cpp:623-628)

@@ -73,17 +73,19 @@ struct Ops {
     static hipError_t cmc_pairs(hipStream_t st, int et, int jm, const SysDev<R>& s, Spin3<R> S, const double* mm,
                                 const int* list, const int* lidx, const int4* tab, int ntab, const int4* perm,
                                 const CmcFrame<R>* frame,
-                                const double* M, const double* sigma, int move, int round, uint64_t sweep,
+                                const CmcMoment& mom, const double* sigma, int move, int round, uint64_t sweep,
                                 double* counts, double* dM);
-    // the permutations of every (colour, round, replica) of a sweep: perm[(2 k + round) nrep + r] =
-    // {a, b, a^-1 mod m, 0} for the run length m = mlen[k nrep + r] (m < 2: {1, 0, 1, 0})
+    // the permutations of every (colour, round, replica) of nsweeps sweeps from `sweep` on:
+    // perm[(2 k + round) nrep + r] of each = {a, b, a^-1 mod m, 0} for the run length m = mlen[k nrep + r]
+    // (m < 2: {1, 0, 1, 0})
     static hipError_t cmc_perm(hipStream_t st, const uint2* rep_key, int nrep, int ncolours, const int* mlen,
-                               uint64_t sweep, int4* perm);
+                               uint64_t sweep, int nsweeps, int4* perm);
     // each replica's sum(mu s) (double [nrep][3]): per-workgroup partials over the one-atom block
     // table, then one workgroup per replica over its partials (rep_blk[r] .. rep_blk[r+1])
-    // (gather: spins in colour order, atom i's at gather[i]; else null)
+    // (gather: spins in colour order, atom i's at gather[i]; else null; finish false: the partials only)
     static hipError_t replica_moment(hipStream_t st, const SysDev<R>& s, Spin3<R> S, Moments mo,
-                                     const int* gather, const int* rep_blk, int nrep, double* partial, double* M);
+                                     const int* gather, const int* rep_blk, int nrep, double* partial, double* M,
+                                     bool finish);
     // M[r] += the sum of the cmc_pairs partials dM[range[r] .. range[r+1]], in a fixed order
     static hipError_t moment_add(hipStream_t st, const int* range, int nrep, const double* dM, double* M);
     // deterministic fitting step and its adjoint (isotropic uniform exchange); grids of 256; p: device

@@ -61,6 +61,11 @@ struct DevBuf {
         bytes = b;
         return VMX_OK;
     }
+    void release() {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        bytes = 0;
+    }
     template <typename T> T* as() const { return static_cast<T*>(p); }
 };
 
@@ -149,8 +154,11 @@ struct HostPipe {
                 chunks.push_back(Seg{(char*)seg[k].host + o, (char*)seg[k].dev + o, std::min(bytes, seg[k].bytes - o)});
                 total += chunks.back().bytes;
             }
-        const int workers = (int)std::min<size_t>(kWorkers, 1 + total / ((size_t)8 << 20));
-        VMX_TRY(ready(workers));
+        int workers = (int)std::min<size_t>(kWorkers, 1 + total / ((size_t)8 << 20));
+        if (ready(workers) != VMX_OK) {          // no pinned memory for more: the first one's slots are there
+            (void)hipGetLastError();
+            workers = 1;
+        }
         int dev = 0;
         VMX_HIP(hipGetDevice(&dev));
         hipError_t err[kWorkers] = {};
@@ -541,6 +549,7 @@ struct vmx_ctx {
     TileDev tile{};
     DevBuf tile_buf;
     int build_tiles(int64_t steps);
+    int make_tiles();
     DevBuf plainF, plainE, plainD;
     int store_euler = 1;          // fused FP64 step: the predictor keeps dS (FP32 keeps nothing)
     DevBuf euler_buf;             // 3N R
@@ -1722,14 +1731,25 @@ int vmx_ctx::fit_forward(const double* h, const double* spins0, double* mz_out) 
     VMX_HIP(hipStreamSynchronize(stream));         // a buffer that grows is freed: nothing may use it
     const int Gr = std::min(fit.nsteps, kFitSegment);
     const size_t all = 2 * (size_t)((fit.nsteps + Gr - 1) / Gr) * Gr * sb;
-    fit.resident = all <= kFitResident && fit.traj.alloc(all) == VMX_OK;
-    if (!fit.resident) (void)hipGetLastError();    // no room for the trajectory: checkpoints
-    fit.G = fit.resident ? Gr : std::min(fit.K, fit.nsteps);
-    fit.keepP = fit.resident || 2 * (size_t)fit.G * sb <= kFitResident;
-    const int G = fit.G, nseg = (fit.nsteps + G - 1) / G;
-    VMX_TRY(fit.ckpt.alloc((size_t)(fit.resident ? 1 : nseg) * sb));
-    VMX_TRY(fit.seg.alloc((size_t)(fit.keepP ? 2 * G + 1 : G + 1) * sb));
-    if (!fit.keepP) VMX_TRY(fit.P.alloc(sb));
+    // 0: the trajectory is kept; 1: checkpoints, a segment's predictor states kept; 2: checkpoints alone.
+    // The next form where there is no room for one.
+    int nseg = 0;
+    for (int form = all <= kFitResident ? 0 : 1;; ++form) {
+        fit.resident = form == 0;
+        fit.G = fit.resident ? Gr : std::min(fit.K, fit.nsteps);
+        fit.keepP = fit.resident || (form == 1 && 2 * (size_t)fit.G * sb <= kFitResident);
+        nseg = (fit.nsteps + fit.G - 1) / fit.G;
+        int rc = fit.resident ? fit.traj.alloc(all) : VMX_OK;
+        if (rc == VMX_OK) rc = fit.ckpt.alloc((size_t)(fit.resident ? 1 : nseg) * sb);
+        if (rc == VMX_OK) rc = fit.seg.alloc((size_t)(fit.keepP ? 2 * fit.G + 1 : fit.G + 1) * sb);
+        if (rc == VMX_OK && !fit.keepP) rc = fit.P.alloc(sb);
+        if (rc == VMX_OK) break;
+        if (form == 2) return rc;
+        (void)hipGetLastError();
+        fit.traj.release();
+        fit.seg.release();
+    }
+    const int G = fit.G;
     VMX_TRY(fit.h.alloc(sb));
     const int parts = std::max(1, std::min(kFitParts, n / 4096));
     VMX_TRY(fit.mz.alloc((size_t)parts * std::max(fit.nrec, 1) * sizeof(double)));
@@ -2125,13 +2145,24 @@ constexpr int kTileMaxSlots = 400000;
 // all (both forms give the same spins).
 int vmx_ctx::build_tiles(int64_t steps) {
     if (tiles_made) return VMX_OK;
-    const int W = zmax;
-    if (kernel != VMX_KERNEL_FUSED || tp == TP_CSR || (int64_t)n * W > kTileMaxSlots) {
+    if (kernel != VMX_KERNEL_FUSED || tp == TP_CSR || (int64_t)n * zmax > kTileMaxSlots) {
         tiles_made = true;
         return VMX_OK;
     }
     steps_before_tiles += steps;
     if (steps_before_tiles < n / 128) return VMX_OK;
+    tiles_made = true;
+    try {
+        const int rc = make_tiles();
+        if (rc != VMX_ERR_NOMEM) return rc;
+        (void)hipGetLastError();
+    } catch (const std::bad_alloc&) {
+    }
+    return VMX_OK;                               // no memory for the tiles: two kernels a step, as before
+}
+
+int vmx_ctx::make_tiles() {
+    const int W = zmax;
     const int B = n <= 12288 ? 128 : (n <= 40000 ? 192 : 256);
     struct Atom { int tile, mark, tried; };      // its tile, the last tile and the last attempt that met it
     std::vector<Atom> at(n, Atom{-1, -1, -1});
@@ -2203,7 +2234,6 @@ int vmx_ctx::build_tiles(int64_t steps) {
     VMX_HIP(precision == VMX_FP64 ? Ops<double>::tile_fill(stream, am(), sys<double>(), tile, (int)hdr.size())
                                   : Ops<float>::tile_fill(stream, am(), sys<float>(), tile, (int)hdr.size()));
     ntiles = (int)hdr.size();
-    tiles_made = true;
     drop_graph();                                // recorded from the two kernels
     return VMX_OK;
 }

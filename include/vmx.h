@@ -342,7 +342,8 @@ int vmx_last_step_time_ms(vmx_ctx* ctx, double* ms);
 /* Runs nsteps Heun steps (Philox noise) with HIP events around every kernel launch and returns
  * the average device time (ms) of each kernel of the step in `avg_ms` (fused: predictor,
  * corrector; plain: spin fields of S, external fields, predictor, spin fields of S', corrector)
- * and their number in `nkernels`.  `avg_ms` must hold 5 values. */
+ * and their number in `nkernels`.  `avg_ms` must hold 5 values.  The fused figures are always of the
+ * two-kernel form, also where steps of a small system run as one kernel. */
 int vmx_time_kernels(vmx_ctx* ctx, int32_t nsteps, double* avg_ms, int32_t* nkernels);
 
 /* ---- differentiation: deterministic trajectory and its adjoint ---------------------------- */

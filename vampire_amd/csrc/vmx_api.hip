@@ -2129,15 +2129,15 @@ static int build_topology(vmx_ctx* c, int request, const std::vector<int>& rowh,
 // followed by the next, so that tiles stay full.
 //
 // Where the line lies (us a step from a replayed graph, whole-step against two kernels, FP64 / FP32):
-//   SC   9^3 4.9/3.5 against 9.4/8.2    SC  33^3 8.6/5.9 against 9.9/8.3    SC  40^3 10.0/6.9 against 10.1/8.3
-//   BCC 16^3 5.7/4.1 against 10.2/8.9   BCC 28^3 9.5/7.0 against 10.8/9.0   BCC 32^3 12.8/10.6 against 10.9/8.8
-//   FCC 12^3 5.7/4.5 against 12.1/9.5   FCC 20^3 9.9/7.4 against 12.3/9.6   FCC 23^3 13.0/9.6 against 12.6/9.7
+//   SC   9^3 4.2/3.5 against 8.5/8.1    SC  33^3 7.9/5.9 against 9.0/8.4    SC  40^3  9.4/7.0  against 9.2/8.5
+//   BCC 16^3 4.9/4.1 against 9.4/9.0    BCC 28^3 9.2/7.1 against 10.0/9.1   BCC 32^3 12.2/10.7 against 10.1/9.0
+//   FCC 12^3 5.1/4.4 against 11.2/9.7   FCC 20^3 9.4/7.5 against 11.4/9.9   FCC 23^3 13.0/10.5 against 11.8/9.8
 // The whole step reads each item's record (slots of neighbour indices) and repeats the halo's
 // arithmetic, so the two meet at a number of slots, 400,000 = SC 40^3 = FCC 20^3.  CSR rows (no fixed
 // slot width) and the plain kernels keep their launches.
-// Items per tile: 128 where the tiles do not fill the CUs (SC 20^3 FP64 5.2 us; 256: 5.7), then larger
-// tiles, whose halo is smaller (SC 33^3 FP32: 128 5.9, 192 5.9, 256 6.3; FCC 20^3: 8.7, 7.4, 8.4;
-// SC 40^3: 8.0, 7.5, 6.9).
+// Items per tile: 128 where the tiles do not fill the CUs (SC 20^3 FP64 4.5 us; 256: 5.1), then larger
+// tiles, whose halo is smaller (SC 33^3 FP32: 128 6.0, 192 5.9, 256 6.4; FCC 20^3: 8.8, 7.5, 8.4;
+// SC 40^3: 8.1, 7.6, 7.0).
 constexpr int kTileMaxSlots = 400000;
 //
 // steps: the steps about to be taken.  Making the tiles takes the host 25-40 ns an atom, about n / 128

@@ -182,7 +182,7 @@ enum : uint32_t { STREAM_THERMAL = 0u, STREAM_MC_MOVE = 1u, STREAM_MC_ACCEPT = 2
 // FP64 Box-Muller for the uniforms that it meets, u = (k + 0.5) 2^-32 of a 32-bit word k, in place of the
 // general log, sqrt, sincos and cos.  Their instructions bound FP64 Metropolis sweeps and their latency the steps
 // of small systems: 92.1 -> 71.3 us a sweep (64 replicas, 2.7M SC atoms), 50.2 -> 44.8 us a Heun step of SC 96^3,
-// 2.56 -> 2.29 us one of SC 20^3.  No argument is zero, infinite, denormal or large, and u is exact in a double,
+// 5.12 -> 4.58 us one of SC 20^3.  No argument is zero, infinite, denormal or large, and u is exact in a double,
 // so there are no special cases to test for and no general reduction of the angle.  Largest relative errors over
 // 2e7 words (dense at both ends, at each power of two and around the quadrants) against 113 bits, hardware
 // estimates taken as good to 2^-22: radius 1.7e-16, as with a correctly rounded log and sqrt; sine and cosine
@@ -1194,7 +1194,7 @@ k_mid_corrector(SysDev<R> s, Spin3Alias<R> S, Spin3<R> P, Spin3Alias<R> O, Spin3
 // ======================= whole-step kernel: one launch per step for small systems ============
 // A system that leaves most of the chip idle is bound by its launches' dependent memory round trips,
 // not by its arithmetic: on SC 20^3 in FP64 the predictor and the corrector each took 4.75 us for 8000
-// atoms.  Here a workgroup owns a tile of atoms and forms the predicted spins of the tile and of its
+// atoms; a step in one launch takes 4.6.  Here a workgroup owns a tile of atoms and forms the predicted spins of the tile and of its
 // halo (every neighbour of a tile atom outside the tile) itself, one atom per thread, leaves them in
 // LDS, and corrects the tile's atoms from there: a step is one launch with two levels of global loads
 // (the item's record; the spins) instead of two launches with three each, and a tile atom's thermal

@@ -921,12 +921,8 @@ struct vmx_ctx {
     }
     // Conditions the device table does not hold yet (n = 0: none).
     CondArg cond_next{};
-    // hands them to a launch that writes them to the table
-    CondArg take_conditions() {
-        const CondArg a = cond_next;
-        cond_next.n = 0;
-        return a;
-    }
+    // a launch that carried them has been queued (one that failed leaves them for the next)
+    void conditions_carried() { cond_next.n = 0; }
     // writes them now, for launches that read the table
     int flush_conditions() {
         if (!cond_next.n) return VMX_OK;
@@ -1059,12 +1055,14 @@ int vmx_ctx::heun_steps(int nsteps, const double* noise, double* kernel_ms) {
         int nk = 0;
         if (kernel == VMX_KERNEL_FUSED && ntiles && !kernel_ms) {
             VMX_HIP(Ops<R>::tile_step(stream, et, jm, wsel, STEP_HEUN, s, tile, ntiles, spins<R>(s_idx), spins<R>(o_idx),
-                                      nd, off0 + (uint32_t)k, take_conditions()));
+                                      nd, off0 + (uint32_t)k, cond_next));
+            conditions_carried();
             std::swap(s_idx, o_idx);
         } else if (kernel == VMX_KERNEL_FUSED) {
             VMX_HIP(mark(0));
             VMX_HIP(Ops<R>::fused_predictor(Lf, et, am(), sf, spins<R>(s_idx), spins<R>(p_idx), euler<R>(),
-                                            field<R>(), nd, off0 + (uint32_t)k, take_conditions()));
+                                            field<R>(), nd, off0 + (uint32_t)k, cond_next));
+            conditions_carried();
             VMX_HIP(mark(1));
             const int out = corrector_in_place() ? s_idx : o_idx;
             VMX_HIP(Ops<R>::fused_corrector(L, et, am(), s, spins<R>(s_idx), spins<R>(p_idx), spins<R>(out),
@@ -1137,12 +1135,14 @@ int vmx_ctx::midpoint_steps(int nsteps, const double* noise) {
         }
         if (ntiles) {
             VMX_HIP(Ops<R>::tile_step(stream, et, jm, wsel, STEP_MIDPOINT, s, tile, ntiles, spins<R>(s_idx),
-                                      spins<R>(o_idx), nd, off0 + (uint32_t)k, take_conditions()));
+                                      spins<R>(o_idx), nd, off0 + (uint32_t)k, cond_next));
+            conditions_carried();
             std::swap(s_idx, o_idx);
         } else {
             const int p_idx = 3 - s_idx - o_idx;
             VMX_HIP(Ops<R>::mid_predictor(Lf, et, am(), sf, spins<R>(s_idx), spins<R>(p_idx), field<R>(), nd,
-                                          off0 + (uint32_t)k, take_conditions()));
+                                          off0 + (uint32_t)k, cond_next));
+            conditions_carried();
             // the midpoint corrector gathers only the midpoint: S_next overwrites S
             VMX_HIP(Ops<R>::mid_corrector(L, et, am(), s, spins<R>(s_idx), spins<R>(p_idx), spins<R>(s_idx), field<R>(),
                                           nd, off0 + (uint32_t)k));

@@ -31,3 +31,29 @@ def test_conditions_outlive_a_launch_that_failed(hip, kernel, argument, L):
             carried = [l.watched[0] for l in launches(log(lambda: c.llg_heun(2)), "{kernel}")]
             assert carried[0] > 0 and carried[1] == 0, carried
     """)
+
+
+@pytest.mark.parametrize("n", [200_000, 750_001])            # one worker, several
+@pytest.mark.parametrize("to_host", [True, False])
+@pytest.mark.parametrize("nth", [1, 2, 3])
+def test_a_transfer_that_failed_leaves_no_copy_in_flight(hip, n, to_host, nth):
+    """Copies still queued would write into the slots (or read from them) while the next transfer uses them."""
+    fake.run(hip, f"""
+        s = RC.isolated_spins({n})
+        with Context(s, precision=FP64, seed=1) as c:
+            sp = S.random_spins(s.n, 2)
+            c.set_spins(sp)
+
+            def fails():
+                hip.fake_fail_copy({nth})
+                try:
+                    c.get_spins() if {to_host} else c.set_spins(sp)
+                    assert 0, "the transfer was to fail"
+                except L.VmxError:
+                    pass
+            lines = log(fails)
+            queued = max(k for k, x in enumerate(lines) if x.startswith("copy"))
+            assert "wait stream" in lines[queued:], lines[-8:]
+            c.set_spins(sp)
+            assert c.get_spins().shape == sp.shape
+    """)

@@ -200,7 +200,10 @@ struct HostPipe {
         for (std::thread& t : more) t.join();
         for (int w = started; w < workers; ++w) work(w);
         for (int w = 0; w < workers; ++w)
-            if (err[w] != hipSuccess) return fail(VMX_ERR_HIP, "host transfer failed: %s", hipGetErrorString(err[w]));
+            if (err[w] != hipSuccess) {
+                (void)hipStreamSynchronize(st);  // copies still queued use the slots
+                return fail(VMX_ERR_HIP, "host transfer failed: %s", hipGetErrorString(err[w]));
+            }
         return VMX_OK;
     }
 };

@@ -30,6 +30,8 @@ int fail(int code, const char* fmt, ...) {
     vsnprintf(buf, sizeof buf, fmt, ap);
     va_end(ap);
     g_last_error = buf;
+    // the runtime keeps the error too, and the next launch's check would report it a second time
+    if (code == VMX_ERR_HIP || code == VMX_ERR_NOMEM) (void)hipGetLastError();
     return code;
 }
 
@@ -155,10 +157,7 @@ struct HostPipe {
                 total += chunks.back().bytes;
             }
         int workers = (int)std::min<size_t>(kWorkers, 1 + total / ((size_t)8 << 20));
-        if (ready(workers) != VMX_OK) {          // no pinned memory for more: the first one's slots are there
-            (void)hipGetLastError();
-            workers = 1;
-        }
+        if (ready(workers) != VMX_OK) workers = 1;   // no pinned memory for more: the first one's slots are there
         int dev = 0;
         VMX_HIP(hipGetDevice(&dev));
         hipError_t err[kWorkers] = {};
@@ -1748,7 +1747,6 @@ int vmx_ctx::fit_forward(const double* h, const double* spins0, double* mz_out) 
         if (rc == VMX_OK && !fit.keepP) rc = fit.P.alloc(sb);
         if (rc == VMX_OK) break;
         if (form == 2) return rc;
-        (void)hipGetLastError();
         fit.traj.release();
         fit.seg.release();
     }
@@ -2158,7 +2156,6 @@ int vmx_ctx::build_tiles(int64_t steps) {
     try {
         const int rc = make_tiles();
         if (rc != VMX_ERR_NOMEM) return rc;
-        (void)hipGetLastError();
     } catch (const std::bad_alloc&) {
     }
     return VMX_OK;                               // no memory for the tiles: two kernels a step, as before

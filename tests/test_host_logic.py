@@ -57,3 +57,17 @@ def test_a_transfer_that_failed_leaves_no_copy_in_flight(hip, n, to_host, nth):
             c.set_spins(sp)
             assert c.get_spins().shape == sp.shape
     """)
+
+
+def test_a_segment_of_many_records_is_summed_within_the_grid_limit(hip):
+    """A checkpoint distance of 100,000 steps with every step recorded: 100,000 records in one segment, and a
+    grid's second dimension holds 65,535."""
+    fake.run(hip, """
+        from vampire_amd.fit import Trajectory
+        s = S.ferromagnet("sc", 16)
+        steps = 100_000                                       # 19.7 GB of states: checkpoints
+        t = Trajectory(s, S.random_spins(s.n, 2), nsteps=steps, record_every=1, checkpoint_every=steps)
+        got = launches(log(lambda: t.forward(S.J_CO, S.KU_CO, 0.1)), "k_fit_mz")
+        assert sum(l.grid[1] for l in got) == steps and max(l.grid[1] for l in got) <= 65535, [l.grid for l in got]
+        t.close()
+    """)

@@ -71,3 +71,23 @@ def test_a_segment_of_many_records_is_summed_within_the_grid_limit(hip):
         assert sum(l.grid[1] for l in got) == steps and max(l.grid[1] for l in got) <= 65535, [l.grid for l in got]
         t.close()
     """)
+
+
+DIPOLE = """
+        def dipole(cells, n):
+            return dict(num_cells=cells, local_cell=np.arange(cells), atom_cell=np.arange(n) % cells,
+                        volume=np.ones(cells), tensor=np.zeros((6, cells, cells)), update_rate=1)
+"""
+
+
+def test_a_dipole_tensor_needs_its_own_memory_once(hip):
+    """Setting the dipole field takes the tensor in the device's layout and a small buffer beside it, not the
+    caller's layout whole as well."""
+    fake.run(hip, DIPOLE + """
+        s = RC.isolated_spins(2001)
+        cells = 1501
+        tensor = 6 * 8 * cells * cells
+        with Context(s, precision=FP64, seed=1) as c:
+            hip.fake_capacity(hip.fake_used() + tensor + tensor // 2)
+            c.set_dipole(**dipole(cells, s.n))
+    """)

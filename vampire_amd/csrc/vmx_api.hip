@@ -328,8 +328,9 @@ __global__ void __launch_bounds__(256) k_dip_cell_mag(int nc, const int* __restr
 }
 
 // The tensor as the field kernel reads it: for each tile of kDipRows local cells one stream
-// [source cell j][xx, xy, xz, yy, yz, zz][row], from the caller's [6][nl][nc]; rows past nl are zero.
+// [source cell j][xx, xy, xz, yy, yz, zz][row], from [6][nl][nc]; rows past nl are zero.
 constexpr int kDipRows = 4;
+constexpr size_t kDipSlabBytes = (size_t)32 << 20;   // of the caller's tensor on the device at a time
 __global__ void __launch_bounds__(256) k_dip_layout(int nl, int nc, const double* __restrict__ in, double* __restrict__ out) {
     const int j = (int)(blockIdx.x * blockDim.x + threadIdx.x), tile = (int)blockIdx.y;
     if (j >= nc) return;
@@ -3212,13 +3213,24 @@ int vmx_set_dipole(vmx_ctx* c, const vmx_dipole* d) {
     VMX_TRY(up(D.local_cell, d->local_cell, (size_t)nl * sizeof(int)));
     VMX_TRY(up(D.count, count.data(), (size_t)nc * sizeof(int)));
     VMX_TRY(up(D.volume, d->volume, (size_t)nc * sizeof(double)));
-    {
-        DevBuf given;
-        VMX_TRY(up(given, d->tensor, 6 * ts * sizeof(double)));
+    {   // laid out in slabs of rows, so that the caller's layout takes little memory beside the device's
         VMX_TRY(D.tensor.alloc((size_t)tiles * kDipRows * nc * 6 * sizeof(double)));
-        hipLaunchKernelGGL(k_dip_layout, dim3((nc + 255) / 256, tiles), dim3(256), 0, c->stream, nl, nc,
-                           given.as<double>(), D.tensor.as<double>());
-        VMX_HIP(hipGetLastError());
+        const size_t tile_reals = (size_t)6 * kDipRows * nc;
+        const int slab = (int)std::min<size_t>(tiles, std::max<size_t>(1, kDipSlabBytes / (tile_reals * sizeof(double))));
+        DevBuf given;
+        VMX_TRY(given.alloc((size_t)slab * tile_reals * sizeof(double)));
+        for (int t0 = 0; t0 < tiles; t0 += slab) {
+            const int l0 = t0 * kDipRows, rows = std::min(slab * kDipRows, nl - l0);
+            const size_t part = (size_t)rows * nc;
+            HostPipe::Seg seg[6];
+            for (int k = 0; k < 6; ++k)
+                seg[k] = HostPipe::Seg{const_cast<double*>(d->tensor) + k * ts + (size_t)l0 * nc,
+                                       given.as<double>() + k * part, part * sizeof(double)};
+            VMX_TRY(c->pipe.move(seg, 6, false, c->stream));
+            hipLaunchKernelGGL(k_dip_layout, dim3((nc + 255) / 256, (rows + kDipRows - 1) / kDipRows), dim3(256), 0,
+                               c->stream, rows, nc, given.as<double>(), D.tensor.as<double>() + (size_t)t0 * tile_reals);
+            VMX_HIP(hipGetLastError());
+        }
         VMX_HIP(hipStreamSynchronize(c->stream));
     }
     VMX_TRY(up(D.acell, acell.data(), (size_t)n * sizeof(int)));

@@ -91,3 +91,27 @@ def test_a_dipole_tensor_needs_its_own_memory_once(hip):
             hip.fake_capacity(hip.fake_used() + tensor + tensor // 2)
             c.set_dipole(**dipole(cells, s.n))
     """)
+
+
+def test_a_dipole_field_that_cannot_be_set_leaves_none(hip):
+    """The tables of an earlier field are overwritten one by one: when one finds no memory, no step may form a
+    field from the mixture."""
+    fake.run(hip, DIPOLE + """
+        s = RC.isolated_spins(2001)
+        with Context(s, precision=FP64, seed=1) as c:
+            c.set_conditions(0.0)
+            c.set_dipole(**dipole(11, s.n))
+            assert launches(log(lambda: c.llg_heun(1)), "k_dip_field")
+            hip.fake_capacity(hip.fake_used() + (4 << 20))
+            try:
+                c.set_dipole(**dipole(501, s.n))
+                assert 0, "there was to be no memory"
+            except L.VmxError as e:
+                assert e.code == L.VMX_ERR_NOMEM
+            assert not launches(log(lambda: c.llg_heun(1)), "k_dip")
+            try:
+                c.dipole_field()
+                assert 0, "no field is set"
+            except L.VmxError as e:
+                assert e.code == L.VMX_ERR_STATE
+    """)

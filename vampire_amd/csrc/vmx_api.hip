@@ -3208,6 +3208,8 @@ int vmx_set_dipole(vmx_ctx* c, const vmx_dipole* d) {
         return c->pipe.move(&seg, 1, false, c->stream);
     };
     vmx_ctx::Dipole& D = c->dip;
+    D.on = 0;                                       // should a table find no memory, no step reads the others
+    c->hdip_on = 0;
     VMX_TRY(up(D.start, start.data(), start.size() * sizeof(int)));
     VMX_TRY(up(D.atoms, atoms.data(), atoms.size() * sizeof(int)));
     VMX_TRY(up(D.local_cell, d->local_cell, (size_t)nl * sizeof(int)));

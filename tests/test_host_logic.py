@@ -115,3 +115,20 @@ def test_a_dipole_field_that_cannot_be_set_leaves_none(hip):
             except L.VmxError as e:
                 assert e.code == L.VMX_ERR_STATE
     """)
+
+
+@pytest.mark.parametrize("step", ["llg_heun", "llg_midpoint"])
+def test_only_rows_that_read_the_staged_exchange_table_stage_it(hip, step):
+    """The step kernels of ELL and stencil rows read exchange tables of up to 8 KiB from LDS; those of CSR rows
+    read the table itself and stage the material and condition records alone."""
+    fake.run(hip, f"""
+        s = S.config_c4(16, 16, 5)                    # a film of tensors, more atoms than make tiles at once
+        staged = {{}}
+        for topology in ("csr", "ell"):
+            with Context(s, precision=FP32, seed=1, topology=topology) as c:
+                assert c.topology[0] == topology
+                c.set_spins(S.random_spins(s.n, 2))
+                staged[topology] = sorted(set(l.shared for l in launches(log(lambda: c.{step}(1)), "tor")))
+        records, tensors = 4 * 2 * (18 + 12), 4 * 9 * 28     # of the two materials; the film's 28
+        assert staged == dict(csr=[records], ell=[records + tensors]), staged
+    """)

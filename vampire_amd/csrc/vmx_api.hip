@@ -749,8 +749,9 @@ struct vmx_ctx {
         // the whole staging area stays within 64 KiB
         s.pat_lds = (tp == TP_PAT && (size_t)npat * zmax * sizeof(int) <= 16384 &&
                      fused_lds_bytes<R>(nmat, npat, zmax, 1) <= 65536) ? 1 : 0;
-        // and an exchange table of up to 8 KiB, while the whole stays within 64 KiB
-        s.njt_lds = (jm == JM_IDX16 && (size_t)njt * K * sizeof(R) <= 8192 &&
+        // and an exchange table of up to 8 KiB, while the whole stays within 64 KiB (CSR rows read the
+        // table itself)
+        s.njt_lds = (jm == JM_IDX16 && tp != TP_CSR && (size_t)njt * K * sizeof(R) <= 8192 &&
                      fused_lds_bytes<R>(nmat, npat, zmax, s.pat_lds, (size_t)njt * K) <= 65536) ? njt : 0;
         s.am = am();
         s.q = q;

@@ -847,25 +847,36 @@ __device__ __forceinline__ void stage_fused(const SysDev<R>& s, int rep, const C
     const int* __restrict__ mat = reinterpret_cast<const int*>(s.mat);
     const int* __restrict__ cond = reinterpret_cast<const int*>(s.cond + rep * s.nmat);
     const int nm = s.nmat * L::kMatInts, nc = s.nmat * L::kCondInts;
-    const int np = (Access<AM>::TP == TP_PAT && s.pat_lds) ? s.npat * Access<AM>::W : 0;
-    const int nj = Access<AM>::JM == JM_IDX16 ? s.njt_lds * KJ * (int)(sizeof(R) / sizeof(int)) : 0;
+    constexpr bool kPat = Access<AM>::TP == TP_PAT, kTab = Access<AM>::JM == JM_IDX16 && Access<AM>::TP != TP_CSR && KJ > 0;
+    const int np = kPat && s.pat_lds ? s.npat * Access<AM>::W : 0;
+    const int nj = kTab ? s.njt_lds * KJ * (int)(sizeof(R) / sizeof(int)) : 0;
     const int* __restrict__ jt = reinterpret_cast<const int*>(s.jtab);
     const int rec = nm + nc, base = L::pat_off(s), jbase = L::jt_off(s), offs = rec + np, total = offs + nj;
     // one pass over the three tables with two loads in flight per thread: every wait for these
     // loads also waits for the own-data loads issued before, so fewer rounds mean fewer waits
     auto src = [&](int k) {
-        if (ca && ca->n && k >= nm && k < rec) return (int)ca->w[rep * nc + k - nm];
-        return k < nm ? mat[k] : (k < rec ? cond[k - nm] : (k < offs ? s.pat_off[k - rec] : jt[k - offs]));
+        if (kTab) return k < nm ? mat[k] : (k < rec ? cond[k - nm] : (!kPat || k >= offs ? jt[k - offs] : s.pat_off[k - rec]));
+        return k < nm ? mat[k] : (!kPat || k < rec ? cond[k - nm] : s.pat_off[k - rec]);
     };
-    auto dst = [&](int k) { return k < rec ? k : (k < offs ? base + (k - rec) : jbase + (k - offs)); };
+    auto dst = [&](int k) {
+        if (kTab) return k < rec ? k : (!kPat || k >= offs ? jbase + (k - offs) : base + (k - rec));
+        return !kPat || k < rec ? k : base + (k - rec);
+    };
     const int bd = (int)blockDim.x;
-    for (int k0 = (int)threadIdx.x; k0 < total; k0 += 2 * bd) {
-        const int k1 = k0 + bd;
-        const int v0 = src(k0);
-        const int v1 = k1 < total ? src(k1) : 0;
-        vmx_lds[dst(k0)] = v0;
-        if (k1 < total) vmx_lds[dst(k1)] = v1;
-    }
+    auto stage = [&](auto&& from) {
+        for (int k0 = (int)threadIdx.x; k0 < total; k0 += 2 * bd) {
+            const int k1 = k0 + bd;
+            const int v0 = from(k0);
+            const int v1 = k1 < total ? from(k1) : 0;
+            vmx_lds[dst(k0)] = v0;
+            if (k1 < total) vmx_lds[dst(k1)] = v1;
+        }
+    };
+    // a loop of its own for carried conditions: their branch within the other's cost every step 0.1 us
+    if (ca && ca->n)
+        stage([&](int k) { return k >= nm && k < rec ? (int)ca->w[rep * nc + k - nm] : src(k); });
+    else
+        stage(src);
     __syncthreads();
 }
 template <typename R, int AM>

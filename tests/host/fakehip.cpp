@@ -1,7 +1,7 @@
 // A HIP runtime that computes nothing, for tests of the library's host logic without a GPU: loaded with
 // its symbols global before libvmx.so, it serves the HIP calls that the library makes.  Device memory is
-// address space of the process (mapped when touched) up to a capacity, copies to and from the host are
-// made at once, kernels do nothing, and every call that a test may ask about is written to a log.  A test
+// address space of the process (mapped when touched) up to a capacity, copies stay within one allocation and
+// those to and from the host are made at once, kernels do nothing, and every call that a test may ask about is written to a log.  A test
 // sets the capacity and makes a launch or a copy fail.
 #include <stddef.h>
 #include <stdint.h>
@@ -51,9 +51,16 @@ int give(void* p) {
     blocks.erase(it);
     return kSuccess;
 }
+bool within_one_block(const void* p, size_t n) {
+    auto it = blocks.upper_bound(const_cast<void*>(p));
+    if (it == blocks.begin()) return false;
+    --it;
+    return (const char*)p + n <= (const char*)it->first + it->second;
+}
 int copy(void* d, const void* s, size_t n, int kind) {
     Lock l(mu);
     note("copy " + num(kind) + " " + num(n));
+    if ((kind != 2 && !within_one_block(d, n)) || (kind != 1 && !within_one_block(s, n))) return done(kInvalidValue);
     if (fail_copy_in > 0 && --fail_copy_in == 0) return done(kUnknown);
     if (kind != 3) memcpy(d, s, n);               // 1: to the device, 2: to the host; 3: within it, not made
     return kSuccess;

@@ -132,3 +132,38 @@ def test_only_rows_that_read_the_staged_exchange_table_stage_it(hip, step):
         records, tensors = 4 * 2 * (18 + 12), 4 * 9 * 28     # of the two materials; the film's 28
         assert staged == dict(csr=[records], ell=[records + tensors]), staged
     """)
+
+
+def test_small_arrays_cross_in_one_copy(hip):
+    """A copy on the link costs about 10 us whatever its size: the three components of a small system's spins or
+    fields share one, an array going to the device is not waited for, and a tensor of megabytes goes in chunks of
+    its own size, not of the system's."""
+    fake.run(hip, DIPOLE + """
+        s = RC.isolated_spins(1000)
+        with Context(s, precision=FP64, seed=1) as c:
+            sp = S.random_spins(s.n, 2)
+            c.set_spins(sp)
+            copies = lambda lines: [x for x in lines if x.startswith("copy")]
+            assert copies(log(c.get_spins)) == ["copy 2 24000"]
+            assert copies(log(c.fields)) == ["copy 2 24000"] * 2
+            lines = log(lambda: c.set_spins(sp))
+            assert copies(lines) == ["copy 1 24000"]
+            assert [x for x in lines if x.startswith("wait")] == ["wait 4", "wait stream"], lines   # the slot's last use
+            lines = log(lambda: c.set_dipole(**dipole(400, s.n)))
+            assert len(copies(lines)) < 60, len(copies(lines))
+            assert copies(log(c.dipole_field)) == ["copy 2 19200"]       # the cells' two fields
+    """)
+
+
+@pytest.mark.parametrize("n", [1, 2730, 2731, 10_923, 50_001, 130_000, 200_000, 750_001])
+def test_chunked_transfers_keep_every_value_in_its_place(hip, n):
+    """Lengths around one chunk (64 KiB), four and more, and several workers: what the runtime holds after the
+    copies is what the caller handed over (the kernels, which would permute, do nothing here)."""
+    fake.run(hip, f"""
+        s = RC.isolated_spins({n})
+        with Context(s, precision=FP64, seed=1) as c:
+            for k in range(3):
+                sp = np.random.default_rng(k).standard_normal((3, s.n))
+                c.set_spins(sp)
+                assert np.array_equal(c.get_spins(), sp)      # both go through the staging array
+    """)

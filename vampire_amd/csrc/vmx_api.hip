@@ -116,18 +116,23 @@ struct PinnedRing {
 
 // Transfers between device memory and the caller's ordinary (pageable) arrays, in chunks of at most
 // 1 MiB through pinned slots: a worker has one chunk on the link while it copies the other between its
-// slot and the caller's array.  Bound by the host side: one worker moves 25 GB/s into memory that is
+// slot and the caller's arrays.  Bound by the host side: one worker moves 25 GB/s into memory that is
 // mapped and 4.7 GB/s into fresh pages (each is faulted in), four 13 GB/s into fresh pages and 25 into
 // mapped ones; the link takes 56.  A pageable hipMemcpy of the same arrays runs at 4.2 GB/s (fresh) and
 // costs 0.4 ms at 1 MiB against 0.07.  So: a second worker for every 8 MiB, four at most (eight gain
 // another third at 64 MiB and cost more at 8).  The first worker's two slots are allocated with the
 // context, the others by the first transfer that uses them; all are freed with it.
+// A copy on the link costs about 10 us before its bytes, one behind another as well as alone, so segments
+// that lie side by side on the device share chunks (an array's three components) and a chunk is at least
+// 512 KiB, whose host side takes longer than that (8000 atoms' spins in one chunk 35 us, in four 73).
 struct HostPipe {
-    struct Seg { void* host; void* dev; size_t bytes; };
-    static constexpr size_t kChunk = (size_t)1 << 20;
+    // joined: lies in one allocation with the segment before it (a copy may span both)
+    struct Seg { void* host; void* dev; size_t bytes; bool joined = false; };
+    static constexpr size_t kChunk = (size_t)1 << 20, kSlot = (size_t)512 << 10;
     static constexpr int kWorkers = 4;
     void* slot[2 * kWorkers] = {};
     hipEvent_t done[2 * kWorkers] = {};
+    bool busy[2 * kWorkers] = {};  // a copy from the slot may still run: wait for done before filling it
     size_t bytes = 0;              // of a slot
     ~HostPipe() {
         for (int k = 0; k < 2 * kWorkers; ++k) {
@@ -142,52 +147,74 @@ struct HostPipe {
         }
         return VMX_OK;
     }
-    int init(size_t largest) {     // largest: the largest transfer expected
-        bytes = std::min(kChunk, std::max<size_t>(largest, 4096));
+    int init(size_t largest) {     // largest: the largest transfer expected often
+        bytes = (std::min(kChunk, std::max(largest, kSlot)) + 4095) & ~(size_t)4095;
         return ready(1);
     }
     // Moves every segment, after the work queued on st.  To the host: returns when the data has
     // arrived.  To the device: returns when the caller's arrays may be reused.
     int move(const Seg* seg, int nseg, bool to_host, hipStream_t st) {
-        std::vector<Seg> chunks;
+        struct Piece { char* host; size_t bytes; };
+        struct Chunk { char* dev; size_t bytes, first, count; };   // its pieces lie side by side on the device
+        std::vector<Piece> pieces;
+        std::vector<Chunk> chunks;
         size_t total = 0;
+        for (int k = 0; k < nseg; ++k) total += seg[k].bytes;
+        const size_t limit = std::min(bytes, std::max(kSlot, (total / 4 + 4095) & ~(size_t)4095));
         for (int k = 0; k < nseg; ++k)
-            for (size_t o = 0; o < seg[k].bytes; o += bytes) {
-                chunks.push_back(Seg{(char*)seg[k].host + o, (char*)seg[k].dev + o, std::min(bytes, seg[k].bytes - o)});
-                total += chunks.back().bytes;
+            for (size_t o = 0, b; o < seg[k].bytes; o += b) {
+                char* dev = (char*)seg[k].dev + o;
+                if (chunks.empty() || chunks.back().bytes == limit || (o == 0 && !seg[k].joined) ||
+                    chunks.back().dev + chunks.back().bytes != dev)
+                    chunks.push_back(Chunk{dev, 0, pieces.size(), 0});
+                Chunk& c = chunks.back();
+                b = std::min(limit - c.bytes, seg[k].bytes - o);
+                pieces.push_back(Piece{(char*)seg[k].host + o, b});
+                c.bytes += b;
+                ++c.count;
             }
+        if (chunks.empty()) return VMX_OK;
+        auto copy = [&](const Chunk& c, void* s) {
+            char* p = (char*)s;
+            for (size_t k = c.first; k < c.first + c.count; p += pieces[k].bytes, ++k)
+                to_host ? std::memcpy(pieces[k].host, p, pieces[k].bytes) : std::memcpy(p, pieces[k].host, pieces[k].bytes);
+        };
+        if (to_host && chunks.size() == 1) {     // nothing to overlap
+            VMX_HIP(hipMemcpyAsync(slot[0], chunks[0].dev, chunks[0].bytes, hipMemcpyDeviceToHost, st));
+            VMX_HIP(hipStreamSynchronize(st));
+            copy(chunks[0], slot[0]);
+            return VMX_OK;
+        }
         int workers = (int)std::min<size_t>(kWorkers, 1 + total / ((size_t)8 << 20));
         if (ready(workers) != VMX_OK) workers = 1;   // no pinned memory for more: the first one's slots are there
         int dev = 0;
-        VMX_HIP(hipGetDevice(&dev));
+        if (workers > 1) VMX_HIP(hipGetDevice(&dev));
         hipError_t err[kWorkers] = {};
         auto work = [&](int w) {
             if (w > 0 && (err[w] = hipSetDevice(dev)) != hipSuccess) return;
-            bool used[2] = {false, false};
-            auto wait = [&](int b) {
-                const hipError_t e = used[b] ? hipEventSynchronize(done[2 * w + b]) : hipSuccess;
-                if (err[w] == hipSuccess) err[w] = e;
+            auto wait = [&](int s) {
+                const hipError_t e = busy[s] ? hipEventSynchronize(done[s]) : hipSuccess;
+                if (e == hipSuccess) busy[s] = false;
+                else if (err[w] == hipSuccess) err[w] = e;
                 return e == hipSuccess;
             };
-            const Seg* last = nullptr;          // to the host: the chunk in flight in the other slot
-            int b = 0;
-            for (size_t k = (size_t)w; k < chunks.size() && err[w] == hipSuccess; k += (size_t)workers, b ^= 1) {
-                const Seg& c = chunks[k];
+            const Chunk* last = nullptr;        // to the host: the chunk in flight in the other slot
+            int s = 2 * w;
+            for (size_t k = (size_t)w; k < chunks.size() && err[w] == hipSuccess; k += (size_t)workers, s ^= 1) {
+                const Chunk& c = chunks[k];
                 if (!to_host) {
-                    if (!wait(b)) break;
-                    std::memcpy(slot[2 * w + b], c.host, c.bytes);
+                    if (!wait(s)) break;
+                    copy(c, slot[s]);
                 }
-                err[w] = to_host ? hipMemcpyAsync(slot[2 * w + b], c.dev, c.bytes, hipMemcpyDeviceToHost, st)
-                                 : hipMemcpyAsync(c.dev, slot[2 * w + b], c.bytes, hipMemcpyHostToDevice, st);
-                if (err[w] == hipSuccess) err[w] = hipEventRecord(done[2 * w + b], st);
+                err[w] = to_host ? hipMemcpyAsync(slot[s], c.dev, c.bytes, hipMemcpyDeviceToHost, st)
+                                 : hipMemcpyAsync(c.dev, slot[s], c.bytes, hipMemcpyHostToDevice, st);
+                if (err[w] == hipSuccess) err[w] = hipEventRecord(done[s], st);
                 if (err[w] != hipSuccess) break;
-                used[b] = true;
-                if (to_host && last && wait(b ^ 1)) std::memcpy(last->host, slot[2 * w + (b ^ 1)], last->bytes);
+                busy[s] = true;
+                if (to_host && last && wait(s ^ 1)) copy(*last, slot[s ^ 1]);
                 last = &c;
             }
-            if (to_host && last && err[w] == hipSuccess && wait(b ^ 1))
-                std::memcpy(last->host, slot[2 * w + (b ^ 1)], last->bytes);
-            if (!to_host) { (void)wait(0); (void)wait(1); }   // the slots are free again
+            if (to_host && last && err[w] == hipSuccess && wait(s ^ 1)) copy(*last, slot[s ^ 1]);
         };
         std::vector<std::thread> more;
         int started = 1;
@@ -200,7 +227,8 @@ struct HostPipe {
         for (int w = started; w < workers; ++w) work(w);
         for (int w = 0; w < workers; ++w)
             if (err[w] != hipSuccess) {
-                (void)hipStreamSynchronize(st);  // copies still queued use the slots
+                // copies still queued use the slots
+                if (hipStreamSynchronize(st) == hipSuccess) std::fill(std::begin(busy), std::end(busy), false);
                 return fail(VMX_ERR_HIP, "host transfer failed: %s", hipGetErrorString(err[w]));
             }
         return VMX_OK;
@@ -591,9 +619,17 @@ struct vmx_ctx {
         int nc = 0, nl = 0, rate = 1;
         long long time = 0;       // Heun steps and Metropolis sweeps since the field was set up
         DevBuf start, atoms;      // per cell: its magnetic atoms (internal index), ascending caller index
-        DevBuf local_cell, count, volume, tensor, mag, B, Hd, acell, amu;
+        DevBuf local_cell, count, volume, tensor, mag, acell, amu;
+        DevBuf field;             // [6][nc] doubles: B, then mu0 Hd
+        double* B() const { return field.as<double>(); }
+        double* Hd() const { return B() + 3 * (size_t)nc; }
         DevBuf hd_atom;           // [3][n] doubles, internal order: mu0 Hd for the energies
+        std::vector<int> acell_h; // caller's order, -1: no field (up to kDipHostAtoms atoms)
     } dip;
+    // Up to here the host spreads the cells' fields over the atoms' (a device copy of two small arrays: 1000
+    // atoms 40 us against 56 permuted by the device, 40,000 105 against 180, 200,000 391 against 440); beyond,
+    // the host's one thread fills pages more slowly than the transfer's four.
+    static constexpr int kDipHostAtoms = 262144;
     int hdip_on = 0;
     DevBuf hdip;
     void drop_graph() {
@@ -609,7 +645,7 @@ struct vmx_ctx {
         hipLaunchKernelGGL((k_dip_field<R>), dim3((dip.nl + kDipRows - 1) / kDipRows), dim3(512), 0, stream, n, dip.nl,
                            dip.nc, dip.local_cell.as<int>(), dip.count.as<int>(), dip.volume.as<double>(),
                            dip.mag.as<double>(), dip.tensor.as<double>(), dip.start.as<int>(), dip.atoms.as<int>(),
-                           dip.B.as<double>(), dip.Hd.as<double>(), hdip.as<R>(), dip.hd_atom.as<double>());
+                           dip.B(), dip.Hd(), hdip.as<R>(), dip.hd_atom.as<double>());
         VMX_HIP(hipGetLastError());
         return VMX_OK;
     }
@@ -677,7 +713,7 @@ struct vmx_ctx {
         double* st = staging.as<double>();
         VMX_HIP(Ops<R>::to_caller(launch(), sys<R>(), src, st));
         const size_t b = (size_t)n * sizeof(double);
-        const HostPipe::Seg seg[3] = {{x, st, b}, {y, st + n, b}, {z, st + 2 * (size_t)n, b}};
+        const HostPipe::Seg seg[3] = {{x, st, b}, {y, st + n, b, true}, {z, st + 2 * (size_t)n, b, true}};
         return pipe.move(seg, 3, true, stream);
     }
     template <typename R>
@@ -685,8 +721,8 @@ struct vmx_ctx {
         double* st = staging.as<double>();
         const size_t b = (size_t)n * sizeof(double);
         const HostPipe::Seg seg[3] = {{const_cast<double*>(x), st, b},
-                                      {const_cast<double*>(y), st + n, b},
-                                      {const_cast<double*>(z), st + 2 * (size_t)n, b}};
+                                      {const_cast<double*>(y), st + n, b, true},
+                                      {const_cast<double*>(z), st + 2 * (size_t)n, b, true}};
         VMX_TRY(pipe.move(seg, 3, false, stream));
         VMX_HIP(Ops<R>::from_caller(launch(), sys<R>(), st, dst));
         return VMX_OK;
@@ -2462,7 +2498,7 @@ int vmx_create(const vmx_system* sys, const vmx_options* opt, vmx_ctx** out) {
     const size_t cond_bytes = (size_t)nrep * c->nmat * sizeof(Cond<double>) + 64;
     // tables that fit a launch's arguments never use the ring
     if (cond_bytes > sizeof(ArgWords)) VMX_TRY(c->ring.init(std::max<size_t>(cond_bytes, 8 * (size_t)nrep + 64)));
-    VMX_TRY(c->pipe.init((size_t)n * sizeof(double)));
+    VMX_TRY(c->pipe.init(3 * (size_t)n * sizeof(double)));
     VMX_TRY(c->upload_conditions_any());
     // Monte Carlo state: adaptive sigma starts at 60 (src/montecarlo/data.cpp:46)
     VMX_TRY(c->mc_state.alloc(3 * (size_t)nrep * sizeof(double)));
@@ -3228,7 +3264,7 @@ int vmx_set_dipole(vmx_ctx* c, const vmx_dipole* d) {
             HostPipe::Seg seg[6];
             for (int k = 0; k < 6; ++k)
                 seg[k] = HostPipe::Seg{const_cast<double*>(d->tensor) + k * ts + (size_t)l0 * nc,
-                                       given.as<double>() + k * part, part * sizeof(double)};
+                                       given.as<double>() + k * part, part * sizeof(double), true};
             VMX_TRY(c->pipe.move(seg, 6, false, c->stream));
             hipLaunchKernelGGL(k_dip_layout, dim3((nc + 255) / 256, (rows + kDipRows - 1) / kDipRows), dim3(256), 0,
                                c->stream, rows, nc, given.as<double>(), D.tensor.as<double>() + (size_t)t0 * tile_reals);
@@ -3237,11 +3273,16 @@ int vmx_set_dipole(vmx_ctx* c, const vmx_dipole* d) {
         VMX_HIP(hipStreamSynchronize(c->stream));
     }
     VMX_TRY(up(D.acell, acell.data(), (size_t)n * sizeof(int)));
-    VMX_TRY(up(D.amu, amu.data(), amu.size() * sizeof(double)));
-    for (DevBuf* b : {&D.mag, &D.B, &D.Hd}) {
-        VMX_TRY(b->alloc(3 * (size_t)nc * sizeof(double)));
-        VMX_HIP(hipMemset(b->p, 0, 3 * (size_t)nc * sizeof(double)));
+    D.acell_h.clear();
+    if (n <= vmx_ctx::kDipHostAtoms) {
+        D.acell_h.resize(n);
+        for (int i = 0; i < n; ++i) D.acell_h[i] = acell[c->q > 1 ? c->pi[i] : i];
     }
+    VMX_TRY(up(D.amu, amu.data(), amu.size() * sizeof(double)));
+    VMX_TRY(D.mag.alloc(3 * (size_t)nc * sizeof(double)));
+    VMX_TRY(D.field.alloc(6 * (size_t)nc * sizeof(double)));
+    VMX_HIP(hipMemset(D.mag.p, 0, 3 * (size_t)nc * sizeof(double)));
+    VMX_HIP(hipMemset(D.field.p, 0, 6 * (size_t)nc * sizeof(double)));
     VMX_TRY(c->hdip.alloc(3 * (size_t)n * c->rsize()));
     VMX_HIP(hipMemset(c->hdip.p, 0, 3 * (size_t)n * c->rsize()));
     VMX_TRY(D.hd_atom.alloc(3 * (size_t)n * sizeof(double)));
@@ -3272,16 +3313,30 @@ int vmx_get_dipole_field(vmx_ctx* c, double* bx, double* by, double* bz, double*
     if (!c->dip.on) return fail(VMX_ERR_STATE, "no dipole field set (vmx_set_dipole)");
     VMX_TRY(c->use_device());
     double* out[6] = {bx, by, bz, hx, hy, hz};
-    const size_t n = (size_t)c->n;
+    const size_t n = (size_t)c->n, nc = (size_t)c->dip.nc;
+    if (c->n <= vmx_ctx::kDipHostAtoms) {
+        std::vector<double> cells(6 * nc);         // B, then mu0 Hd
+        const HostPipe::Seg seg{cells.data(), c->dip.field.p, 6 * nc * sizeof(double)};
+        VMX_TRY(c->pipe.move(&seg, 1, true, c->stream));
+        for (int k = 0; k < 6; ++k) {
+            if (!out[k]) continue;
+            const double* F = cells.data() + k * nc;
+            for (size_t i = 0; i < n; ++i) {
+                const int cell = c->dip.acell_h[i];
+                out[k][i] = cell < 0 ? 0.0 : F[cell];
+            }
+        }
+        return VMX_OK;
+    }
     double* st = c->staging.as<double>();
     for (int f = 0; f < 2; ++f) {                  // B, then mu0 Hd
         HostPipe::Seg seg[3];
         int k = 0;
         for (int x = 0; x < 3; ++x)
-            if (out[3 * f + x]) seg[k++] = HostPipe::Seg{out[3 * f + x], st + x * n, n * sizeof(double)};
+            if (out[3 * f + x]) seg[k++] = HostPipe::Seg{out[3 * f + x], st + x * n, n * sizeof(double), true};
         if (!k) continue;
         hipLaunchKernelGGL(k_dip_to_caller, dim3(c->launch().grid), dim3(c->block), 0, c->stream, c->sys<double>(),
-                           c->dip.nc, c->dip.acell.as<int>(), (f ? c->dip.Hd : c->dip.B).as<double>(), st);
+                           c->dip.nc, c->dip.acell.as<int>(), f ? c->dip.Hd() : c->dip.B(), st);
         VMX_HIP(hipGetLastError());
         VMX_TRY(c->pipe.move(seg, k, true, c->stream));
     }

@@ -167,3 +167,21 @@ def test_chunked_transfers_keep_every_value_in_its_place(hip, n):
                 c.set_spins(sp)
                 assert np.array_equal(c.get_spins(), sp)      # both go through the staging array
     """)
+
+
+def test_the_step_takes_the_form_it_reports(hip):
+    """tiles is what the next step uses, and two kernels kept means two kernels, eagerly and in a recording."""
+    fake.run(hip, """
+        s = S.ferromagnet("sc", 13)                           # tiles from the 17th step on
+        with Context(s, precision=FP64, seed=1) as c:
+            c.set_spins(S.random_spins(s.n, 2))
+            whole = lambda call: {l.name.startswith("k_tile_step") for l in launches(log(call))
+                                  if re.match("k_(tile_step|fused|mid)", l.name)}
+            assert c.tiles == 0 and whole(lambda: c.llg_heun(1)) == {False}
+            c.llg_heun(20)
+            assert c.tiles > 0
+            for run in (lambda: c.llg_heun(1), lambda: c.llg_midpoint(1), lambda: c.llg_heun_graph(2, 1)):
+                for on in (False, True):
+                    c.set_whole_step(on)
+                    assert (c.tiles > 0) == on and whole(run) == {on}
+    """)

@@ -139,6 +139,8 @@ SIGNATURES = [
     ("vmx_llg_heun", C.c_int, [_VP, C.c_int32, _DP]),
     ("vmx_llg_midpoint", C.c_int, [_VP, C.c_int32, _DP]),
     ("vmx_llg_heun_graph", C.c_int, [_VP, C.c_int32, C.c_int32]),
+    ("vmx_set_whole_step", C.c_int, [_VP, C.c_int32]),
+    ("vmx_get_whole_step", C.c_int, [_VP, _P(C.c_int32)]),
     ("vmx_get_step", C.c_int, [_VP, _P(C.c_int64)]),
     ("vmx_set_step", C.c_int, [_VP, C.c_int64]),
     ("vmx_get_sweep", C.c_int, [_VP, _P(C.c_int64)]),

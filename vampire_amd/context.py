@@ -186,6 +186,17 @@ class Context:
     def llg_heun_graph(self, nsteps: int, nrepeat: int) -> None:
         L.check(self.lib.vmx_llg_heun_graph(self.h, int(nsteps), int(nrepeat)))
 
+    @property
+    def tiles(self) -> int:
+        """Tiles of the whole-step kernel in use (0: a step takes two kernels)."""
+        v = C.c_int32(0)
+        L.check(self.lib.vmx_get_whole_step(self.h, C.byref(v)))
+        return int(v.value)
+
+    def set_whole_step(self, on: bool) -> None:
+        """False: steps take two kernels at every size; True (default): one where that is faster."""
+        L.check(self.lib.vmx_set_whole_step(self.h, int(bool(on))))
+
     def synchronize(self) -> None:
         L.check(self.lib.vmx_synchronize(self.h))
 

@@ -573,8 +573,10 @@ struct vmx_ctx {
     // can write S_next over S, and a step touches two spin arrays instead of three; the FP64
     // corrector that recomputes dS gathers S and cannot.
     bool corrector_in_place() const { return precision == VMX_FP32 || store_euler; }
-    // Tiles of the whole-step kernel (k_tile_step); ntiles == 0: the step takes two kernels.
+    // Tiles of the whole-step kernel (k_tile_step); none: the step takes two kernels.
     int ntiles = 0;
+    int whole_step = 1;           // 0: two kernels whether or not there are tiles
+    int tiles() const { return whole_step ? ntiles : 0; }
     bool tiles_made = false;      // or found to be out of question
     int64_t steps_before_tiles = 0;
     TileDev tile{};
@@ -1093,7 +1095,7 @@ int vmx_ctx::heun_steps(int nsteps, const double* noise, double* kernel_ms) {
         }
         const int p_idx = 3 - s_idx - o_idx;
         int nk = 0;
-        if (kernel == VMX_KERNEL_FUSED && ntiles && !kernel_ms) {
+        if (kernel == VMX_KERNEL_FUSED && tiles() && !kernel_ms) {
             VMX_HIP(Ops<R>::tile_step(stream, et, jm, wsel, STEP_HEUN, s, tile, ntiles, spins<R>(s_idx), spins<R>(o_idx),
                                       nd, off0 + (uint32_t)k, cond_next));
             conditions_carried();
@@ -1173,7 +1175,7 @@ int vmx_ctx::midpoint_steps(int nsteps, const double* noise) {
         } else if (normals64) {
             VMX_TRY(draw_fp64_normals(step + (uint64_t)k));
         }
-        if (ntiles) {
+        if (tiles()) {
             VMX_HIP(Ops<R>::tile_step(stream, et, jm, wsel, STEP_MIDPOINT, s, tile, ntiles, spins<R>(s_idx),
                                       spins<R>(o_idx), nd, off0 + (uint32_t)k, cond_next));
             conditions_carried();
@@ -1206,9 +1208,9 @@ int vmx_ctx::capture_graph(int nsteps) {
     int si = s_idx, oi = o_idx;
     for (int k = 0; k < nsteps; ++k) {
         const int pi = 3 - si - oi;
-        const int out = corrector_in_place() && !ntiles ? si : oi;
+        const int out = corrector_in_place() && !tiles() ? si : oi;
         hipError_t e;
-        if (ntiles) {
+        if (tiles()) {
             e = Ops<R>::tile_step(stream, et, jm, wsel, STEP_HEUN, s, tile, ntiles, spins<R>(si), spins<R>(out), nullptr,
                                   (uint32_t)k, CondArg{});
         } else {
@@ -2183,7 +2185,7 @@ constexpr int kTileMaxSlots = 400000;
 // steps' worth of what they save, so a context makes them when it has been asked for that many steps in
 // all (both forms give the same spins).
 int vmx_ctx::build_tiles(int64_t steps) {
-    if (tiles_made) return VMX_OK;
+    if (tiles_made || !whole_step) return VMX_OK;
     if (kernel != VMX_KERNEL_FUSED || tp == TP_CSR || (int64_t)n * zmax > kTileMaxSlots) {
         tiles_made = true;
         return VMX_OK;
@@ -2646,6 +2648,21 @@ int vmx_llg_heun_graph(vmx_ctx* c, int32_t nsteps, int32_t nrepeat) {
     c->timed_steps = nsteps * nrepeat;
     c->step += (uint64_t)nsteps * nrepeat;
     c->dev_step = c->step;
+    return VMX_OK;
+}
+
+int vmx_set_whole_step(vmx_ctx* c, int32_t on) {
+    g_last_error.clear();
+    if (!c) return fail(VMX_ERR_ARG, "null context");
+    if ((on != 0) != (c->whole_step != 0)) c->drop_graph();   // recorded from the other form
+    c->whole_step = on ? 1 : 0;
+    return VMX_OK;
+}
+
+int vmx_get_whole_step(vmx_ctx* c, int32_t* tiles) {
+    g_last_error.clear();
+    if (!c || !tiles) return fail(VMX_ERR_ARG, "null argument");
+    *tiles = c->tiles();
     return VMX_OK;
 }
 

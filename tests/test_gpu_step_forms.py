@@ -130,3 +130,22 @@ def test_switching_between_forms_drops_the_recorded_graph(gpu):
             c.llg_heun_graph(4, 2)
             d.llg_heun(8)
             assert np.array_equal(c.get_spins(), d.get_spins())
+
+
+@pytest.mark.parametrize("precision", [FP64, FP32])
+@pytest.mark.parametrize("before", [0, 40])
+def test_autotuning_leaves_the_run_as_it_was(gpu, precision, before):
+    """Before and after the tiles are made: spins, step counter and form stay, later steps give the same spins."""
+    s = S.ferromagnet("bcc", 13)                     # 4394 atoms: tiles from the 34th step on
+    sp = S.random_spins(s.n, 6)
+    with Context(s, precision=precision, seed=3) as c, TwoKernels(s, precision=precision, seed=3) as d:
+        for x in (c, d):
+            x.set_conditions(200.0, (0.0, 0.1, 0.2))
+            x.set_spins(sp)
+            x.llg_heun(before)
+        tiles = c.tiles
+        assert c.autotune(12) in (64, 128, 256, 512)
+        assert c.tiles == tiles and c.step == before and np.array_equal(c.get_spins(), d.get_spins())
+        for x in (c, d):
+            x.llg_heun(50)
+        assert c.tiles > 0 and np.array_equal(c.get_spins(), d.get_spins())

@@ -185,3 +185,27 @@ def test_the_step_takes_the_form_it_reports(hip):
                     c.set_whole_step(on)
                     assert (c.tiles > 0) == on and whole(run) == {on}
     """)
+
+
+def test_autotuning_times_the_launch_shape_it_chooses(hip):
+    """The workgroup size and remapping shape the two kernels, not the whole-step kernel: every trial is of the
+    two, and the trials are not counted towards the tiles."""
+    fake.run(hip, """
+        s = S.ferromagnet("sc", 13)                           # tiles from the 17th step on
+        for made in (False, True):
+            with Context(s, precision=FP64, seed=1) as c:
+                c.set_spins(S.random_spins(s.n, 2))
+                if made:
+                    c.llg_heun(20)
+                tiles = c.tiles
+                assert (tiles > 0) == made
+                lines = log(lambda: c.autotune(10))
+                assert not launches(lines, "k_tile"), launches(lines, "k_tile")[0].name
+                shapes = {(l.grid[0], l.block) for l in launches(lines, "k_fused_corrector")}
+                assert len(shapes) == 8 or len({b for _, b in shapes}) == 4, shapes
+                assert c.tiles == tiles
+                c.llg_heun(16)
+                assert (c.tiles > 0) == made
+                c.llg_heun(1)
+                assert c.tiles > 0
+    """)

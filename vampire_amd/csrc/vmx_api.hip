@@ -3163,6 +3163,14 @@ int vmx_autotune(vmx_ctx* c, int32_t steps_per_trial, int32_t* chosen) {
         ~PauseDipole() { c->dip.on = on; }
     } pause{c, c->dip.on};
     c->dip.on = 0;
+    // and they are of the two kernels, whose launches the choice shapes: the whole-step kernel's are not,
+    // and its tiles would appear between one trial and the next
+    struct TwoKernels {
+        vmx_ctx* c;
+        int on;
+        ~TwoKernels() { c->whole_step = on; }
+    } two{c, c->whole_step};
+    c->whole_step = 0;
     // save spins and step counter
     const size_t bytes = 3 * (size_t)c->n * c->rsize();
     DevBuf save;

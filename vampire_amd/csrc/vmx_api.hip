@@ -562,7 +562,7 @@ struct vmx_ctx {
     }
 
     // device state
-    DevBuf row, col, jidx, jtab, type, mat, cond, blk, blk_fused, rep_off, rep_key, step_base;
+    DevBuf row, col, jidx, jtab, type, mat, cond, blk, blk_fused, blk_energy, rep_off, rep_key, step_base;
     std::vector<uint2> rep_key_h;    // the replicas' Philox keys (seed + r)
     DevBuf deg, pat, pat_off, pat_jid, pat_deg;
     DevBuf rep_m;                 // [nrep] replica size / q
@@ -611,6 +611,7 @@ struct vmx_ctx {
     DevBuf partial;               // statistics partial sums
     int nblocks = 0;
     int nblocks_fused = 0;        // entries of blk_fused (each FusedAtoms * block atoms)
+    int nblocks_energy = 0;       // entries of blk_energy (each kEnergySpan atoms)
     std::vector<MagStat*> mags;
     std::vector<EnergyStat*> energies;
 
@@ -1268,10 +1269,12 @@ int vmx_ctx::stats_update(double* fixed) {
         VMX_HIP(Ops<R>::magnetization(grid, stream, n, S, st->mask.as<int>(), moments(), st->nbins, part, st->out()));
     }
     if (!energies.empty()) {
-        const SysDev<R> s = sys<R>();
+        SysDev<R> s = sys<R>();
+        s.blk = blk_energy.as<int4>();
+        s.nblocks = nblocks_energy;
         for (EnergyStat* st : energies) {
             const int grid = stats_grid(st->nbins);
-            VMX_HIP(Ops<R>::energy(grid, stream, et, am(), s, (block + 63) / 64, S, st->mask.as<int>(), moments(), st->nbins, part,
+            VMX_HIP(Ops<R>::energy(grid, stream, et, am(), s, S, st->mask.as<int>(), moments(), st->nbins, part,
                                    st->out()));
         }
     }
@@ -2486,6 +2489,11 @@ int vmx_create(const vmx_system* sys, const vmx_options* opt, vmx_ctx** out) {
     if (c->precision == VMX_FP64) VMX_TRY(c->upload_materials<double>());
     else VMX_TRY(c->upload_materials<float>());
     VMX_TRY(c->build_blocks());
+    {
+        const std::vector<int4> tab = vmx_ctx::block_table(nrep, roff, q, kEnergySpan);
+        VMX_TRY(upload(c->blk_energy, tab));
+        c->nblocks_energy = (int)tab.size();
+    }
     for (int b = 0; b < 3; ++b) {
         VMX_TRY(c->spin[b].alloc(3 * (size_t)n * rs));
         VMX_HIP(hipMemset(c->spin[b].p, 0, 3 * (size_t)n * rs));

@@ -1804,13 +1804,16 @@ __device__ __forceinline__ R magnetostatic_energy(const SysDev<R>& s, int i, R s
 }
 
 // W = 4: exchange, anisotropy, applied, magnetostatic, each times m_i (energy.cpp:155-203); the
-// last is zero without a device dipole field.  A workgroup takes a contiguous run of the block table's
-// 64-atom units (units per entry; with XCD remapping, of its XCD's stretch), a wavefront a unit, so the rows it gathers lie in its own L2, the replica and its
-// conditions come with the entry, and the stencil offsets are staged in LDS.  Bound by the gathers, like a
-// step's field (FP32: 4M FCC atoms 67 -> 56 us, 472,014-atom film 26.5 -> 22.7; FP64 1M FCC 42.8 -> 36.7).
+// last is zero without a device dipole field.  A workgroup takes a contiguous run of the 64-atom units of
+// its own block table (of kEnergySpan atoms an entry, whatever the step kernels' workgroups), of its XCD's
+// stretch, a wavefront a unit, so the rows it gathers lie in its own L2, the replica and its conditions come
+// with the entry, and the stencil offsets are staged in LDS.  The order of additions depends on the system
+// alone.  Bound by the gathers, like a step's field (FP32: 4M FCC atoms 67 -> 56 us, 472,014-atom film
+// 26.5 -> 22.7; FP64 1M FCC 42.8 -> 36.7).
+constexpr int kEnergySpan = 256;
 template <typename R, int ET, int AM>
 __global__ void __launch_bounds__(256)
-k_energy(SysDev<R> s, int units, Spin3<R> S, const int* __restrict__ mask, Moments mo, int nbins,
+k_energy(SysDev<R> s, Spin3<R> S, const int* __restrict__ mask, Moments mo, int nbins,
          double* __restrict__ partial) {
     constexpr int TP = Access<AM>::TP, W = Access<AM>::W;
     const bool few = nbins <= 4;     // few bins: register histograms, as k_mag_regs
@@ -1826,8 +1829,8 @@ k_energy(SysDev<R> s, int units, Spin3<R> S, const int* __restrict__ mask, Momen
     for (int b = 0; b < 4; ++b) { acc[b][0] = 0.0; acc[b][1] = 0.0; acc[b][2] = 0.0; acc[b][3] = 0.0; }
     const UniformJ<R, ET> ju(s, Access<AM>::JM);
     const SpinRsrc<R> rs(s, S.x, S.y, S.z);
-    const bool remap = s.xcd_remap && (gridDim.x & 7) == 0;
-    const long long lb = logical_block(remap ? 1 : 0);
+    constexpr int units = kEnergySpan / 64;
+    const long long lb = logical_block((gridDim.x & 7) == 0 ? 1 : 0);
     const long long all = (long long)s.nblocks * units;
     const long long u0 = lb * all / gridDim.x, u1 = (lb + 1) * all / gridDim.x;
     int cur = -1;

@@ -54,9 +54,9 @@ struct Ops {
     // statistics: partial sums (`grid` workgroups of 256), then the result by a launch of one workgroup
     static hipError_t magnetization(int grid, hipStream_t st, int n, Spin3<R> S, const int* mask, Moments mo, int nbins,
                                     double* partial, const StatOut& out);
-    // units: 64-atom units of a block table entry
-    static hipError_t energy(int grid, hipStream_t st, int et, int jm, const SysDev<R>& s, int units, Spin3<R> S,
-                             const int* mask, Moments mo, int nbins, double* partial, const StatOut& out);
+    // s: with the energies' block table (kEnergySpan)
+    static hipError_t energy(int grid, hipStream_t st, int et, int jm, const SysDev<R>& s, Spin3<R> S, const int* mask,
+                             Moments mo, int nbins, double* partial, const StatOut& out);
     // Monte Carlo: one launch of a sweep, workgroups wg0 .. wg0 + nwg - 1; workgroup w takes
     // entries [w * 256 * McAtoms, ...) of atom (and pat, the stencil ids) and wg[w] = {replica,
     // replica's first atom}

@@ -367,8 +367,10 @@ typedef struct vmx_fit_params {
 } vmx_fit_params;
 
 /* Runs nsteps steps from spins0 [3][N] and writes <m_z> after every record_every steps to
- * mz [nsteps/record_every].  While the predicted and corrected spins of every step fit 8 GiB of
- * device memory, all are kept for the adjoint; else a checkpoint every checkpoint_every steps.
+ * mz [nsteps/record_every].  While the predicted and corrected spins of every step are within the
+ * context's limit (vmx_fit_set_resident) and find memory, all are kept for the adjoint; else a
+ * checkpoint every checkpoint_every steps.  The kept ones stay with the context until a forward pass
+ * that keeps none, or vmx_destroy.
  * h: per-site field [3][N] or NULL.  nsteps must be a multiple of record_every. */
 int vmx_fit_forward(vmx_ctx* ctx, const vmx_fit_params* p, const double* h, const double* spins0,
                     int32_t nsteps, int32_t record_every, int32_t checkpoint_every, double* mz);
@@ -377,6 +379,16 @@ int vmx_fit_forward(vmx_ctx* ctx, const vmx_fit_params* p, const double* h, cons
  * grad = {dL/dJ, dL/dku2, dL/dalpha} and, if dL_dh is not NULL, dL/dh_i [3][N].  The steps are swept backward
  * over the kept trajectory, or over segments recomputed from the checkpoints (hand-written adjoint kernels). */
 int vmx_fit_backward(vmx_ctx* ctx, const double* dL_dmz, double* grad, double* dL_dh);
+
+/* Bytes of states a forward pass may keep beyond its checkpoints, 8 GiB if never set (2 nsteps
+ * states of 3 num_atoms reals for the whole trajectory).  Less memory, the same results: a limit
+ * that holds the 2 checkpoint_every states of a segment keeps those while it steps back over it,
+ * 0 keeps checkpoints alone.  Applies from the next forward pass on. */
+int vmx_fit_set_resident(vmx_ctx* ctx, uint64_t bytes);
+
+/* What the last forward pass kept: 0 the trajectory, 1 checkpoints and a segment's predicted
+ * spins, 2 checkpoints alone; -1 without a forward pass. */
+int vmx_fit_get_form(vmx_ctx* ctx, int32_t* form);
 
 /* Chooses the workgroup size (64, 128, 256, 512) and whether workgroups are remapped to give
  * each XCD one contiguous stretch of the system, by timing a few Heun steps of each candidate

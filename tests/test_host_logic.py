@@ -209,3 +209,66 @@ def test_autotuning_times_the_launch_shape_it_chooses(hip):
                 c.llg_heun(1)
                 assert c.tiles > 0
     """)
+
+
+FIT = """
+        from vampire_amd.fit import Trajectory
+        s = S.ferromagnet("sc", 16)                           # 4096 atoms, 98,304 bytes a state
+        state = 24 * s.n
+        sp = S.random_spins(s.n, 2)
+        traj = lambda **kw: Trajectory(s, sp, nsteps=1000, record_every=10, checkpoint_every=100, **kw)
+        both = lambda t: (t.forward(S.J_CO, S.KU_CO, 0.1), t.backward(np.ones(100)))
+        memory = lambda lines: [x for x in lines if x.startswith(("malloc", "free", "capture"))]
+"""
+
+
+def test_the_kept_trajectory_leaves_room_for_the_backward_pass(hip):
+    """Where the trajectory alone would fit and the working arrays of the backward pass would not beside it,
+    checkpoints are taken: both passes run."""
+    fake.run(hip, FIT + """
+        for spare in (105, 108, 112, 130):                    # segments and small arrays take 103 states
+            t = traj()
+            hip.fake_capacity(hip.fake_used() + (2000 + spare) * state)
+            both(t)
+            print(spare, t.form)
+            t.close()
+    """)
+
+
+def test_a_form_that_found_no_memory_is_not_tried_again(hip):
+    """Each try would free and allocate the segment, and so record both passes anew."""
+    fake.run(hip, FIT + """
+        t = traj()
+        hip.fake_capacity(hip.fake_used() + 600 * state)
+        both(t)
+        assert t.form == 1
+        both(t)
+        assert memory(log(lambda: both(t))) == []
+        hip.fake_capacity(288 << 30)
+        assert memory(log(lambda: both(t))) == [] and t.form == 1
+        L.check(t.ctx.lib.vmx_fit_set_resident(t.ctx.h, 8 << 30))      # asked again
+        both(t)
+        assert t.form == 0
+    """)
+
+
+def test_checkpoints_bound_the_memory_when_asked_to(hip):
+    fake.run(hip, FIT + """
+        used = hip.fake_used()
+        t = traj(resident_bytes=0)
+        base = hip.fake_used() - used
+        both(t)
+        assert t.form == 2
+        states = (hip.fake_used() - used - base) / state      # 10 checkpoints, 101 of a segment, 11 arrays
+        assert states < 125, states
+        L.check(t.ctx.lib.vmx_fit_set_resident(t.ctx.h, 200 * state))
+        both(t)
+        assert t.form == 1
+        L.check(t.ctx.lib.vmx_fit_set_resident(t.ctx.h, 2000 * state))
+        both(t)
+        assert t.form == 0
+        kept = hip.fake_used()
+        L.check(t.ctx.lib.vmx_fit_set_resident(t.ctx.h, 2000 * state - 1))
+        both(t)
+        assert t.form == 1 and hip.fake_used() <= kept - 2000 * state, (hip.fake_used(), kept)
+    """)

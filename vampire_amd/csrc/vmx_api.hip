@@ -1008,18 +1008,23 @@ struct vmx_ctx {
     int colour();
 
     // Deterministic fitting trajectory and its adjoint.  A segment of G steps lies in `seg`: states
-    // S_0 .. S_G, then (keepP) the predicted P_0 .. P_{G-1}.  While every S and P of the trajectory fits
-    // kFitResident, they are kept (traj: per segment S_1 .. S_G, P_0 .. P_{G-1}) and the backward pass
-    // recomputes nothing; else the forward pass keeps a checkpoint every K steps and the backward pass
-    // recomputes a segment of K before it steps back over it.  Segments of equal length replay graphs
-    // whose kernels read the parameters from device memory, so one recording serves every call until a
-    // buffer moves.
+    // S_0 .. S_G, then (keepP) the predicted P_0 .. P_{G-1}.  Three forms, the first whose kept bytes are
+    // within the limit and find memory (the working arrays of the backward pass are made before them):
+    //   0  every S and P is kept (traj: per segment S_1 .. S_G, P_0 .. P_{G-1}), nothing is recomputed;
+    //   1  a checkpoint every K steps, and a segment of K recomputed with its P before the steps back over it;
+    //   2  as 1 without the P, which each step back forms once more.
+    // Segments of equal length replay graphs whose kernels read the parameters from device memory, so one
+    // recording serves every call until a buffer moves.
+    static constexpr size_t kFitResident = (size_t)8 << 30;   // bytes: 3 % of this device's memory
     struct Fit {
         bool ready = false;
         int nsteps = 0, record_every = 1, K = 100, nrec = 0;
         double J = 0, k = 0, alpha = 0, gamma_rel = 1, H[3] = {0, 0, 0};
         bool has_h = false;
+        int form = -1;            // of the last forward pass
         bool resident = false, keepP = false;
+        size_t limit = kFitResident;
+        size_t refused[2] = {SIZE_MAX, SIZE_MAX};   // kept bytes for which forms 0 and 1 found no memory
         int G = 1;                // steps of a full segment
         DevBuf prm, traj, ckpt, seg, P, lH1, lPd, lT, H0, sumS, lH0, lSp, dh, nhat, h, acc, mz;
         // backward: dL/dm_z injections per step (inj[q], zero between records) and the slice of the
@@ -1041,12 +1046,14 @@ struct vmx_ctx {
     } fit;
     template <typename F>
     int fit_replay(Fit::Replay& r, const std::vector<const void*>& key, F&& record);
-    static constexpr size_t kFitResident = (size_t)8 << 30;   // bytes: 3 % of this device's memory
     static constexpr int kFitSegment = 50;                    // steps of a recorded segment
     static constexpr int kFitParts = 8;                       // partial sums of a recorded state's S_z
+    int fit_waves() const { return (n + 255) / 256 * 4; }     // of the backward kernels: one slot of 4 sums each
     bool symmetric_checked = false, symmetric = false;
     template <typename R>
     FitPrm<R> fit_prm() const;
+    template <typename R>
+    int fit_backward_buffers();
     template <typename R>
     int fit_forward(const double* h, const double* spins0, double* mz_out);
     template <typename R>
@@ -1769,6 +1776,17 @@ int vmx_ctx::fit_replay(Fit::Replay& r, const std::vector<const void*>& key, F&&
     return VMX_OK;
 }
 
+// The backward pass's own arrays, for the steps and the segment length of the last forward pass.
+template <typename R>
+int vmx_ctx::fit_backward_buffers() {
+    for (DevBuf* b : {&fit.lH1, &fit.lPd, &fit.lT, &fit.H0, &fit.sumS, &fit.lH0, &fit.lSp, &fit.dh})
+        VMX_TRY(b->alloc(3 * (size_t)n * sizeof(R)));
+    VMX_TRY(fit.nhat.alloc((size_t)n * sizeof(R)));
+    VMX_TRY(fit.acc.alloc((size_t)4 * fit_waves() * sizeof(double)));
+    VMX_TRY(fit.inj.alloc((size_t)fit.nsteps * sizeof(R)));
+    return fit.inj_seg.alloc((size_t)fit.G * sizeof(R));
+}
+
 template <typename R>
 int vmx_ctx::fit_forward(const double* h, const double* spins0, double* mz_out) {
     const size_t N3 = 3 * (size_t)n, sb = N3 * sizeof(R);   // reals and bytes of a state
@@ -1776,28 +1794,33 @@ int vmx_ctx::fit_forward(const double* h, const double* spins0, double* mz_out) 
     VMX_HIP(hipStreamSynchronize(stream));         // a buffer that grows is freed: nothing may use it
     const int Gr = std::min(fit.nsteps, kFitSegment);
     const size_t all = 2 * (size_t)((fit.nsteps + Gr - 1) / Gr) * Gr * sb;
-    // 0: the trajectory is kept; 1: checkpoints, a segment's predictor states kept; 2: checkpoints alone.
-    // The next form where there is no room for one.
-    int nseg = 0;
-    for (int form = all <= kFitResident ? 0 : 1;; ++form) {
-        fit.resident = form == 0;
-        fit.G = fit.resident ? Gr : std::min(fit.K, fit.nsteps);
-        fit.keepP = fit.resident || (form == 1 && 2 * (size_t)fit.G * sb <= kFitResident);
-        nseg = (fit.nsteps + fit.G - 1) / fit.G;
-        int rc = fit.resident ? fit.traj.alloc(all) : VMX_OK;
-        if (rc == VMX_OK) rc = fit.ckpt.alloc((size_t)(fit.resident ? 1 : nseg) * sb);
-        if (rc == VMX_OK) rc = fit.seg.alloc((size_t)(fit.keepP ? 2 * fit.G + 1 : fit.G + 1) * sb);
-        if (rc == VMX_OK && !fit.keepP) rc = fit.P.alloc(sb);
-        if (rc == VMX_OK) break;
-        if (form == 2) return rc;
-        fit.traj.release();
-        fit.seg.release();
-    }
-    const int G = fit.G;
     VMX_TRY(fit.h.alloc(sb));
     const int parts = std::max(1, std::min(kFitParts, n / 4096));
     VMX_TRY(fit.mz.alloc((size_t)parts * std::max(fit.nrec, 1) * sizeof(double)));
     VMX_TRY(fit.prm.alloc(sizeof(FitPrm<R>)));
+    int nseg = 0;
+    for (int form = 0;; ++form) {
+        fit.form = form;
+        fit.resident = form == 0;
+        fit.keepP = form < 2;
+        fit.G = fit.resident ? Gr : std::min(fit.K, fit.nsteps);
+        nseg = (fit.nsteps + fit.G - 1) / fit.G;
+        const size_t kept = form == 0 ? all : 2 * (size_t)fit.G * sb;
+        if (form < 2 && (kept > fit.limit || kept >= fit.refused[form])) continue;
+        if (!fit.resident || fit.traj.bytes > fit.limit) fit.traj.release();
+        int rc = form < 2 ? fit_backward_buffers<R>() : VMX_OK;
+        if (rc == VMX_OK) rc = fit.ckpt.alloc((size_t)(fit.resident ? 1 : nseg) * sb);
+        if (rc == VMX_OK) rc = fit.seg.alloc((size_t)(fit.keepP ? 2 * fit.G + 1 : fit.G + 1) * sb);
+        if (rc == VMX_OK && fit.resident) rc = fit.traj.alloc(all);
+        if (rc == VMX_OK && !fit.keepP) rc = fit.P.alloc(sb);
+        if (rc == VMX_OK) break;
+        if (form == 2 || rc != VMX_ERR_NOMEM) return rc;
+        fit.refused[form] = kept;                  // the next form has all the memory, and later passes begin with it
+        for (DevBuf* b : {&fit.traj, &fit.seg, &fit.lH1, &fit.lPd, &fit.lT, &fit.H0, &fit.sumS, &fit.lH0, &fit.lSp,
+                          &fit.dh, &fit.nhat})
+            b->release();
+    }
+    const int G = fit.G;
     fit.has_h = h != nullptr;
     R* ck = fit.ckpt.as<R>();
     R* seg = fit.seg.as<R>();
@@ -1855,11 +1878,8 @@ template <typename R>
 int vmx_ctx::fit_backward(const double* dmz, double* grad, double* dh_out) {
     const size_t N3 = 3 * (size_t)n, sb = N3 * sizeof(R);
     const int G = fit.G, nseg = (fit.nsteps + G - 1) / G;
-    for (DevBuf* b : {&fit.lH1, &fit.lPd, &fit.lT, &fit.H0, &fit.sumS, &fit.lH0, &fit.lSp, &fit.dh})
-        VMX_TRY(b->alloc(sb));
-    VMX_TRY(fit.nhat.alloc((size_t)n * sizeof(R)));
-    const int nwave = (n + 255) / 256 * 4;   // wavefronts of the backward kernels: one slot of 4 sums each
-    VMX_TRY(fit.acc.alloc((size_t)4 * nwave * sizeof(double)));
+    VMX_TRY(fit_backward_buffers<R>());
+    const int nwave = fit_waves();
     const SysDev<R> s = sys<R>();
     const Spin3<R> hh = fit.has_h ? arr3<R>(fit.h) : Spin3<R>{nullptr, nullptr, nullptr};
     const FitPrm<R>* pp = fit.prm.as<FitPrm<R>>();
@@ -1881,10 +1901,8 @@ int vmx_ctx::fit_backward(const double* dmz, double* grad, double* dh_out) {
         std::vector<R> inj((size_t)fit.nsteps, R(0));
         for (int q = 0; q < fit.nsteps; ++q)
             if ((q + 1) % fit.record_every == 0) inj[q] = (R)(dmz[(q + 1) / fit.record_every - 1] / n);
-        VMX_TRY(fit.inj.alloc(inj.size() * sizeof(R)));
         const HostPipe::Seg is{inj.data(), fit.inj.p, inj.size() * sizeof(R)};
         VMX_TRY(pipe.move(&is, 1, false, stream));
-        VMX_TRY(fit.inj_seg.alloc((size_t)G * sizeof(R)));
     }
     // One segment: its states recomputed from the checkpoint in seg[0] unless the trajectory was kept,
     // then the steps back over them.  inj: the segment's injections (inj[t] after local step t).
@@ -3149,6 +3167,21 @@ int vmx_fit_backward(vmx_ctx* c, const double* dL_dmz, double* grad, double* dL_
     VMX_TRY(c->use_device());
     return c->precision == VMX_FP64 ? c->fit_backward<double>(dL_dmz, grad, dL_dh)
                                     : c->fit_backward<float>(dL_dmz, grad, dL_dh);
+}
+
+int vmx_fit_set_resident(vmx_ctx* c, uint64_t bytes) {
+    g_last_error.clear();
+    if (!c) return fail(VMX_ERR_ARG, "null context");
+    c->fit.limit = (size_t)bytes;
+    c->fit.refused[0] = c->fit.refused[1] = SIZE_MAX;
+    return VMX_OK;
+}
+
+int vmx_fit_get_form(vmx_ctx* c, int32_t* form) {
+    g_last_error.clear();
+    if (!c || !form) return fail(VMX_ERR_ARG, "null argument");
+    *form = c->fit.ready ? c->fit.form : -1;
+    return VMX_OK;
 }
 
 int vmx_get_launch_config(vmx_ctx* c, int32_t* block_size, int32_t* xcd_remap) {

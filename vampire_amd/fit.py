@@ -3,8 +3,8 @@ trajectory.
 
 The trajectory is the deterministic (T = 0) Heun step of sim::LLG_Heun
 (src/simulate/LLGHeun.cpp:160-282) run on the device by libvmx; its gradient comes from the
-library's hand-written discrete adjoint (vmx_fit_backward), with segments between checkpoints
-recomputed.  PyTorch only wraps the two calls as a torch.autograd.Function so a loss written in
+library's hand-written discrete adjoint (vmx_fit_backward), over the kept trajectory while that is
+within a limit (8 GiB unless set), else over segments recomputed between checkpoints.  PyTorch only wraps the two calls as a torch.autograd.Function so a loss written in
 torch can be minimised with torch optimisers; no spin dynamics runs in torch.
 
 Parameters are in SI: J (J), Ku (J), alpha, and per-site fields h (T, [3, N]).  The library works
@@ -24,12 +24,17 @@ from .system import MU_B, System
 
 
 class Trajectory:
-    """A device context set up for fitting (one material, uniform isotropic exchange)."""
+    """A device context set up for fitting (one material, uniform isotropic exchange).
+
+    resident_bytes: device memory the trajectory may keep beyond its checkpoints (None: 8 GiB; 0: none,
+    segments of checkpoint_every steps are recomputed).  The results do not depend on it."""
 
     def __init__(self, system: System, spins0: np.ndarray, nsteps: int, record_every: int = 1,
                  checkpoint_every: int = 100, precision: str = "fp64", H: Sequence[float] = (0.0, 0.0, 0.0),
-                 topology: str = "auto"):
+                 topology: str = "auto", resident_bytes: Optional[int] = None):
         self.ctx = Context(system, precision=precision, topology=topology)
+        if resident_bytes is not None:
+            L.check(self.ctx.lib.vmx_fit_set_resident(self.ctx.h, int(resident_bytes)))
         self.n = system.n
         self.mu_s = system.materials[0]["mu_s_SI"]
         self.spins0 = np.ascontiguousarray(spins0, dtype=np.float64).reshape(3, self.n)
@@ -52,6 +57,14 @@ class Trajectory:
         d = np.ascontiguousarray(dL_dmz, dtype=np.float64)
         L.check(self.ctx.lib.vmx_fit_backward(self.ctx.h, L.dptr(d), L.dptr(g), None if dh is None else L.dptr(dh)))
         return g[0] / self.mu_s, g[1] / self.mu_s, g[2], (None if dh is None else dh.reshape(3, self.n))
+
+    @property
+    def form(self) -> int:
+        """What the last forward kept: 0 the trajectory, 1 checkpoints and a segment's predicted spins,
+        2 checkpoints alone, -1 before the first."""
+        v = C.c_int32(0)
+        L.check(self.ctx.lib.vmx_fit_get_form(self.ctx.h, C.byref(v)))
+        return int(v.value)
 
     def close(self):
         self.ctx.close()

@@ -272,3 +272,37 @@ def test_checkpoints_bound_the_memory_when_asked_to(hip):
         both(t)
         assert t.form == 1 and hip.fake_used() <= kept - 2000 * state, (hip.fake_used(), kept)
     """)
+
+
+def test_an_allocation_done_without_leaves_no_error(hip):
+    """Tiles, a kept trajectory and further transfer slots are taken where there is memory for them: a call that
+    went on without has nothing to report, and an earlier error's text stays."""
+    fake.run(hip, FIT + """
+        lib = L.load()
+        t = traj()
+        hip.fake_capacity(hip.fake_used() + 600 * state)
+        t.forward(S.J_CO, S.KU_CO, 0.1)
+        assert t.ctx.lib.vmx_last_error() == b""
+        hip.fake_capacity(288 << 30)
+        t.close()
+
+        def earlier(c):
+            assert lib.vmx_mc_set_sigma(c.h, 99, 1.0) == L.VMX_ERR_ARG
+            return lib.vmx_last_error()
+
+        with Context(S.ferromagnet("sc", 20), precision=FP64, seed=1) as c:      # no memory for tiles
+            c.set_spins(S.random_spins(8000, 2))
+            text = earlier(c)
+            hip.fake_capacity(hip.fake_used())
+            c.llg_heun(100)
+            assert text and lib.vmx_last_error() == text, lib.vmx_last_error()
+            assert c.tiles == 0
+            hip.fake_capacity(288 << 30)
+        big = RC.isolated_spins(1_000_001)
+        with Context(big, precision=FP64, seed=1) as c:                          # nor for more slots
+            text = earlier(c)
+            hip.fake_capacity(hip.fake_used())
+            c.set_spins(np.zeros((3, big.n)))
+            assert lib.vmx_last_error() == text, lib.vmx_last_error()
+            hip.fake_capacity(288 << 30)
+    """)

@@ -140,16 +140,18 @@ struct HostPipe {
             if (done[k]) (void)hipEventDestroy(done[k]);
         }
     }
-    int ready(int workers) {
-        for (int k = 0; k < 2 * workers; ++k) {
-            if (!slot[k]) VMX_HIP(hipHostMalloc(&slot[k], bytes, hipHostMallocDefault));
-            if (!done[k]) VMX_HIP(hipEventCreateWithFlags(&done[k], hipEventDisableTiming));
+    hipError_t ready(int workers) {
+        hipError_t e = hipSuccess;
+        for (int k = 0; k < 2 * workers && e == hipSuccess; ++k) {
+            if (!slot[k] && (e = hipHostMalloc(&slot[k], bytes, hipHostMallocDefault)) != hipSuccess) slot[k] = nullptr;
+            if (e == hipSuccess && !done[k]) e = hipEventCreateWithFlags(&done[k], hipEventDisableTiming);
         }
-        return VMX_OK;
+        return e;
     }
     int init(size_t largest) {     // largest: the largest transfer expected often
         bytes = (std::min(kChunk, std::max(largest, kSlot)) + 4095) & ~(size_t)4095;
-        return ready(1);
+        VMX_HIP(ready(1));
+        return VMX_OK;
     }
     // Moves every segment, after the work queued on st.  To the host: returns when the data has
     // arrived.  To the device: returns when the caller's arrays may be reused.
@@ -186,7 +188,10 @@ struct HostPipe {
             return VMX_OK;
         }
         int workers = (int)std::min<size_t>(kWorkers, 1 + total / ((size_t)8 << 20));
-        if (ready(workers) != VMX_OK) workers = 1;   // no pinned memory for more: the first one's slots are there
+        if (ready(workers) != hipSuccess) {      // no pinned memory for more: the first one's slots are there
+            (void)hipGetLastError();
+            workers = 1;
+        }
         int dev = 0;
         if (workers > 1) VMX_HIP(hipGetDevice(&dev));
         hipError_t err[kWorkers] = {};
@@ -1798,6 +1803,7 @@ int vmx_ctx::fit_forward(const double* h, const double* spins0, double* mz_out) 
     const int parts = std::max(1, std::min(kFitParts, n / 4096));
     VMX_TRY(fit.mz.alloc((size_t)parts * std::max(fit.nrec, 1) * sizeof(double)));
     VMX_TRY(fit.prm.alloc(sizeof(FitPrm<R>)));
+    const std::string before = g_last_error;       // of a form done without there is nothing to report
     int nseg = 0;
     for (int form = 0;; ++form) {
         fit.form = form;
@@ -1815,6 +1821,7 @@ int vmx_ctx::fit_forward(const double* h, const double* spins0, double* mz_out) 
         if (rc == VMX_OK && !fit.keepP) rc = fit.P.alloc(sb);
         if (rc == VMX_OK) break;
         if (form == 2 || rc != VMX_ERR_NOMEM) return rc;
+        g_last_error = before;
         fit.refused[form] = kept;                  // the next form has all the memory, and later passes begin with it
         for (DevBuf* b : {&fit.traj, &fit.seg, &fit.lH1, &fit.lPd, &fit.lT, &fit.H0, &fit.sumS, &fit.lH0, &fit.lSp,
                           &fit.dh, &fit.nhat})
@@ -2214,11 +2221,13 @@ int vmx_ctx::build_tiles(int64_t steps) {
     steps_before_tiles += steps;
     if (steps_before_tiles < n / 128) return VMX_OK;
     tiles_made = true;
+    const std::string before = g_last_error;
     try {
         const int rc = make_tiles();
         if (rc != VMX_ERR_NOMEM) return rc;
     } catch (const std::bad_alloc&) {
     }
+    g_last_error = before;
     return VMX_OK;                               // no memory for the tiles: two kernels a step, as before
 }
 

@@ -306,3 +306,21 @@ def test_an_allocation_done_without_leaves_no_error(hip):
             assert lib.vmx_last_error() == text, lib.vmx_last_error()
             hip.fake_capacity(288 << 30)
     """)
+
+
+@pytest.mark.parametrize("L,folded", [(50, True), (52, False)])
+def test_a_constrained_sweeps_first_round_adds_a_bounded_number_of_partials(hip, L, folded):
+    """A basis-major crystal has four runs of cells: 7816 and 8788 entries of 64 atoms, around the 8192 that every
+    workgroup of the sweep's first round may add; the later rounds' own partials are few either way."""
+    fake.run(hip, f"""
+        s = S.ferromagnet("fcc", {L})
+        with Context(s, precision=FP32, seed=1, block_size=64) as c:
+            c.set_conditions(300.0)
+            c.set_spins(S.random_spins(s.n, 2))
+            c.cmc_set_constraint(10.0, 20.0)
+            c.cmc_sweep(1)
+            names = [l.name for l in launches(log(lambda: c.cmc_sweep(3)))]
+            assert sum("k_cmc_pairs" in x for x in names) == 3 * 8, names
+            assert sum("k_moment_finish" in x for x in names) == (0 if {folded} else 3), names
+            assert not any("k_moment_add" in x for x in names), names
+    """)

@@ -572,6 +572,7 @@ struct vmx_ctx {
     DevBuf deg, pat, pat_off, pat_jid, pat_deg;
     DevBuf rep_m;                 // [nrep] replica size / q
     DevBuf rep_blk;               // [nrep+1] each replica's first entry of the one-atom block table
+    int rep_blk_most = 0;         // the most entries of one replica
     DevBuf spin[3];               // three buffers of 3N R each (S, P, O roles rotate)
     int s_idx = 0, o_idx = 2;     // current spin buffer and the corrector's output buffer
     // The fused correctors read their own atom's S and gather only S' (or the midpoint), so they
@@ -681,7 +682,13 @@ struct vmx_ctx {
     // Rounds sum the partials of the round before themselves (CmcMoment) while a replica has at most
     // kCmcFoldPartials of them, two loads a thread; the first colour without pairs ends a replica's rounds.
     bool cmc_fold = false;
+    // A sweep's first round adds the full sum's partials too, one an entry of the block table, while a replica
+    // has at most kCmcFoldSum of them; with more, a launch finishes the sum, since each of the round's
+    // workgroups reads them all (one replica FP32, us a sweep folded / with the launch: SC 40^3, 1000
+    // entries 44.8 / 46.8; SC 80^3, 8000 entries 69.9 / 71.1; FCC 63^3, 3908 entries 195.2 / 195.1, 15,628
+    // entries 214.6 / 214.2).
     static constexpr int kCmcFoldPartials = 512;
+    static constexpr int kCmcFoldSum = 8192;
     static constexpr size_t kCmcPermBytes = (size_t)1 << 20;   // permutations made ahead of their sweeps
     int colour_order(const std::vector<int>& c, const std::vector<int>& lau, int nc);
     template <typename R>
@@ -890,6 +897,8 @@ struct vmx_ctx {
         for (int e = (int)tab.size() - 1; e >= 0; --e)
             if (tab[e].z > tab[e].x) first[tab[e].y] = e;
         for (int r = nrep - 1; r >= 0; --r) first[r] = std::min(first[r], first[r + 1]);
+        rep_blk_most = 0;
+        for (int r = 0; r < nrep; ++r) rep_blk_most = std::max(rep_blk_most, first[r + 1] - first[r]);
         VMX_TRY(upload(rep_blk, first));
         return VMX_OK;
     }
@@ -1481,7 +1490,6 @@ int vmx_ctx::colour() {
             if (parts > kCmcFoldPartials || (parts > 0 && done)) cmc_fold = false;
             done = done || parts == 0;
         }
-        if ((rep_off_h[r + 1] - rep_off_h[r]) / 64 / q + 2 * q > 8 * kCmcFoldPartials) cmc_fold = false;
     }
     ncolours = nc;
     coloured = true;
@@ -1705,14 +1713,15 @@ int vmx_ctx::cmc_sweeps(int nsweeps) {
     const size_t nperm = 2 * (size_t)ncolours * nrep, ndm = 3 * (size_t)cmc_tab_start[ncolours];
     const int ahead = (int)std::max<size_t>(1, std::min<size_t>(64, cmc_perm.bytes / (nperm * sizeof(int4))));
     double* const dm0 = cmc_dm.as<double>();
+    const bool fold_sum = cmc_fold && rep_blk_most <= kCmcFoldSum;
     for (int w = 0; w < nsweeps; ++w) {
         if (last < 0) { ++sweep; continue; }
         if (w % ahead == 0) VMX_TRY(cmc_permutations(sweep, std::min(ahead, nsweeps - w)));
         VMX_HIP(Ops<R>::replica_moment(stream, s, C, moments(), gather, rep_blk.as<int>(), nrep,
-                                       cmc_part.as<double>(), cmc_M.as<double>(), !cmc_fold));
+                                       cmc_part.as<double>(), cmc_M.as<double>(), !fold_sum));
         // folded: a round starts from the sums before it; the sweep's first from the full sum's partials
-        CmcMoment mom{cmc_M.as<double>(), nullptr, nullptr, nullptr};
-        if (cmc_fold) mom = CmcMoment{nullptr, cmc_part.as<double>(), rep_blk.as<int>(), cmc_M.as<double>()};
+        CmcMoment mom{cmc_M.as<double>(), nullptr, nullptr, cmc_M.as<double>()};
+        if (fold_sum) mom = CmcMoment{nullptr, cmc_part.as<double>(), rep_blk.as<int>(), cmc_M.as<double>()};
         for (int k = 0; k <= last; ++k) {
             const int ntab = cmc_tab_start[k + 1] - cmc_tab_start[k];
             if (ntab == 0) continue;

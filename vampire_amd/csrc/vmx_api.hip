@@ -2480,7 +2480,7 @@ int vmx_create(const vmx_system* sys, const vmx_options* opt, vmx_ctx** out) {
     c->rowh_.swap(rowh);
     c->colh_.swap(colh);
     c->njt = (int)std::min<size_t>(table.size() / K, 1u << 30);
-    VMX_TRY(c->jtab.alloc(table.size() * rs));
+    VMX_TRY(c->jtab.alloc((table.size() * rs + 15) & ~(size_t)15));   // staged in 16-byte words
     if (c->precision == VMX_FP64) {
         VMX_HIP(hipMemcpy(c->jtab.p, table.data(), table.size() * sizeof(double), hipMemcpyHostToDevice));
     } else {

@@ -805,7 +805,7 @@ template <typename R>
 __host__ __device__ inline size_t fused_lds_bytes(int nmat, int npat, int zmax, int pat_lds, size_t jt_reals = 0) {
     const size_t rec = (size_t)nmat * ((sizeof(MatConst<R>) + sizeof(Cond<R>)) / sizeof(int));
     const size_t pat = pat_lds ? ((size_t)npat * (size_t)zmax + 3) & ~(size_t)3 : 0;
-    return (((rec + 3) & ~(size_t)3) + pat) * sizeof(int) + jt_reals * sizeof(R);
+    return (((rec + 3) & ~(size_t)3) + pat) * sizeof(int) + ((jt_reals * sizeof(R) + 15) & ~(size_t)15);
 }
 // the table's words from the launch's arguments to the device table (one workgroup)
 template <typename R>
@@ -850,10 +850,16 @@ __device__ __forceinline__ void stage_fused(const SysDev<R>& s, int rep, const C
     constexpr bool kPat = Access<AM>::TP == TP_PAT, kTab = Access<AM>::JM == JM_IDX16 && Access<AM>::TP != TP_CSR && KJ > 0;
     const int np = kPat && s.pat_lds ? s.npat * Access<AM>::W : 0;
     const int nj = kTab ? s.njt_lds * KJ * (int)(sizeof(R) / sizeof(int)) : 0;
+    const int bd = (int)blockDim.x, tid = (int)threadIdx.x;
+    const int rec = nm + nc, base = L::pat_off(s), jbase = L::jt_off(s), offs = rec + np;
+    // One pass over the tables with two loads in flight per thread: every wait for these loads also waits for
+    // the own-data loads issued before, so fewer rounds mean fewer waits.  An exchange table that would take it
+    // beyond one round goes in 16-byte words after it (its allocation ends on one): 8 KiB of scalars in words
+    // of the pass made a step of SC 43^3 slower than reading them from memory, 11.1 us against 9.9 in FP32 and
+    // 14.2 against 12.9 in FP64; now 9.5 and 12.7.
+    const bool wide = kTab && offs + nj > 2 * bd;
+    const int total = offs + (wide ? 0 : nj);
     const int* __restrict__ jt = reinterpret_cast<const int*>(s.jtab);
-    const int rec = nm + nc, base = L::pat_off(s), jbase = L::jt_off(s), offs = rec + np, total = offs + nj;
-    // one pass over the three tables with two loads in flight per thread: every wait for these
-    // loads also waits for the own-data loads issued before, so fewer rounds mean fewer waits
     auto src = [&](int k) {
         if (kTab) return k < nm ? mat[k] : (k < rec ? cond[k - nm] : (!kPat || k >= offs ? jt[k - offs] : s.pat_off[k - rec]));
         return k < nm ? mat[k] : (!kPat || k < rec ? cond[k - nm] : s.pat_off[k - rec]);
@@ -862,9 +868,8 @@ __device__ __forceinline__ void stage_fused(const SysDev<R>& s, int rep, const C
         if (kTab) return k < rec ? k : (!kPat || k >= offs ? jbase + (k - offs) : base + (k - rec));
         return !kPat || k < rec ? k : base + (k - rec);
     };
-    const int bd = (int)blockDim.x;
     auto stage = [&](auto&& from) {
-        for (int k0 = (int)threadIdx.x; k0 < total; k0 += 2 * bd) {
+        for (int k0 = tid; k0 < total; k0 += 2 * bd) {
             const int k1 = k0 + bd;
             const int v0 = from(k0);
             const int v1 = k1 < total ? from(k1) : 0;
@@ -877,6 +882,17 @@ __device__ __forceinline__ void stage_fused(const SysDev<R>& s, int rep, const C
         stage([&](int k) { return k >= nm && k < rec ? (int)ca->w[rep * nc + k - nm] : src(k); });
     else
         stage(src);
+    if (wide) {
+        const int4* __restrict__ jt4 = reinterpret_cast<const int4*>(s.jtab);
+        int4* const jl4 = reinterpret_cast<int4*>(vmx_lds + jbase);
+        const int jv = (nj + 3) >> 2;
+        for (int k0 = tid; k0 < jv; k0 += 2 * bd) {
+            const int k1 = min(k0 + bd, jv - 1);
+            const int4 v0 = jt4[k0], v1 = jt4[k1];
+            jl4[k0] = v0;
+            jl4[k1] = v1;
+        }
+    }
     __syncthreads();
 }
 template <typename R, int AM>
@@ -890,7 +906,14 @@ __device__ __forceinline__ void fused_row_index(const SysDev<R>& s, int i, int h
 // The spin field of a staged row in the step kernels.  A table of up to 8 KiB of exchange entries is read
 // from LDS: an edge's entry is 1, 3 or 9 reals, and through the texture path the 9 of a tensor cost three
 // times the neighbour's spin (diluted film of 472,014 atoms, 28 tensors, FP32: predictor 16.0 -> 13.4 us,
-// corrector 15.5 -> 12.8; the step with its temperature set before it 32.6 -> 26.3).
+// corrector 15.5 -> 12.8; the step with its temperature set before it 32.6 -> 26.3).  A step of ELL rows, table in
+// memory / staged, us:
+//                    scalars 1 KiB   8 KiB        vectors 1 KiB   8 KiB        tensors 1 KiB   8 KiB
+//   SC  43^3 FP32     9.7 /  9.4    9.8 /  9.5     9.9 /  9.5   10.0 /  9.6    11.9 / 10.1   12.4 / 11.0
+//            FP64    12.8 / 12.5   12.9 / 12.7    13.7 / 12.5   13.9 / 12.7    16.8 / 13.1   18.0 / 13.7
+//   FCC 50^3 FP32    31.0 / 24.6   33.3 / 25.0    33.6 / 24.9   34.6 / 25.7    47.0 / 26.0   53.8 / 32.5
+//            FP64    53.6 / 44.6   54.8 / 45.4    59.1 / 44.8   61.1 / 45.8    79.5 / 49.1   90.5 / 56.5
+// Beyond 8 KiB the copy would take a second round, and fewer workgroups would fit a CU.
 template <typename R, int ET, int AM, int Parts>
 __device__ __forceinline__ void step_field(const SysDev<R>& s, const SpinRsrc<R>& rs, const RowIdx<AM>& r, const R* ju,
                                            const MatConst<R>& mc, R sx, R sy, R sz, R& fx, R& fy, R& fz) {

@@ -152,12 +152,15 @@ def test_small_arrays_cross_in_one_copy(hip):
             lines = log(lambda: c.set_dipole(**dipole(400, s.n)))
             assert len(copies(lines)) < 60, len(copies(lines))
             assert copies(log(c.dipole_field)) == ["copy 2 19200"]       # the cells' two fields
+        s = RC.isolated_spins(43_000)                         # just within a slot
+        with Context(s, precision=FP32, seed=1) as c:
+            assert copies(log(c.get_spins)) == ["copy 2 1032000"]
     """)
 
 
-@pytest.mark.parametrize("n", [1, 2730, 2731, 10_923, 50_001, 130_000, 200_000, 750_001])
+@pytest.mark.parametrize("n", [1, 2731, 21_846, 43_690, 43_691, 50_001, 130_000, 200_000, 750_001])
 def test_chunked_transfers_keep_every_value_in_its_place(hip, n):
-    """Lengths around one chunk (64 KiB), four and more, and several workers: what the runtime holds after the
+    """Lengths around a slot (512 KiB to 1 MiB), two and more, and several workers: what the runtime holds after the
     copies is what the caller handed over (the kernels, which would permute, do nothing here)."""
     fake.run(hip, f"""
         s = RC.isolated_spins({n})

@@ -123,8 +123,9 @@ struct PinnedRing {
 // another third at 64 MiB and cost more at 8).  The first worker's two slots are allocated with the
 // context, the others by the first transfer that uses them; all are freed with it.
 // A copy on the link costs about 10 us before its bytes, one behind another as well as alone, so segments
-// that lie side by side on the device share chunks (an array's three components) and a chunk is at least
-// 512 KiB, whose host side takes longer than that (8000 atoms' spins in one chunk 35 us, in four 73).
+// that lie side by side on the device share chunks (an array's three components), a transfer that fits a
+// slot goes in one (8000 atoms' spins in one chunk 34 us, in four 73; 41,000 atoms' in one 67, in two 81, in
+// four 93), and the chunks of a longer one are at least 512 KiB, whose host side takes longer than that.
 struct HostPipe {
     // joined: lies in one allocation with the segment before it (a copy may span both)
     struct Seg { void* host; void* dev; size_t bytes; bool joined = false; };
@@ -162,7 +163,7 @@ struct HostPipe {
         std::vector<Chunk> chunks;
         size_t total = 0;
         for (int k = 0; k < nseg; ++k) total += seg[k].bytes;
-        const size_t limit = std::min(bytes, std::max(kSlot, (total / 4 + 4095) & ~(size_t)4095));
+        const size_t limit = total <= bytes ? bytes : std::min(bytes, std::max(kSlot, (total / 4 + 4095) & ~(size_t)4095));
         for (int k = 0; k < nseg; ++k)
             for (size_t o = 0, b; o < seg[k].bytes; o += b) {
                 char* dev = (char*)seg[k].dev + o;

@@ -327,3 +327,20 @@ def test_a_constrained_sweeps_first_round_adds_a_bounded_number_of_partials(hip,
             assert sum("k_moment_finish" in x for x in names) == (0 if {folded} else 3), names
             assert not any("k_moment_add" in x for x in names), names
     """)
+
+
+def test_a_trajectory_of_one_segment_is_not_copied(hip):
+    """50 steps and fewer stay where they were computed: no second copy of the states, in memory or time."""
+    fake.run(hip, FIT + """
+        for nsteps, copies in ((10, 1), (50, 1), (51, None)):
+            t = Trajectory(s, sp, nsteps=nsteps, record_every=1)
+            used = hip.fake_used()
+            f = log(lambda: t.forward(S.J_CO, S.KU_CO, 0.1))
+            b = log(lambda: t.backward(np.ones(nsteps)))
+            inside = lambda lines: sum(x.startswith("copy 3") for x in lines)
+            assert t.form == 0
+            if copies:
+                assert inside(f) == inside(b) == copies, (nsteps, inside(f), inside(b))     # the first state
+                assert hip.fake_used() - used < (2 * nsteps + 15) * state
+            t.close()
+    """)

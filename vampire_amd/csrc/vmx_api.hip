@@ -1025,7 +1025,8 @@ struct vmx_ctx {
     // Deterministic fitting trajectory and its adjoint.  A segment of G steps lies in `seg`: states
     // S_0 .. S_G, then (keepP) the predicted P_0 .. P_{G-1}.  Three forms, the first whose kept bytes are
     // within the limit and find memory (the working arrays of the backward pass are made before them):
-    //   0  every S and P is kept (traj: per segment S_1 .. S_G, P_0 .. P_{G-1}), nothing is recomputed;
+    //   0  every S and P is kept (traj: per segment S_1 .. S_G, P_0 .. P_{G-1}; one segment stays in seg),
+    //      nothing is recomputed;
     //   1  a checkpoint every K steps, and a segment of K recomputed with its P before the steps back over it;
     //   2  as 1 without the P, which each step back forms once more.
     // Segments of equal length replay graphs whose kernels read the parameters from device memory, so one
@@ -1808,7 +1809,8 @@ int vmx_ctx::fit_forward(const double* h, const double* spins0, double* mz_out) 
     fit.ready = false;
     VMX_HIP(hipStreamSynchronize(stream));         // a buffer that grows is freed: nothing may use it
     const int Gr = std::min(fit.nsteps, kFitSegment);
-    const size_t all = 2 * (size_t)((fit.nsteps + Gr - 1) / Gr) * Gr * sb;
+    // a trajectory of one segment stays in seg
+    const size_t all = 2 * (size_t)((fit.nsteps + Gr - 1) / Gr) * Gr * sb, apart = fit.nsteps > Gr ? all : 0;
     VMX_TRY(fit.h.alloc(sb));
     const int parts = std::max(1, std::min(kFitParts, n / 4096));
     VMX_TRY(fit.mz.alloc((size_t)parts * std::max(fit.nrec, 1) * sizeof(double)));
@@ -1823,11 +1825,11 @@ int vmx_ctx::fit_forward(const double* h, const double* spins0, double* mz_out) 
         nseg = (fit.nsteps + fit.G - 1) / fit.G;
         const size_t kept = form == 0 ? all : 2 * (size_t)fit.G * sb;
         if (form < 2 && (kept > fit.limit || kept >= fit.refused[form])) continue;
-        if (!fit.resident || fit.traj.bytes > fit.limit) fit.traj.release();
+        if (!fit.resident || apart == 0 || fit.traj.bytes > fit.limit) fit.traj.release();
         int rc = form < 2 ? fit_backward_buffers<R>() : VMX_OK;
         if (rc == VMX_OK) rc = fit.ckpt.alloc((size_t)(fit.resident ? 1 : nseg) * sb);
         if (rc == VMX_OK) rc = fit.seg.alloc((size_t)(fit.keepP ? 2 * fit.G + 1 : fit.G + 1) * sb);
-        if (rc == VMX_OK && fit.resident) rc = fit.traj.alloc(all);
+        if (rc == VMX_OK && fit.resident && apart) rc = fit.traj.alloc(apart);
         if (rc == VMX_OK && !fit.keepP) rc = fit.P.alloc(sb);
         if (rc == VMX_OK) break;
         if (form == 2 || rc != VMX_ERR_NOMEM) return rc;
@@ -1869,7 +1871,7 @@ int vmx_ctx::fit_forward(const double* h, const double* spins0, double* mz_out) 
             VMX_HIP(hipMemcpyAsync(ck + (size_t)c * N3, seg, sb, hipMemcpyDeviceToDevice, stream));
         if (replay && len == G) VMX_TRY(fit_replay(fit.fwd, key, [&] { return segment(G); }));
         else VMX_HIP(segment(len));
-        if (fit.resident)
+        if (fit.resident && apart)
             VMX_HIP(hipMemcpyAsync(fit.traj.as<R>() + (size_t)c * 2 * G * N3, seg + N3,
                                    (size_t)(len == G ? 2 * G : G + len) * sb, hipMemcpyDeviceToDevice, stream));
         // recorded states: those after a multiple of record_every steps
@@ -1954,7 +1956,7 @@ int vmx_ctx::fit_backward(const double* dmz, double* grad, double* dh_out) {
         const int start = c * G, len = std::min(G, fit.nsteps - start);
         if (!fit.resident || c == 0)
             VMX_HIP(hipMemcpyAsync(seg, ck + (size_t)c * N3, sb, hipMemcpyDeviceToDevice, stream));
-        if (fit.resident) {
+        if (fit.resident && nseg > 1) {
             const R* tr = fit.traj.as<R>() + (size_t)c * 2 * G * N3;
             if (c) VMX_HIP(hipMemcpyAsync(seg, tr - (size_t)(G + 1) * N3, sb, hipMemcpyDeviceToDevice, stream));
             VMX_HIP(hipMemcpyAsync(seg + N3, tr, (size_t)(len == G ? 2 * G : G + len) * sb, hipMemcpyDeviceToDevice, stream));

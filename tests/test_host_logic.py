@@ -148,7 +148,7 @@ def test_small_arrays_cross_in_one_copy(hip):
             assert copies(log(c.fields)) == ["copy 2 24000"] * 2
             lines = log(lambda: c.set_spins(sp))
             assert copies(lines) == ["copy 1 24000"]
-            assert [x for x in lines if x.startswith("wait")] == ["wait 4", "wait stream"], lines   # the slot's last use
+            assert sum(x.startswith("wait") for x in lines) == 1, lines     # for the call, not for the slot
             lines = log(lambda: c.set_dipole(**dipole(400, s.n)))
             assert len(copies(lines)) < 60, len(copies(lines))
             assert copies(log(c.dipole_field)) == ["copy 2 19200"]       # the cells' two fields
@@ -343,4 +343,19 @@ def test_a_trajectory_of_one_segment_is_not_copied(hip):
                 assert inside(f) == inside(b) == copies, (nsteps, inside(f), inside(b))     # the first state
                 assert hip.fake_used() - used < (2 * nsteps + 15) * state
             t.close()
+    """)
+
+
+def test_transfers_wait_for_events(hip):
+    """hipStreamSynchronize sleeps and may wake milliseconds late; an event is waited for by spinning."""
+    fake.run(hip, """
+        for n in (100, 60_000, 750_001):                      # one copy, several, several workers
+            s = RC.isolated_spins(n)
+            with Context(s, precision=FP64, seed=1) as c:
+                sp = S.random_spins(n, 2)
+                h, e = c.add_magnetization(np.zeros(n, np.int32), 1), c.add_energy(np.zeros(n, np.int32), 2)
+                for call in (lambda: c.set_spins(sp), c.get_spins, lambda: c.magnetization(h), lambda: c.energy(e),
+                             c.mc_state, c.cmc_counts):
+                    lines = log(call)
+                    assert any(x.startswith("wait ") for x in lines) and "wait stream" not in lines, lines
     """)

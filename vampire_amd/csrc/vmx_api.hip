@@ -126,6 +126,8 @@ struct PinnedRing {
 // that lie side by side on the device share chunks (an array's three components), a transfer that fits a
 // slot goes in one (8000 atoms' spins in one chunk 34 us, in four 73; 41,000 atoms' in one 67, in two 81, in
 // four 93), and the chunks of a longer one are at least 512 KiB, whose host side takes longer than that.
+// All waits are for events: hipStreamSynchronize sleeps, and in some contexts wakes 4 or 8 ms late (208k-atom
+// passes of 3.0 ms took 8.0 with it).
 struct HostPipe {
     // joined: lies in one allocation with the segment before it (a copy may span both)
     struct Seg { void* host; void* dev; size_t bytes; bool joined = false; };
@@ -182,12 +184,6 @@ struct HostPipe {
             for (size_t k = c.first; k < c.first + c.count; p += pieces[k].bytes, ++k)
                 to_host ? std::memcpy(pieces[k].host, p, pieces[k].bytes) : std::memcpy(p, pieces[k].host, pieces[k].bytes);
         };
-        if (to_host && chunks.size() == 1) {     // nothing to overlap
-            VMX_HIP(hipMemcpyAsync(slot[0], chunks[0].dev, chunks[0].bytes, hipMemcpyDeviceToHost, st));
-            VMX_HIP(hipStreamSynchronize(st));
-            copy(chunks[0], slot[0]);
-            return VMX_OK;
-        }
         int workers = (int)std::min<size_t>(kWorkers, 1 + total / ((size_t)8 << 20));
         if (ready(workers) != hipSuccess) {      // no pinned memory for more: the first one's slots are there
             (void)hipGetLastError();
@@ -718,7 +714,7 @@ struct vmx_ctx {
     hipGraph_t graph = nullptr;
     long long graph_key = -1;     // nsteps, block size, XCD mapping and buffer roles at capture
 
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_done = nullptr;
     int timed_steps = 0;
     PinnedRing ring;
     HostPipe pipe;
@@ -752,6 +748,7 @@ struct vmx_ctx {
         fit.drop_graph();
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
+        if (ev_done) (void)hipEventDestroy(ev_done);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -2471,6 +2468,7 @@ int vmx_create(const vmx_system* sys, const vmx_options* opt, vmx_ctx** out) {
     VMX_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     VMX_HIP(hipEventCreate(&c->ev0));
     VMX_HIP(hipEventCreate(&c->ev1));
+    VMX_HIP(hipEventCreateWithFlags(&c->ev_done, hipEventDisableTiming));
 
     std::vector<double> table;
     std::vector<uint16_t> idx16;
@@ -2593,7 +2591,8 @@ int vmx_set_spins(vmx_ctx* c, const double* sx, const double* sy, const double* 
     VMX_TRY(c->use_device());
     VMX_TRY(c->precision == VMX_FP64 ? c->upload3(sx, sy, sz, c->spins<double>(c->s_idx))
                                      : c->upload3(sx, sy, sz, c->spins<float>(c->s_idx)));
-    VMX_HIP(hipStreamSynchronize(c->stream));
+    VMX_HIP(hipEventRecord(c->ev_done, c->stream));   // a wait that spins (HostPipe)
+    VMX_HIP(hipEventSynchronize(c->ev_done));
     return VMX_OK;
 }
 

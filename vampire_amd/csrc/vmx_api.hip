@@ -1021,7 +1021,7 @@ struct vmx_ctx {
 
     // Deterministic fitting trajectory and its adjoint.  A segment of G steps lies in `seg`: states
     // S_0 .. S_G, then (keepP) the predicted P_0 .. P_{G-1}.  Three forms, the first whose kept bytes are
-    // within the limit and find memory (the working arrays of the backward pass are made before them):
+    // within the limit and find memory beside the working arrays of the backward pass (made with them):
     //   0  every S and P is kept (traj: per segment S_1 .. S_G, P_0 .. P_{G-1}; one segment stays in seg),
     //      nothing is recomputed;
     //   1  a checkpoint every K steps, and a segment of K recomputed with its P before the steps back over it;
@@ -1808,10 +1808,7 @@ int vmx_ctx::fit_forward(const double* h, const double* spins0, double* mz_out) 
     const int Gr = std::min(fit.nsteps, kFitSegment);
     // a trajectory of one segment stays in seg
     const size_t all = 2 * (size_t)((fit.nsteps + Gr - 1) / Gr) * Gr * sb, apart = fit.nsteps > Gr ? all : 0;
-    VMX_TRY(fit.h.alloc(sb));
     const int parts = std::max(1, std::min(kFitParts, n / 4096));
-    VMX_TRY(fit.mz.alloc((size_t)parts * std::max(fit.nrec, 1) * sizeof(double)));
-    VMX_TRY(fit.prm.alloc(sizeof(FitPrm<R>)));
     const std::string before = g_last_error;       // of a form done without there is nothing to report
     int nseg = 0;
     for (int form = 0;; ++form) {
@@ -1823,16 +1820,19 @@ int vmx_ctx::fit_forward(const double* h, const double* spins0, double* mz_out) 
         const size_t kept = form == 0 ? all : 2 * (size_t)fit.G * sb;
         if (form < 2 && (kept > fit.limit || kept >= fit.refused[form])) continue;
         if (!fit.resident || apart == 0 || fit.traj.bytes > fit.limit) fit.traj.release();
-        int rc = form < 2 ? fit_backward_buffers<R>() : VMX_OK;
+        int rc = fit.resident && apart ? fit.traj.alloc(apart) : VMX_OK;
         if (rc == VMX_OK) rc = fit.ckpt.alloc((size_t)(fit.resident ? 1 : nseg) * sb);
         if (rc == VMX_OK) rc = fit.seg.alloc((size_t)(fit.keepP ? 2 * fit.G + 1 : fit.G + 1) * sb);
-        if (rc == VMX_OK && fit.resident && apart) rc = fit.traj.alloc(apart);
         if (rc == VMX_OK && !fit.keepP) rc = fit.P.alloc(sb);
+        if (rc == VMX_OK) rc = fit.h.alloc(sb);
+        if (rc == VMX_OK) rc = fit.mz.alloc((size_t)parts * std::max(fit.nrec, 1) * sizeof(double));
+        if (rc == VMX_OK) rc = fit.prm.alloc(sizeof(FitPrm<R>));
+        if (rc == VMX_OK && form < 2) rc = fit_backward_buffers<R>();
         if (rc == VMX_OK) break;
         if (form == 2 || rc != VMX_ERR_NOMEM) return rc;
         g_last_error = before;
         fit.refused[form] = kept;                  // the next form has all the memory, and later passes begin with it
-        for (DevBuf* b : {&fit.traj, &fit.seg, &fit.lH1, &fit.lPd, &fit.lT, &fit.H0, &fit.sumS, &fit.lH0, &fit.lSp,
+        for (DevBuf* b : {&fit.traj, &fit.ckpt, &fit.seg, &fit.lH1, &fit.lPd, &fit.lT, &fit.H0, &fit.sumS, &fit.lH0, &fit.lSp,
                           &fit.dh, &fit.nhat})
             b->release();
     }

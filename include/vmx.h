@@ -229,7 +229,7 @@ int vmx_llg_heun_graph(vmx_ctx* ctx, int32_t nsteps, int32_t nrepeat);
 
 /* Steps of small systems run as one kernel over tiles of atoms and their halos once the context has
  * been asked for num_atoms/128 of them (fused kernels, rows of at most 16 neighbours, up to 400,000
- * neighbour slots); the spins are the same bit for bit.  on = 0 keeps the two kernels, 1 (default)
+ * neighbour slots; the tiles' tables are allocated then); the spins are the same bit for bit.  on = 0 keeps the two kernels, 1 (default)
  * allows the one.  vmx_get_whole_step returns the number of tiles in use, 0 for two kernels.  No
  * counterpart in the reference: for measurements and tests of either form. */
 int vmx_set_whole_step(vmx_ctx* ctx, int32_t on);

@@ -1169,8 +1169,8 @@ int vmx_ctx::heun_steps(int nsteps, const double* noise, double* kernel_ms) {
     return VMX_OK;
 }
 
-// sim::LLG_Midpoint (src/simulate/LLGMidpoint.cpp:87-186) with the fused workgroup organisation:
-// predictor into the spare buffer, corrector into the output buffer, roles swapped per step.
+// sim::LLG_Midpoint (src/simulate/LLGMidpoint.cpp:87-186) with the fused workgroup organisation: predictor
+// into the spare buffer, corrector over S; as one kernel into the output buffer, roles swapped per step.
 template <typename R>
 int vmx_ctx::midpoint_steps(int nsteps, const double* noise) {
     const SysDev<R> s = sys<R>(), sf = sys_fused<R>();
@@ -2206,13 +2206,20 @@ static int build_topology(vmx_ctx* c, int request, const std::vector<int>& rowh,
 // atoms while they and their halo fit its items (one per thread); a component that ends early is
 // followed by the next, so that tiles stay full.
 //
-// Where the line lies (us a step from a replayed graph, whole-step against two kernels, FP64 / FP32):
-//   SC   9^3 4.2/3.5 against 8.5/8.1    SC  33^3 7.9/5.9 against 9.0/8.4    SC  40^3  9.4/7.0  against 9.2/8.5
-//   BCC 16^3 4.9/4.1 against 9.4/9.0    BCC 28^3 9.2/7.1 against 10.0/9.1   BCC 32^3 12.2/10.7 against 10.1/9.0
-//   FCC 12^3 5.1/4.4 against 11.2/9.7   FCC 20^3 9.4/7.5 against 11.4/9.9   FCC 23^3 13.0/10.5 against 11.8/9.8
+// Where the line lies (us a step, whole step against two kernels; replayed / launched one by one, where the
+// two kernels wait for the host):
+//                  FP64 replayed    launched        FP32 replayed    launched       midpoint FP64   FP32
+//   SC   20^3     4.8 /  8.8      4.7 / 10.2      4.0 /  8.6       3.9 / 10.0      4.8 /  9.7    4.0 /  9.8
+//   SC   33^3     8.0 /  9.2      7.9 / 10.5      6.1 /  8.7       6.0 / 10.0      8.0 /  9.9    6.1 /  9.8
+//   SC   38^3     9.2 /  9.3      9.1 / 10.6      6.8 /  8.6       6.9 / 10.0      9.2 /  9.9    7.0 /  9.7
+//   SC   40^3     9.5 /  9.4      9.5 / 10.6      7.1 /  8.6       7.1 / 10.0      9.6 / 10.0    7.3 /  9.8
+//   BCC  29^3     9.6 / 10.5      9.6 / 11.7      7.3 /  9.4       7.4 / 10.7      9.7 / 11.0    7.5 / 10.4
+//   FCC  20^3     9.5 / 11.5      9.5 / 12.9      7.7 /  9.8       7.7 / 11.2      9.5 / 12.4    7.8 / 10.9
+//   film 90x90x8 11.8 / 12.4     11.8 / 13.1      8.8 / 11.3       8.9 / 12.1     11.9 / 12.7    9.1 / 12.3
+// and beyond it BCC 32^3 12.2 / 10.1 and 10.7 / 9.0, FCC 23^3 13.0 / 11.8 and 10.5 / 9.8 (replayed).
 // The whole step reads each item's record (slots of neighbour indices) and repeats the halo's
-// arithmetic, so the two meet at a number of slots, 400,000 = SC 40^3 = FCC 20^3.  CSR rows (no fixed
-// slot width) and the plain kernels keep their launches.
+// arithmetic, so the two meet at a number of slots, 400,000 = SC 40^3 = FCC 20^3; replayed in FP64 a little
+// before it, launched a little after.  CSR rows (no fixed slot width) and the plain kernels keep their launches.
 // Items per tile: 128 where the tiles do not fill the CUs (SC 20^3 FP64 4.5 us; 256: 5.1), then larger
 // tiles, whose halo is smaller (SC 33^3 FP32: 128 6.0, 192 5.9, 256 6.4; FCC 20^3: 8.8, 7.5, 8.4;
 // SC 40^3: 8.1, 7.6, 7.0).

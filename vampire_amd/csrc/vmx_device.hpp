@@ -1633,7 +1633,7 @@ struct Moments {
 // Masks of at most MAXB bins: each thread keeps every bin's four sums in registers and adds each
 // atom to its bin with predicated adds, so the cost does not depend on how often the id changes
 // along the atoms (a random alloy's material mask changes at nearly every atom).  The workgroup
-// then reduces its threads' sums in a fixed order (wavefront shuffles, then the wavefronts in
+// then reduces its threads' sums in a fixed order (each wavefront in registers, then the wavefronts in
 // order) into partial[block][nbins*4], the layout k_mag_hist writes.
 template <typename R, int MAXB>
 __global__ void __launch_bounds__(256)

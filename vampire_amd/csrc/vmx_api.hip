@@ -125,7 +125,8 @@ struct PinnedRing {
 // A copy on the link costs about 10 us before its bytes, one behind another as well as alone, so segments
 // that lie side by side on the device share chunks (an array's three components), a transfer that fits a
 // slot goes in one (8000 atoms' spins in one chunk 34 us, in four 73; 41,000 atoms' in one 67, in two 81, in
-// four 93), and the chunks of a longer one are at least 512 KiB, whose host side takes longer than that.
+// four 93), and the chunks of a longer one are a third of it, 512 KiB to 1 MiB, whose host side takes longer than
+// that (80,000 atoms' spins set in three chunks 106 us, in four 121).
 // All waits are for events: hipStreamSynchronize sleeps, and in some contexts wakes 4 or 8 ms late (208k-atom
 // passes of 3.0 ms took 8.0 with it).
 struct HostPipe {
@@ -165,7 +166,7 @@ struct HostPipe {
         std::vector<Chunk> chunks;
         size_t total = 0;
         for (int k = 0; k < nseg; ++k) total += seg[k].bytes;
-        const size_t limit = total <= bytes ? bytes : std::min(bytes, std::max(kSlot, (total / 4 + 4095) & ~(size_t)4095));
+        const size_t limit = total <= bytes ? bytes : std::min(bytes, std::max(kSlot, (total / 3 + 4095) & ~(size_t)4095));
         for (int k = 0; k < nseg; ++k)
             for (size_t o = 0, b; o < seg[k].bytes; o += b) {
                 char* dev = (char*)seg[k].dev + o;
